@@ -138,6 +138,29 @@ struct EmuBackend {
         }
     }
 
+    // the first pass with FP32 corner state, two cells per wavefront
+    void clip_pairs(const ClipParams& P) {
+#pragma omp parallel
+        {
+            std::unique_ptr<PairLds> L(new PairLds());
+            std::memset(L.get(), 0, sizeof(PairLds));
+#pragma omp for schedule(dynamic, 8)
+            for (int it = 0; it < P.n_items; it += 2) {
+                if (P.weighted) {
+                    if (P.counters)
+                        process_pair<true, true>(P, it, *L);
+                    else
+                        process_pair<true, false>(P, it, *L);
+                } else {
+                    if (P.counters)
+                        process_pair<false, true>(P, it, *L);
+                    else
+                        process_pair<false, false>(P, it, *L);
+                }
+            }
+        }
+    }
+
     template <int S, bool E, bool G>
     void clip_s(const ClipParams& P) {
 #pragma omp parallel
@@ -146,16 +169,6 @@ struct EmuBackend {
             std::memset(L.get(), 0, sizeof(CellLds<S>));
 #pragma omp for schedule(dynamic, 16)
             for (int it = 0; it < P.n_items; ++it) {
-                if constexpr (S == 1 && G && !E) {
-                    if (P.fp32) {
-                        // the first pass with FP32 corner state
-                        if (P.weighted)
-                            process_cell<S, false, G, true, true, float>(P, it, *L);
-                        else
-                            process_cell<S, false, G, false, false, float>(P, it, *L);
-                        continue;
-                    }
-                }
                 if (P.weighted)
                     process_cell<S, E, G, true>(P, it, *L);
                 else if (G && P.corner)
@@ -186,6 +199,10 @@ struct EmuBackend {
     int clip_waves() const { return waves_; }
     int waves_ = kDefaultClipWaves;
     void clip(int S, bool exact, bool gather, const ClipParams& P) {
+        if (P.fp32) {
+            clip_pairs(P);
+            return;
+        }
         if (exact) {
             if (gather)
                 clip_eg<true, true>(S, P);

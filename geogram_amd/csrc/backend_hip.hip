@@ -153,16 +153,24 @@ __device__ __forceinline__ int xcd_block() {
 // one-wave work-groups that measured 7 % faster than 168 registers and 3
 // waves — the wait for dependent LDS and memory round trips is hidden by
 // occupancy.  The exact re-clip (a few cells) keeps its registers.
-// F32: the first pass with FP32 corner state (the cells it cannot certify
-// are left to the FP64 kernel).
-template <int S, int WAVES, bool EXACT, bool GATHER, bool W, bool CORNER = W, bool F32 = false>
+template <int S, int WAVES, bool EXACT, bool GATHER, bool W, bool CORNER = W>
 __global__ __launch_bounds__(64 * WAVES, (S == 1 && !EXACT) ? 4 : 1) void k_clip(ClipParams P) {
     __shared__ CellLds<S> lds[WAVES];
-    const int wave = threadIdx.x >> 6;
+    const int wave = WAVES == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int item = xcd_block() * WAVES + wave;
     if (item >= P.n_items) return;  // whole wavefront
-    process_cell<S, EXACT, GATHER, W, CORNER, typename std::conditional<F32, float, double>::type>(
-        P, item, lds[wave]);
+    process_cell<S, EXACT, GATHER, W, CORNER>(P, item, lds[wave]);
+}
+
+// The first pass with FP32 corner state: two cells per wavefront
+// (pair_cell.h).
+template <int WAVES, bool W, bool COUNT>
+__global__ __launch_bounds__(64 * WAVES, 4) void k_pair(ClipParams P) {
+    __shared__ PairLds lds[WAVES];
+    const int wave = WAVES == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int item = 2 * (xcd_block() * WAVES + wave);
+    if (item >= P.n_items) return;  // whole wavefront
+    process_pair<W, COUNT>(P, item, lds[wave]);
 }
 
 __global__ void k_radius_r2(const int* __restrict__ items, int ni, const pt4* __restrict__ pts,
@@ -1592,15 +1600,6 @@ struct HipBackend {
                     return;
                 }
             }
-            if constexpr (G && !E) {
-                if (P.fp32) {
-                    if (waves_ == 1)
-                        k_clip<1, 1, false, true, W, W, true><<<g1, 64, 0, stream_>>>(P);
-                    else
-                        k_clip<1, 4, false, true, W, W, true><<<g4, 256, 0, stream_>>>(P);
-                    return;
-                }
-            }
             if (waves_ == 1)
                 k_clip<1, 1, E, G, W><<<g1, 64, 0, stream_>>>(P);
             else
@@ -1617,6 +1616,13 @@ struct HipBackend {
                 throw std::runtime_error("clip: 512-corner cells run from lists only");
         }
     }
+    template <bool W, bool COUNT>
+    void clip_pairs(const ClipParams& P) {
+        if (waves_ == 1)
+            k_pair<1, W, COUNT><<<blocks_for(P.n_items, 2), 64, 0, stream_>>>(P);
+        else
+            k_pair<4, W, COUNT><<<blocks_for(P.n_items, 8), 256, 0, stream_>>>(P);
+    }
     template <bool E, bool G>
     void clip_eg(int S, const ClipParams& P) {
         if (P.weighted)
@@ -1630,7 +1636,12 @@ struct HipBackend {
     int clip_waves() const { return waves_; }
     void clip(int S, bool exact, bool gather, const ClipParams& P) {
         if (P.n_items <= 0) return;
-        if (exact) {
+        if (P.fp32) {
+            if (P.weighted)
+                P.counters ? clip_pairs<true, true>(P) : clip_pairs<true, false>(P);
+            else
+                P.counters ? clip_pairs<false, true>(P) : clip_pairs<false, false>(P);
+        } else if (exact) {
             if (gather)
                 clip_eg<true, true>(S, P);
             else

@@ -30,15 +30,11 @@
 // follows the tie rule above and flags the cell.  Plane equations, new-corner
 // jobs and the two border-walk tables live in the wave's slice of LDS.
 //
-// Corner state in FP32 (the first pass over every cell).  Plane rows stay
-// FP64 in LDS; the corners' N, D and error magnitudes are FP32, built from
-// the rows rounded to FP32, and a sign is certified against the exact
-// determinant of the FP64 rows (the bound of Prec<float>).  A cell with a sign
-// or corner it cannot certify stops at once and is left to the FP64 pass.
-// Every other cell took the decisions the FP64 pass takes, in the same order
-// and into the same corner slots; its corners are rebuilt in FP64 from their
-// plane triples for the integration, exactly as the FP64 pass computed them,
-// so its outputs equal the FP64 pass's bit for bit.
+// The first pass over every cell keeps its corners in FP32, two cells per
+// wavefront (pair_cell.h): a sign it certifies is the sign of the exact
+// determinant of the FP64 rows (the bound of Prec<float>), so it takes the
+// decisions of the FP64 code below, in the same order and into the same corner
+// slots; a cell it cannot certify comes here.
 #pragma once
 
 #include <type_traits>
@@ -98,10 +94,10 @@ constexpr int kMaxVoronoiRings = 16;
 constexpr double kGamma9 = 1.2e-15;  // > gamma_9 for the conflict determinant
 constexpr double kGamma5 = 0.8e-15;  // > gamma_5 for the corner determinant D
 
-// Error bounds of the corner state of scalar type T.  gamma9: relative bound
-// on the conflict determinant t = e.N - h D against the exact determinant of
-// the FP64 plane rows; gamma5: corners with D <= gamma5 |D|_abs are
-// degenerate (flagged).
+// Error bounds of corners of scalar type T (FP64 here, FP32 in pair_cell.h).
+// gamma9: relative bound on the conflict determinant t = e.N - h D against the
+// exact determinant of the FP64 plane rows; gamma5: corners with
+// D <= gamma5 |D|_abs are degenerate (flagged).
 template <class T>
 struct Prec;
 template <>
@@ -115,8 +111,7 @@ struct Prec<double> {
 // term is off by at most gamma_13 < 7.8e-7 of its magnitude; 1.2e-6 also
 // covers the rounding of the magnitude sum.  N and D are off by at most
 // gamma9 of their magnitudes, so with D > 1e-5 |D|_abs the position N / D is
-// known to 12 % of D.  Magnitudes outside [1e-30, 1e30] (FP32 underflow or
-// overflow) are uncertain.
+// known to 12 % of D.
 template <>
 struct Prec<float> {
     static constexpr float gamma9 = 1.2e-6f;
@@ -188,8 +183,7 @@ struct ClipParams {
     // with piece set, writes its outputs and flags by item, not by seed
     const double* item_box;
     int piece;
-    // host dispatch: run the first pass (S = 1, gather, FP64 signs) with FP32
-    // corner state
+    // host dispatch: the first pass with FP32 corner state (pair_cell.h)
     int fp32;
 };
 
@@ -243,24 +237,17 @@ VGC_HD LU adj_of(const LU& w, int k) {
     return (w >> LU(CornerBits<S>::value * k)) & LU(CornerBits<S>::mask);
 }
 
-template <class T>
-struct CornerT {
-    Lane<T> nx, ny, nz, d, nmax, dabs, r2;
+struct Corner {
+    LD nx, ny, nz, d, nmax, dabs, r2;
     LB degenerate;
 };
-typedef CornerT<double> Corner;
 
 // Corner of planes a, b, c (outward normals e, offsets h), oriented so that
 // D = det(ea, eb, ec) > 0.  N = ha (eb x ec) + hb (ec x ea) + hc (ea x eb).
-// In FP32, r2 is an upper bound of the squared distance of the exact corner
-// of the FP64 rows (the security radius may then only stop later).
-template <class T>
-VGC_HD CornerT<T> make_corner(const Lane<T>& eax, const Lane<T>& eay, const Lane<T>& eaz,
-                              const Lane<T>& ha, const Lane<T>& ebx, const Lane<T>& eby,
-                              const Lane<T>& ebz, const Lane<T>& hb, const Lane<T>& ecx,
-                              const Lane<T>& ecy, const Lane<T>& ecz, const Lane<T>& hc) {
-    typedef Lane<T> LD;  // the lane type of the corner state
-    CornerT<T> C;
+VGC_HD Corner make_corner(const LD& eax, const LD& eay, const LD& eaz, const LD& ha, const LD& ebx,
+                          const LD& eby, const LD& ebz, const LD& hb, const LD& ecx, const LD& ecy,
+                          const LD& ecz, const LD& hc) {
+    Corner C;
     // cross products and their magnitude sums
     LD bcx = vfma(eby, ecz, -(ebz * ecy)), bcy = vfma(ebz, ecx, -(ebx * ecz)),
        bcz = vfma(ebx, ecy, -(eby * ecx));
@@ -287,24 +274,11 @@ VGC_HD CornerT<T> make_corner(const Lane<T>& eax, const Lane<T>& eay, const Lane
     LD naz = vfma(Aha, abcz, vfma(Ahb, acaz, Ahc * aabz));
     C.nmax = vmax(nax, vmax(nay, naz));
     C.dabs = vfma(Aeax, abcx, vfma(Aeay, abcy, Aeaz * abcz));
-    C.degenerate = C.d <= T(Prec<T>::gamma5) * C.dabs;
-    if constexpr (Prec<T>::fp32)
-        C.degenerate = C.degenerate | !(C.dabs >= T(1e-30f)) | !(C.dabs < T(1e30f)) |
-                       !(C.nmax < T(1e30f));
-    LD dd = select(C.degenerate, LD(T(1)), C.d);
-    LD inv = T(1) / dd;
+    C.degenerate = C.d <= kGamma5 * C.dabs;
+    LD dd = select(C.degenerate, LD(1.0), C.d);
+    LD inv = 1.0 / dd;
     LD qx = C.nx * inv, qy = C.ny * inv, qz = C.nz * inv;
     C.r2 = vfma(qx, qx, vfma(qy, qy, qz * qz));
-    if constexpr (Prec<T>::fp32) {
-        // (|N| + a)^2 / (D - gamma9 |D|_abs)^2 with a = 1.8 gamma9 max|N|abs
-        // (the length of N's error), plus 1e-5 for the rounding of this
-        // evaluation; |N| <= sqrt(3) max_i |N_i| in the cross term
-        const LD a = T(1.8f * Prec<T>::gamma9) * C.nmax;
-        const LD m = vmax(vabs(C.nx), vmax(vabs(C.ny), vabs(C.nz)));
-        const LD num = vfma(C.nx, C.nx, vfma(C.ny, C.ny, C.nz * C.nz)) + a * vfma(T(3.47f), m, a);
-        const LD den = select(C.degenerate, LD(T(1)), C.d - T(Prec<T>::gamma9) * C.dabs);
-        C.r2 = (num / (den * den)) * T(1.00001f);
-    }
     return C;
 }
 
@@ -318,20 +292,19 @@ struct CellState {
     uint64_t valid[S];
 };
 
-// Plane row p of the wave's table (FP64 in LDS) in the corner state's type.
-template <class T, int S>
-VGC_HD void load_row(const CellLds<S>& L, const LI& p, Lane<T>& ex, Lane<T>& ey, Lane<T>& ez,
-                     Lane<T>& h) {
+// Plane row p of the wave's table.
+template <int S>
+VGC_HD void load_row(const CellLds<S>& L, const LI& p, LD& ex, LD& ey, LD& ez, LD& h) {
     const double* pe = &L.pe[0][0];
-    ex = cvt<T>(lds_ld(pe, p * 4 + 0));
-    ey = cvt<T>(lds_ld(pe, p * 4 + 1));
-    ez = cvt<T>(lds_ld(pe, p * 4 + 2));
-    h = cvt<T>(lds_ld(pe, p * 4 + 3));
+    ex = lds_ld(pe, p * 4 + 0);
+    ey = lds_ld(pe, p * 4 + 1);
+    ez = lds_ld(pe, p * 4 + 2);
+    h = lds_ld(pe, p * 4 + 3);
 }
 
 // Box planes 0..5 = +x -x +y -y +z -z (outward), corners in lanes 0..7.
-template <int S, class T>
-VGC_HD void init_box(CellState<S, T>& st, CellLds<S>& L, const double* box, const pt4& pc) {
+template <int S>
+VGC_HD void init_box(CellState<S>& st, CellLds<S>& L, const double* box, const pt4& pc) {
     const LI lane = lane_id();
     {
         LB m = lane < 6;
@@ -365,18 +338,18 @@ VGC_HD void init_box(CellState<S, T>& st, CellLds<S>& L, const double* box, cons
         LI a0 = l8 ^ 4;
         LI a1 = select(pos, l8 ^ 1, l8 ^ 2);
         LI a2 = select(pos, l8 ^ 2, l8 ^ 1);
-        Lane<T> eax, eay, eaz, ha, ebx, eby, ebz, hb, ecx, ecy, ecz, hc;
-        load_row<T>(L, a, eax, eay, eaz, ha);
-        load_row<T>(L, b, ebx, eby, ebz, hb);
-        load_row<T>(L, c, ecx, ecy, ecz, hc);
-        CornerT<T> C = make_corner<T>(eax, eay, eaz, ha, ebx, eby, ebz, hb, ecx, ecy, ecz, hc);
+        LD eax, eay, eaz, ha, ebx, eby, ebz, hb, ecx, ecy, ecz, hc;
+        load_row(L, a, eax, eay, eaz, ha);
+        load_row(L, b, ebx, eby, ebz, hb);
+        load_row(L, c, ecx, ecy, ecz, hc);
+        Corner C = make_corner(eax, eay, eaz, ha, ebx, eby, ebz, hb, ecx, ecy, ecz, hc);
         st.nx[0] = C.nx;
         st.ny[0] = C.ny;
         st.nz[0] = C.nz;
         st.d[0] = C.d;
         st.nmax[0] = C.nmax;
         st.dabs[0] = C.dabs;
-        st.r2[0] = select(m, C.r2, Lane<T>(T(0)));
+        st.r2[0] = select(m, C.r2, LD(0.0));
         st.pl[0] = cvt<uint32_t>(a) | (cvt<uint32_t>(b) << LU(8)) | (cvt<uint32_t>(c) << LU(16));
         st.adj[0] = cvt<uint32_t>(a0) | (cvt<uint32_t>(a1) << LU(CornerBits<S>::value)) |
                     (cvt<uint32_t>(a2) << LU(2 * CornerBits<S>::value));
@@ -384,9 +357,9 @@ VGC_HD void init_box(CellState<S, T>& st, CellLds<S>& L, const double* box, cons
 #pragma unroll
         for (int s = 1; s < S; ++s) {
             st.valid[s] = 0;
-            st.nx[s] = st.ny[s] = st.nz[s] = T(0);
-            st.d[s] = T(1);
-            st.nmax[s] = st.dabs[s] = st.r2[s] = T(0);
+            st.nx[s] = st.ny[s] = st.nz[s] = 0.0;
+            st.d[s] = 1.0;
+            st.nmax[s] = st.dabs[s] = st.r2[s] = 0.0;
             st.pl[s] = 0;
             st.adj[s] = 0;
         }
@@ -436,33 +409,25 @@ VGC_HD LI exact_sign_lanes(const CellLds<S>& L, const LU& pl, const LB& m, doubl
 
 // Clip by plane (e, h) stored at slot np with neighbour id j.  Returns the
 // updated flags; *cut tells whether the plane removed a corner.
-template <int S, bool EXACT, class T>
-VGC_HD uint32_t clip_plane(CellState<S, T>& st, CellLds<S>& L, int& np, double ex, double ey,
+template <int S, bool EXACT>
+VGC_HD uint32_t clip_plane(CellState<S>& st, CellLds<S>& L, int& np, double ex, double ey,
                            double ez, double h, int j, uint32_t flags, bool& cut,
                            unsigned long long& nlive, unsigned long long& nnew) {
-    static_assert(!(EXACT && Prec<T>::fp32), "exact signs run with FP64 corners");
-    typedef Lane<T> LT;
     constexpr int kPMax = PMax<S>::value;
     const LI lane = lane_id();
-    // the plane in the corner state's type (FP64: itself)
-    const T ext = T(ex), eyt = T(ey), ezt = T(ez), ht = T(h);
-    const T e1 = vabs(ext) + vabs(eyt) + vabs(ezt);
-    const T ha = vabs(ht);
+    const double e1 = vabs(ex) + vabs(ey) + vabs(ez);
+    const double ha = vabs(h);
     uint64_t cm[S];
     bool anyc = false, allc = true, anyu = false;
 #pragma unroll
     for (int s = 0; s < S; ++s) nlive += (unsigned long long)popc64(st.valid[s]);
 #pragma unroll
     for (int s = 0; s < S; ++s) {
-        LT t = vfma(LT(ext), st.nx[s], vfma(LT(eyt), st.ny[s], vfma(LT(ezt), st.nz[s], -(ht * st.d[s]))));
-        LT bnd = T(Prec<T>::gamma9) * vfma(LT(e1), st.nmax[s], ha * st.dabs[s]);
+        LD t = vfma(LD(ex), st.nx[s], vfma(LD(ey), st.ny[s], vfma(LD(ez), st.nz[s], -(h * st.d[s]))));
+        LD bnd = kGamma9 * vfma(LD(e1), st.nmax[s], ha * st.dabs[s]);
         LB vs = mask_bit(st.valid[s]);
-        LB conf = t >= T(0);
-        LB unc;
-        if constexpr (Prec<T>::fp32)
-            unc = vs & !((vabs(t) > bnd) & (bnd >= T(1e-30f)) & (bnd < T(1e30f)));
-        else
-            unc = vs & (vabs(t) <= bnd);
+        LB conf = t >= 0.0;
+        LB unc = vs & (vabs(t) <= bnd);
         if constexpr (EXACT) {
             if (any(unc)) {
                 LI sg = exact_sign_lanes<S>(L, st.pl[s], unc, ex, ey, ez, h);
@@ -553,11 +518,11 @@ VGC_HD uint32_t clip_plane(CellState<S, T>& st, CellLds<S>& L, int& np, double e
                 LI a = cvt<int>(jb & LU(0xFF)) & (kPMax - 1);
                 LI b = cvt<int>((jb >> LU(8)) & LU(0xFF)) & (kPMax - 1);
                 LU y = (jb >> LU(16)) & LU(CornerBits<S>::mask);
-                LT eax, eay, eaz, hav, ebx, eby, ebz, hbv;
-                load_row<T>(L, a, eax, eay, eaz, hav);
-                load_row<T>(L, b, ebx, eby, ebz, hbv);
-                CornerT<T> C = make_corner<T>(eax, eay, eaz, hav, ebx, eby, ebz, hbv, LT(ext),
-                                              LT(eyt), LT(ezt), LT(T(hn)));
+                LD eax, eay, eaz, hav, ebx, eby, ebz, hbv;
+                load_row(L, a, eax, eay, eaz, hav);
+                load_row(L, b, ebx, eby, ebz, hbv);
+                Corner C = make_corner(eax, eay, eaz, hav, ebx, eby, ebz, hbv, LD(ex), LD(ey), LD(ez),
+                                       LD(hn));
                 if (any(is_t & C.degenerate)) flags |= CELL_UNCERTAIN;
                 st.nx[s] = select(is_t, C.nx, st.nx[s]);
                 st.ny[s] = select(is_t, C.ny, st.ny[s]);
@@ -638,15 +603,15 @@ struct CellRun {
 // One candidate neighbour j (Morton position) in nearest-first order: the
 // coincident-seed rule, the security-radius stop, then the clip.  Returns
 // true when the cell is finished (or failed) and the candidate loop must end.
-template <int S, bool EXACT, bool W, class T>
-VGC_HD bool consider(const ClipParams& P, CellLds<S>& L, CellRun<S, T>& R, int j, const pt4& pj) {
+template <int S, bool EXACT, bool W>
+VGC_HD bool consider(const ClipParams& P, CellLds<S>& L, CellRun<S>& R, int j, const pt4& pj) {
     if (j == R.c) return false;
     const double ex = pj.x - R.pc.x, ey = pj.y - R.pc.y, ez = pj.z - R.pc.z;
     const double d2 = ex * ex + ey * ey + ez * ez;
     if (d2 == 0.0) {
         if (P.orig[j] < R.orig_c) {
             wave_sync();
-            init_box<S, T>(R.st, L, R.box, R.pc);
+            init_box<S>(R.st, L, R.box, R.pc);
             R.np = 6;
             R.flags = CELL_DISCONNECTED;
             R.stopped = true;
@@ -660,14 +625,14 @@ VGC_HD bool consider(const ClipParams& P, CellLds<S>& L, CellRun<S, T>& R, int j
         bool anyin = false;
 #pragma unroll
         for (int s = 0; s < S; ++s)
-            anyin = anyin || any(mask_bit(R.st.valid[s]) & (T(4.1) * R.st.r2[s] >= T(d2)));
+            anyin = anyin || any(mask_bit(R.st.valid[s]) & (4.1 * R.st.r2[s] >= d2));
         reach = !anyin;
     } else {
         const double sd = d2 + R.cw;
         bool anyin = false;
 #pragma unroll
         for (int s = 0; s < S; ++s)
-            anyin = anyin || any(mask_bit(R.st.valid[s]) & (T(4.1 * d2) * R.st.r2[s] >= T(sd * sd)));
+            anyin = anyin || any(mask_bit(R.st.valid[s]) & (4.1 * d2 * R.st.r2[s] >= sd * sd));
         reach = (sd > 0.0) && !anyin;
     }
     if (reach) {
@@ -687,14 +652,10 @@ VGC_HD bool consider(const ClipParams& P, CellLds<S>& L, CellRun<S, T>& R, int j
     const double h = W ? 0.5 * (d2 + (R.wi - pj.w)) : 0.5 * d2;
     bool cut = false;
     ++R.ntest;
-    R.flags = clip_plane<S, EXACT, T>(R.st, L, R.np, ex, ey, ez, h, j, R.flags, cut, R.nlive, R.nnew);
+    R.flags = clip_plane<S, EXACT>(R.st, L, R.np, ex, ey, ez, h, j, R.flags, cut, R.nlive, R.nnew);
     R.prev_slot = (cut && !(R.flags & (CELL_EMPTY | CELL_OVERFLOW))) ? R.np - 1 : -1;
     if (cut) ++R.nclip;
-    // FP32 corners: the first sign or corner that is not certified ends the
-    // cell (the FP64 pass takes it over)
-    constexpr uint32_t kEnd =
-        CELL_EMPTY | CELL_OVERFLOW | CELL_BAD_TOPO | (Prec<T>::fp32 ? uint32_t(CELL_UNCERTAIN) : 0u);
-    if (R.flags & kEnd) {
+    if (R.flags & (CELL_EMPTY | CELL_OVERFLOW | CELL_BAD_TOPO)) {
         R.stopped = (R.flags & CELL_EMPTY) != 0;
         return true;
     }
@@ -776,8 +737,8 @@ VGC_HD LF lane_dist2(const pf4* pf, const LI& idx, const LB& m, float px, float 
 // overflows its buffers.  Breadth-first walk of the implicit tree, one node
 // per lane; boxes entirely inside the inner ball are skipped.  With F.on,
 // only seeds (and subtrees) that pass the power-distance filter are taken.
-template <int S>
-VGC_HD int gather_ring(const ClipParams& P, CellLds<S>& L, int c, int inst, float px, float py,
+template <class LDS>
+VGC_HD int gather_ring(const ClipParams& P, LDS& L, int c, int inst, float px, float py,
                        float pz, float rlo2, float rhi2, const PowerFilter& F) {
     const LI lane = lane_id();
     const int p0 = P.IL.p0[inst], n = P.IL.n[inst], nb = P.IL.nb[inst], Lv = P.IL.L[inst];
@@ -872,8 +833,8 @@ VGC_HD int gather_ring(const ClipParams& P, CellLds<S>& L, int c, int inst, floa
 }
 
 // Bitonic sort of L.cand[0..cnt) (cnt <= kCandCap), padded to 64 or 128.
-template <int S>
-VGC_HD void sort_cand(CellLds<S>& L, int cnt) {
+template <class LDS>
+VGC_HD void sort_cand(LDS& L, int cnt) {
     const LI lane = lane_id();
     const int P2 = cnt <= 64 ? 64 : 128;
     for (int i0 = 0; i0 < P2; i0 += kWave) {
@@ -948,8 +909,8 @@ VGC_HD LB corner_may_cut(const CornerTab& CT, const LF& ex, const LF& ey, const 
 
 // The candidates L.cand[0..cnt) that pass the corner test, compacted in
 // place (order kept); returns their count.
-template <int S>
-VGC_HD int corner_filter_cand(const ClipParams& P, CellLds<S>& L, int cnt, float px, float py,
+template <class LDS>
+VGC_HD int corner_filter_cand(const ClipParams& P, LDS& L, int cnt, float px, float py,
                               float pz, const CornerTab& CT) {
     static_assert(kCandCap == 2 * kWave, "two candidates per lane");
     const LI lane = lane_id();
@@ -985,8 +946,8 @@ VGC_HD int corner_filter_cand(const ClipParams& P, CellLds<S>& L, int cnt, float
 // below that distance, so the ring (rlo2, rhi2] it returns is complete.
 // Returns the count (<= kCandCap), or -1 when the stack overflows or the
 // nearest 64 are all at one distance.
-template <int S, bool CORNER>
-VGC_HD int gather_dfs(const ClipParams& P, CellLds<S>& L, int c, int inst, float px, float py,
+template <bool CORNER, class LDS>
+VGC_HD int gather_dfs(const ClipParams& P, LDS& L, int c, int inst, float px, float py,
                       float pz, float rlo2, float& rhi2, const PowerFilter& F,
                       const CornerTab& CT, bool& ct_on) {
     constexpr int kStack = 2 * kFrontCap;
@@ -1071,13 +1032,13 @@ VGC_HD int gather_dfs(const ClipParams& P, CellLds<S>& L, int c, int inst, float
                     // later rings, seeds must also pass the corner test (the
                     // buffer and this batch first)
                     ct_on = true;
-                    cnt = corner_filter_cand<S>(P, L, cnt, px, py, pz, CT);
+                    cnt = corner_filter_cand(P, L, cnt, px, py, pz, CT);
                     if (any(take)) take = take & corner_may_cut(CT, ex, ey, ez, d2, q.w, take);
                 }
             }
             if (cnt + popc64(ballot(take)) > kCandCap) {
                 // keep the seeds strictly nearer than the 64th nearest so far
-                sort_cand<S>(L, cnt);
+                sort_cand(L, cnt);
                 const float d64 = __builtin_bit_cast(float, uint32_t(L.cand[kWave - 1] >> 32));
                 const float nl2 = nextafterf(d64, 0.0f);
                 if (!(nl2 > rlo2)) return -1;
@@ -1101,7 +1062,7 @@ VGC_HD int gather_dfs(const ClipParams& P, CellLds<S>& L, int c, int inst, float
     }
     if (cnt > 0 && lim < rhi2) {
         // candidates taken before the bound came down
-        sort_cand<S>(L, cnt);
+        sort_cand(L, cnt);
         const uint64_t kmax = uint64_t(__builtin_bit_cast(uint32_t, lim)) << 32 | 0xFFFFFFFFull;
         int kept = 0;
         for (int i0 = 0; i0 < cnt; i0 += kWave) {
@@ -1476,7 +1437,7 @@ VGC_HD void mesh_emit(const ClipParams& P, CellLds<S>& L, const CS& st, int np,
 // Security-radius loop + integration for work item `item`.  GATHER: the
 // wave finds the neighbours itself, ring after ring of distance; otherwise
 // it reads them from P.list.
-template <int S, bool EXACT, bool GATHER, bool W, bool CORNER = W, class T = double>
+template <int S, bool EXACT, bool GATHER, bool W, bool CORNER = W>
 VGC_HD void process_cell(const ClipParams& P, int item, CellLds<S>& L) {
     constexpr int kPMax = PMax<S>::value;
     const LI lane = lane_id();
@@ -1512,7 +1473,7 @@ VGC_HD void process_cell(const ClipParams& P, int item, CellLds<S>& L) {
         return;
     }
 
-    CellRun<S, T> R;
+    CellRun<S> R;
     R.pc = pc;
     R.c = c;
     R.orig_c = P.orig[c];
@@ -1525,7 +1486,7 @@ VGC_HD void process_cell(const ClipParams& P, int item, CellLds<S>& L) {
     R.prev.x = R.prev.y = R.prev.z = R.prev.w = NAN;
     R.prev_slot = -1;
     R.nclip = R.ntest = R.nlive = R.nnew = 0;
-    init_box<S, T>(R.st, L, box, pc);
+    init_box<S>(R.st, L, box, pc);
     bool complete = false;
 
     if (!GATHER) {
@@ -1546,7 +1507,7 @@ VGC_HD void process_cell(const ClipParams& P, int item, CellLds<S>& L) {
                 complete = true;  // short list: the instance has fewer seeds
                 break;
             }
-            if (consider<S, EXACT, W, T>(P, L, R, j, L.stage[jj & (kWave - 1)])) break;
+            if (consider<S, EXACT, W>(P, L, R, j, L.stage[jj & (kWave - 1)])) break;
         }
     } else {
         const pf4 pq = P.pf[c];
@@ -1588,8 +1549,8 @@ VGC_HD void process_cell(const ClipParams& P, int item, CellLds<S>& L) {
             // first ring: level-synchronous walk; later rings: depth first,
             // bounded to the nearest seeds when the buffer fills
             int cnt = rlo2 >= 0.0f
-                          ? gather_dfs<S, CORNER>(P, L, c, inst, pq.x, pq.y, pq.z, rlo2, rhi2, F, CT, ct_on)
-                          : gather_ring<S>(P, L, c, inst, pq.x, pq.y, pq.z, rlo2, rhi2, F);
+                          ? gather_dfs<CORNER>(P, L, c, inst, pq.x, pq.y, pq.z, rlo2, rhi2, F, CT, ct_on)
+                          : gather_ring(P, L, c, inst, pq.x, pq.y, pq.z, rlo2, rhi2, F);
             if (F.on && ++nfilt > P.ring_limit) {
                 // a second gather (then the list tiers) takes the cell
                 R.flags |= CELL_NEED_K | CELL_WHY_RINGS;
@@ -1612,12 +1573,12 @@ VGC_HD void process_cell(const ClipParams& P, int item, CellLds<S>& L) {
                 rhi2 = nh;
                 continue;
             }
-            sort_cand<S>(L, cnt);
+            sort_cand(L, cnt);
             bool done = false;
             for (int jj = 0; jj < cnt; ++jj) {
                 if ((jj & (kWave - 1)) == 0) stage_cand<S>(P, L, jj, cnt);
                 const int j = int(uint32_t(L.cand[jj]));
-                if (consider<S, EXACT, W, T>(P, L, R, j, L.stage[jj & (kWave - 1)])) {
+                if (consider<S, EXACT, W>(P, L, R, j, L.stage[jj & (kWave - 1)])) {
                     done = true;
                     break;
                 }
@@ -1627,7 +1588,7 @@ VGC_HD void process_cell(const ClipParams& P, int item, CellLds<S>& L) {
             LD r2m = LD(0.0);
 #pragma unroll
             for (int s = 0; s < S; ++s)
-                r2m = vmax(r2m, select(mask_bit(R.st.valid[s]), cvt<double>(R.st.r2[s]), LD(0.0)));
+                r2m = vmax(r2m, select(mask_bit(R.st.valid[s]), R.st.r2[s], LD(0.0)));
             const double r2now = wave_max(r2m);
             const float need2 = radius_for(r2now, R.wi, W ? P.wmax[inst] : 0.0, W);
             if (need2 <= rhi2 || rhi2 >= all2) {
@@ -1650,7 +1611,7 @@ VGC_HD void process_cell(const ClipParams& P, int item, CellLds<S>& L) {
     }
     const bool stopped = R.stopped;
     uint32_t flags = R.flags;
-    CellState<S, T>& st = R.st;
+    CellState<S>& st = R.st;
     int np = R.np;
     const unsigned long long nclip = R.nclip, ntest = R.ntest, nlive = R.nlive, nnew = R.nnew;
     const int orig_c = R.orig_c;
@@ -1660,23 +1621,14 @@ VGC_HD void process_cell(const ClipParams& P, int item, CellLds<S>& L) {
     LD r2m = LD(0.0);
 #pragma unroll
     for (int s = 0; s < S; ++s)
-        r2m = vmax(r2m, select(mask_bit(st.valid[s]), cvt<double>(st.r2[s]), LD(0.0)));
-    double r2max = wave_max(r2m);
+        r2m = vmax(r2m, select(mask_bit(st.valid[s]), st.r2[s], LD(0.0)));
+    const double r2max = wave_max(r2m);
 
     if (P.counters && lane0()) {
         atomic_add_u64(P.counters + 0, nclip);
         atomic_add_u64(P.counters + 1, ntest);
         atomic_add_u64(P.counters + 2, nlive);
         atomic_add_u64(P.counters + 3, nnew);
-    }
-    if (Prec<T>::fp32 && (flags & CELL_UNCERTAIN)) {
-        // FP32 corners that could not certify a decision: only the flag (the
-        // FP64 pass redoes the cell and writes every output)
-        if (lane0()) {
-            P.flags[fc] = CELL_UNCERTAIN;
-            P.r2[fc] = 0.0;
-        }
-        return;
     }
     if (flags & (CELL_NEED_K | CELL_OVERFLOW | CELL_BAD_TOPO)) {
         // the partial cell contains the cell: its ball filters the list tiers
@@ -1720,39 +1672,17 @@ VGC_HD void process_cell(const ClipParams& P, int item, CellLds<S>& L) {
         return;
     }
     // corner points and topology to LDS
-    LD r2f = LD(0.0);
 #pragma unroll
     for (int s = 0; s < S; ++s) {
         LB vs = mask_bit(st.valid[s]);
         LI cid = lane + 64 * s;
-        LD nx, ny, nz, dd;
-        if constexpr (Prec<T>::fp32) {
-            // the FP64 corner of the plane triple, as the FP64 pass builds it
-            LD eax, eay, eaz, ha, ebx, eby, ebz, hb, ecx, ecy, ecz, hc;
-            load_row<double>(L, cvt<int>(byte_of(st.pl[s], 0)) & (kPMax - 1), eax, eay, eaz, ha);
-            load_row<double>(L, cvt<int>(byte_of(st.pl[s], 1)) & (kPMax - 1), ebx, eby, ebz, hb);
-            load_row<double>(L, cvt<int>(byte_of(st.pl[s], 2)) & (kPMax - 1), ecx, ecy, ecz, hc);
-            const Corner C = make_corner<double>(eax, eay, eaz, ha, ebx, eby, ebz, hb, ecx, ecy, ecz, hc);
-            nx = C.nx;
-            ny = C.ny;
-            nz = C.nz;
-            dd = C.d;
-            r2f = vmax(r2f, select(vs, C.r2, LD(0.0)));
-        } else {
-            nx = st.nx[s];
-            ny = st.ny[s];
-            nz = st.nz[s];
-            dd = st.d[s];
-        }
-        LD inv = 1.0 / select(vs, dd, LD(1.0));
-        lds_st(&L.q[0][0], cid * 3 + 0, nx * inv, vs);
-        lds_st(&L.q[0][0], cid * 3 + 1, ny * inv, vs);
-        lds_st(&L.q[0][0], cid * 3 + 2, nz * inv, vs);
+        LD inv = 1.0 / select(vs, st.d[s], LD(1.0));
+        lds_st(&L.q[0][0], cid * 3 + 0, st.nx[s] * inv, vs);
+        lds_st(&L.q[0][0], cid * 3 + 1, st.ny[s] * inv, vs);
+        lds_st(&L.q[0][0], cid * 3 + 2, st.nz[s] * inv, vs);
         lds_st(L.cpl, cid, st.pl[s], vs);
         lds_st(L.cadj, cid, st.adj[s], vs);
     }
-    // the FP64 cell's radius (the FP32 one bounds it from above)
-    if constexpr (Prec<T>::fp32) r2max = wave_max(r2f);
     for (int f0 = 0; f0 < np; f0 += 64) {
         LI f = f0 + lane;
         lds_st(L.v2t, select(f < np, f, LI(0)), LI(0x7FFFFFFF), f < np);
@@ -1872,9 +1802,7 @@ VGC_HD void process_cell(const ClipParams& P, int item, CellLds<S>& L) {
     }
     const double V = wave_sum(vacc);
     const double ntets = wave_sum(ntet);
-    // (the FP32 pass runs without cell meshes: the host sends mesh exports to
-    // the FP64 pass)
-    if (!Prec<T>::fp32 && P.mesh_mode && !face_overflow) {
+    if (P.mesh_mode && !face_overflow) {
         const double iv = V > 0.0 ? 1.0 / V : 0.0;
         mesh_emit<S>(P, L, st, np, orig_c, pc, wave_sum(mxa) * iv, wave_sum(mya) * iv,
                      wave_sum(mza) * iv);

@@ -10,7 +10,7 @@
 #include <hip/hip_runtime.h>
 #endif
 
-#include "clip_cell.h"
+#include "pair_cell.h"
 
 namespace vgc {
 

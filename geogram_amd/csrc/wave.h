@@ -264,6 +264,21 @@ inline LU fbits(const LF& a) {
     for (int i = 0; i < kWave; ++i) std::memcpy(&r.v[i], &a.v[i], 4);
     return r;
 }
+inline LF from_bits(const LU& a) {
+    LF r;
+    for (int i = 0; i < kWave; ++i) std::memcpy(&r.v[i], &a.v[i], 4);
+    return r;
+}
+inline LF vcbrtf(const LF& a) {
+    LF r;
+    for (int i = 0; i < kWave; ++i) r.v[i] = std::cbrt(a.v[i]);
+    return r;
+}
+// a wave-uniform value (in a scalar register on the GPU)
+template <class T>
+inline T uni(T x) {
+    return x;
+}
 // global-memory gather: base[idx] on the lanes of m, T() elsewhere
 template <class T>
 inline Lane<T> gld(const T* base, const LI& idx, const LB& m) {
@@ -286,6 +301,7 @@ inline uint64_t ballot(const LB& b) {
 }
 
 inline int popc64(uint64_t m) { return __builtin_popcountll(m); }
+inline int popc32(uint32_t m) { return __builtin_popcount(m); }
 inline int ffs64(uint64_t m) { return m ? __builtin_ctzll(m) : -1; }
 
 // number of set bits of m below each lane
@@ -344,6 +360,25 @@ inline float wave_maxf(const LF& a) {
     return x.v[0];
 }
 
+// per half of 32 lanes: the butterfly sum / maximum in every lane
+inline LD half_sum(const LD& a) {
+    LD x = a;
+    for (int m = 16; m >= 1; m >>= 1) x = x + shfl_xor(x, m);
+    return x;
+}
+inline LD half_max(const LD& a) {
+    LD x = a;
+    for (int m = 16; m >= 1; m >>= 1) x = vmax(x, shfl_xor(x, m));
+    return x;
+}
+// lane i's value from lane i - k (mod 16) of its row of 16
+template <class T>
+inline Lane<T> row_ror(const Lane<T>& a, int k) {
+    Lane<T> r;
+    for (int i = 0; i < kWave; ++i) r.v[i] = a.v[(i & ~15) | ((i - k) & 15)];
+    return r;
+}
+
 // LDS access: gather, masked scatter (lane order: higher lane wins on a
 // collision, like the hardware's unspecified order; callers never rely on it)
 template <class T>
@@ -374,6 +409,16 @@ inline void atomic_add_u64(unsigned long long* p, unsigned long long v) {
 // a flag shared by the cells of a pass: read, and raised once set
 inline unsigned flag_load(const unsigned* p) { return __atomic_load_n(p, __ATOMIC_RELAXED); }
 inline void flag_raise(unsigned* p) { __atomic_fetch_or(p, 1u, __ATOMIC_RELAXED); }
+// the same per lane: p[idx]
+inline LB flag_up(const unsigned* p, const LI& idx) {
+    LB r;
+    for (int i = 0; i < kWave; ++i) r.v[i] = flag_load(p + idx.v[i]) != 0;
+    return r;
+}
+inline void flag_set(unsigned* p, const LI& idx, const LB& m) {
+    for (int i = 0; i < kWave; ++i)
+        if (m.v[i]) flag_raise(p + idx.v[i]);
+}
 
 }  // namespace vgc
 
@@ -428,6 +473,21 @@ VGC_HD float vsqrtf(float a) { return __builtin_sqrtf(a); }
 VGC_HD float vabsf(float a) { return __builtin_fabsf(a); }
 VGC_HD float vminf(float a, float b) { return __builtin_fminf(a, b); }
 VGC_HD uint32_t fbits(float a) { return __float_as_uint(a); }
+VGC_HD float from_bits(uint32_t a) { return __uint_as_float(a); }
+VGC_HD float vcbrtf(float a) { return cbrtf(a); }
+// a wave-uniform value in a scalar register
+template <class T>
+VGC_HD T uni(T x) {
+    if constexpr (sizeof(T) == 8) {
+        const uint64_t u = __builtin_bit_cast(uint64_t, x);
+        const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)u);
+        const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(u >> 32));
+        return __builtin_bit_cast(T, (uint64_t(hi) << 32) | lo);
+    } else if constexpr (sizeof(T) == 4)
+        return __builtin_bit_cast(T, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, x)));
+    else
+        return T(__builtin_amdgcn_readfirstlane(int(x)));
+}
 template <class T>
 VGC_HD T gld(const T* base, int idx, bool m) {
     return m ? base[idx] : T();
@@ -438,6 +498,7 @@ VGC_HD int lane_id() { return __lane_id(); }
 VGC_HD uint64_t ballot(bool b) { return __ballot(b); }
 
 VGC_HD int popc64(uint64_t m) { return __popcll(m); }
+VGC_HD int popc32(uint32_t m) { return __popc(m); }
 VGC_HD int ffs64(uint64_t m) { return m ? __builtin_ctzll(m) : -1; }
 
 VGC_HD int mbcnt(uint64_t m) {
@@ -445,7 +506,8 @@ VGC_HD int mbcnt(uint64_t m) {
                                      __builtin_amdgcn_mbcnt_lo(uint32_t(m), 0u));
 }
 
-VGC_HD bool mask_bit(uint64_t m) { return (m >> __lane_id()) & 1; }
+// m is wave-uniform at every call: the mask itself is the lanes' predicate
+VGC_HD bool mask_bit(uint64_t m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
 VGC_HD bool mask_test(uint64_t m, int idx) { return (m >> (idx & 63)) & 1; }
 
 template <class T>
@@ -518,6 +580,52 @@ VGC_HD float wave_maxf(float a) {
     return readlane(x, 63);
 }
 
+// Per half of 32 lanes, the butterfly x + x(lane ^ m), m = 16, 8, 4, 2, 1, in
+// every lane: 16 by an LDS-crossbar swizzle, the others by DPP moves (8: row
+// rotation by 8; 4: rotation by 4, since lanes 8 apart agree by then; 2 and
+// 1: quad permutations).
+VGC_HD double swz16_f64(double x) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, x);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_ds_swizzle((int)(uint32_t)u, 0x401F);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_ds_swizzle((int)(uint32_t)(u >> 32), 0x401F);
+    return __builtin_bit_cast(double, (uint64_t(hi) << 32) | lo);
+}
+VGC_HD double half_sum(double a) {
+    double x = a + swz16_f64(a);
+    x = x + dpp_f64<0x128, 0xF>(x);  // row_ror:8
+    x = x + dpp_f64<0x124, 0xF>(x);  // row_ror:4
+    x = x + dpp_f64<0x4E, 0xF>(x);   // quad_perm [2, 3, 0, 1]
+    return x + dpp_f64<0xB1, 0xF>(x);  // quad_perm [1, 0, 3, 2]
+}
+VGC_HD double half_max(double a) {
+    double x = __builtin_fmax(a, swz16_f64(a));
+    x = __builtin_fmax(x, dpp_f64<0x128, 0xF>(x));
+    x = __builtin_fmax(x, dpp_f64<0x124, 0xF>(x));
+    x = __builtin_fmax(x, dpp_f64<0x4E, 0xF>(x));
+    return __builtin_fmax(x, dpp_f64<0xB1, 0xF>(x));
+}
+// lane i's value from lane i - K (mod 16) of its row of 16; k is a constant
+// at every call (unrolled loops)
+VGC_HD float row_ror(float x, int k) {
+    switch (k) {
+        case 1: return dpp_f32<0x121, 0xF>(x);
+        case 2: return dpp_f32<0x122, 0xF>(x);
+        case 3: return dpp_f32<0x123, 0xF>(x);
+        case 4: return dpp_f32<0x124, 0xF>(x);
+        case 5: return dpp_f32<0x125, 0xF>(x);
+        case 6: return dpp_f32<0x126, 0xF>(x);
+        case 7: return dpp_f32<0x127, 0xF>(x);
+        case 8: return dpp_f32<0x128, 0xF>(x);
+        case 9: return dpp_f32<0x129, 0xF>(x);
+        case 10: return dpp_f32<0x12A, 0xF>(x);
+        case 11: return dpp_f32<0x12B, 0xF>(x);
+        case 12: return dpp_f32<0x12C, 0xF>(x);
+        case 13: return dpp_f32<0x12D, 0xF>(x);
+        case 14: return dpp_f32<0x12E, 0xF>(x);
+        default: return dpp_f32<0x12F, 0xF>(x);
+    }
+}
+
 template <class T>
 VGC_HD T lds_ld(const T* p, int idx) {
     return p[idx];
@@ -551,6 +659,10 @@ VGC_HD unsigned flag_load(const unsigned* p) {
     return __hip_atomic_load(const_cast<unsigned*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 VGC_HD void flag_raise(unsigned* p) { atomicOr(p, 1u); }
+VGC_HD bool flag_up(const unsigned* p, int idx) { return flag_load(p + idx) != 0; }
+VGC_HD void flag_set(unsigned* p, int idx, bool m) {
+    if (m) flag_raise(p + idx);
+}
 
 }  // namespace vgc
 
