@@ -140,22 +140,24 @@ struct EmuBackend {
 
     // the first pass with FP32 corner state, two cells per wavefront
     void clip_pairs(const ClipParams& P) {
+        constexpr int kGroup = 16;  // cells per wavefront (the results do not depend on it)
 #pragma omp parallel
         {
             std::unique_ptr<PairLds> L(new PairLds());
             std::memset(L.get(), 0, sizeof(PairLds));
 #pragma omp for schedule(dynamic, 8)
-            for (int it = 0; it < P.n_items; it += 2) {
+            for (int it = 0; it < P.n_items; it += kGroup) {
+                const int m = std::min(kGroup, P.n_items - it);
                 if (P.weighted) {
                     if (P.counters)
-                        process_pair<true, true>(P, it, *L);
+                        process_pairs<true, true>(P, it, m, *L);
                     else
-                        process_pair<true, false>(P, it, *L);
+                        process_pairs<true, false>(P, it, m, *L);
                 } else {
                     if (P.counters)
-                        process_pair<false, true>(P, it, *L);
+                        process_pairs<false, true>(P, it, m, *L);
                     else
-                        process_pair<false, false>(P, it, *L);
+                        process_pairs<false, false>(P, it, m, *L);
                 }
             }
         }

@@ -168,9 +168,9 @@ template <int WAVES, bool W, bool COUNT>
 __global__ __launch_bounds__(64 * WAVES, 4) void k_pair(ClipParams P) {
     __shared__ PairLds lds[WAVES];
     const int wave = WAVES == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int item = 2 * (xcd_block() * WAVES + wave);
-    if (item >= P.n_items) return;  // whole wavefront
-    process_pair<W, COUNT>(P, item, lds[wave]);
+    const int first = P.group * (xcd_block() * WAVES + wave);
+    if (first >= P.n_items) return;  // whole wavefront
+    process_pairs<W, COUNT>(P, first, min(P.group, P.n_items - first), lds[wave]);
 }
 
 __global__ void k_radius_r2(const int* __restrict__ items, int ni, const pt4* __restrict__ pts,
@@ -1616,12 +1616,18 @@ struct HipBackend {
                 throw std::runtime_error("clip: 512-corner cells run from lists only");
         }
     }
+    // Cells per wavefront of k_pair: 8, which share one walk of the tree, once
+    // that leaves enough wavefronts for the 4096 resident ones to even out,
+    // else 4 or 2.
+    static int pair_group(int n) { return n >= 400000 ? 8 : n >= 150000 ? 4 : 2; }
     template <bool W, bool COUNT>
     void clip_pairs(const ClipParams& P) {
+        ClipParams Q = P;
+        Q.group = pair_group(P.n_items);
         if (waves_ == 1)
-            k_pair<1, W, COUNT><<<blocks_for(P.n_items, 2), 64, 0, stream_>>>(P);
+            k_pair<1, W, COUNT><<<blocks_for(Q.n_items, Q.group), 64, 0, stream_>>>(Q);
         else
-            k_pair<4, W, COUNT><<<blocks_for(P.n_items, 8), 256, 0, stream_>>>(P);
+            k_pair<4, W, COUNT><<<blocks_for(Q.n_items, 4 * Q.group), 256, 0, stream_>>>(Q);
     }
     template <bool E, bool G>
     void clip_eg(int S, const ClipParams& P) {

@@ -183,8 +183,10 @@ struct ClipParams {
     // with piece set, writes its outputs and flags by item, not by seed
     const double* item_box;
     int piece;
-    // host dispatch: the first pass with FP32 corner state (pair_cell.h)
+    // host dispatch: the first pass with FP32 corner state (pair_cell.h), and
+    // its cells per wavefront (even, at most 16)
     int fp32;
+    int group;
 };
 
 template <int S>

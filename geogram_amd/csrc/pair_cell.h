@@ -37,7 +37,8 @@
 namespace vgc {
 
 constexpr int kPairPlanes = 64;   // plane rows per cell
-constexpr int kStageCap = kWave;  // staged candidates per cell
+constexpr int kStageCap = kWave;  // candidates of a ring, sorted and staged
+constexpr int kNearCap = 256;     // buckets around a wave's cells
 // corner magnitudes |D|_abs and max|N|_abs outside these bounds are left to
 // the FP64 pass: (|N|_abs)^2, D^2 and the products of the sign bound then
 // neither overflow nor underflow
@@ -50,7 +51,7 @@ struct alignas(16) PairHalf {
     uint8_t st_tab[kPairPlanes];   // new corner whose first plane is p
     uint8_t en_tab[kPairPlanes];   // new corner whose second plane is p
     uint32_t job[64];              // new corners: a | b << 8 | across << 16
-    uint64_t key[kCandCap];        // the ring's candidates, sorted
+    uint64_t key[kStageCap];       // the ring's candidates, sorted
 };
 // FP32 rows of the next candidates of a half
 struct alignas(16) PairStage {
@@ -79,7 +80,10 @@ struct alignas(16) PairLds {
             uint64_t cand[kCandCap];
             union {
                 struct {
-                    int front[2][kFrontCap];
+                    union {
+                        int front[2][kFrontCap];
+                        uint64_t cand_b[kCandCap];  // those of the upper half's cell
+                    };
                     int bucket[kBucketCap];
                 };
                 PairStage stage[2];
@@ -87,6 +91,7 @@ struct alignas(16) PairLds {
         };
         PairInt in[2];
     };
+    int near_list[kNearCap];  // buckets around the wave's cells
 };
 static_assert(sizeof(PairLds) <= 10240, "16 wavefronts per CU");
 
@@ -427,47 +432,18 @@ VGC_HD uint64_t pair_cut(PairState& st, PairLds& L, LI& np, const RowLanes& r, c
     return fail | halves(bad);
 }
 
-// L.cand[0..cnt) (cnt <= kCandCap, keys distinct) into out in ascending
-// order: each lane counts the keys below its own
-template <class LDS>
-VGC_HD void rank_cand(LDS& L, int cnt, uint64_t* out) {
-    const LI lane = lane_id();
-    const LB in0 = lane < cnt, in1 = lane + kWave < cnt;
-    const LU64 a = lds_ld(L.cand, select(in0, lane, LI(0)));
-    LI r0 = LI(0);
-    if (cnt <= kWave) {
-        for (int i = 0; i < cnt; ++i) {
-            const LU64 k = lds_ld(L.cand, LI(i));
-            r0 = r0 + select(k < a, LI(1), LI(0));
-        }
-    } else {
-        const LU64 b = lds_ld(L.cand, select(in1, lane + kWave, LI(0)));
-        LI r1 = LI(0);
-        for (int i = 0; i < cnt; ++i) {
-            const LU64 k = lds_ld(L.cand, LI(i));
-            r0 = r0 + select(k < a, LI(1), LI(0));
-            r1 = r1 + select(k < b, LI(1), LI(0));
-        }
-        lds_st(out, select(in1, r1, LI(0)), b, in1);
-    }
-    lds_st(out, select(in0, r0, LI(0)), a, in0);
-    wave_sync();
-}
-
-// Candidates base .. base + 63 (below cnt) of half h as FP32 rows; returns the
+// The cnt <= kStageCap sorted candidates of half h as FP32 rows; returns the
 // number staged.  A candidate with the position and weight of the one before
 // it gives the same plane and is not staged: its id takes the other's place
 // (under the exact tie rule the copy takes over the face of the first one).
 // -1 when a candidate needs the general kernel: one at the seed's own
-// position, a row out of the range of the FP32 bounds, or equal FP32
-// distances across two batches (where a copy would go unseen).
+// position, or a row out of the range of the FP32 bounds.
 template <bool W>
 VGC_HD int pair_stage(const ClipParams& P, PairLds& L, int h, float scale, const pt4& pc, double cw,
-                      int base, int cnt) {
+                      int cnt) {
     const LI lane = lane_id();
-    const LI k = lane + base;
-    const LB ok = k < cnt;
-    const LU64 key = lds_ld(L.h[h].key, select(ok, k, LI(0)));
+    const LB ok = lane < cnt;
+    const LU64 key = lds_ld(L.h[h].key, select(ok, lane, LI(0)));
     const LI j = cvt<int>(cvt<uint32_t>(key));
     const Lane<pt4> q = gld(P.pts, j, ok);
     const LD s = LD(double(scale));
@@ -486,34 +462,29 @@ VGC_HD int pair_stage(const ClipParams& P, PairLds& L, int h, float scale, const
     const LF e1 = vabs(fx) + vabs(fy) + vabs(fz);
     float* row = &L.stage[h].row[0][0];
     float* aux = &L.stage[h].aux[0][0];
-    wave_sync();  // the previous batch is consumed
+    wave_sync();  // the previous ring is consumed
     lds_st_row(row, lane, fx, fy, fz, fh, ok);
     lds_st(aux, lane * 2, fr, ok);
     lds_st(aux, lane * 2 + 1, e1, ok);
     wave_sync();
-    LB out = ok & (!(d2 > 0.0) | !(e1 >= kPairE1Min) | !(e1 <= kPairE1Max) | !(vabs(fh) <= kPairHMax));
-    if (base > 0) {
-        const LU64 kp = lds_ld(L.h[h].key, LI(base - 1));
-        out = out | ((lane == 0) & ((kp >> LU64(32)) == (key >> LU64(32))));
-    }
+    const LB out = ok & (!(d2 > 0.0) | !(e1 >= kPairE1Min) | !(e1 <= kPairE1Max) | !(vabs(fh) <= kPairHMax));
     if (ballot(out)) return -1;
     // copies follow one another in the sorted order, at one FP32 distance
-    const LU64 kp = lds_ld(L.h[h].key, select(ok & (lane > 0), k - 1, LI(0)));
+    const LU64 kp = lds_ld(L.h[h].key, select(ok & (lane > 0), lane - 1, LI(0)));
     const LB same = ok & (lane > 0) & ((kp >> LU64(32)) == (key >> LU64(32)));
-    const int n = cnt - base < kStageCap ? cnt - base : kStageCap;
-    if (ballot(same) == 0) return n;
+    if (ballot(same) == 0) return cnt;
     const LI jp = cvt<int>(cvt<uint32_t>(kp));
     const Lane<pt4> qp = gld(P.pts, jp, same);
     const uint64_t dm = ballot(same & (pt_x(qp) == pt_x(q)) & (pt_y(qp) == pt_y(q)) &
                                (pt_z(qp) == pt_z(q)) & (pt_w(qp) == pt_w(q)));
-    if (dm == 0) return n;
+    if (dm == 0) return cnt;
     const uint64_t okm = ballot(ok), keep = okm & ~dm, last = okm & ~(dm >> 1);
     const LI at = mbcnt(keep) - select(mask_bit(keep), LI(0), LI(1));
     wave_sync();
     lds_st_row(row, at, fx, fy, fz, fh, mask_bit(keep));
     lds_st(aux, at * 2, fr, mask_bit(keep));
     lds_st(aux, at * 2 + 1, e1, mask_bit(keep));
-    lds_st(L.h[h].key, at + base, key, mask_bit(last));
+    lds_st(L.h[h].key, at, key, mask_bit(last));
     wave_sync();
     return popc64(keep);
 }
@@ -525,13 +496,229 @@ VGC_HD LF pair_to_wave(const LF& x0, const LF& x1, int h) {
     return select(lane < 32, shfl(x0, src), shfl(x1, src));
 }
 
+// ---------------------------------------------------- neighbour search
+//
+// A wave's cells are consecutive in Morton order, so they share one walk of
+// the tree: the buckets within a radius r of the box of their seeds go to
+// L.near_list once, and each cell's first ring (and its next ones, while
+// they stay within r) is a scan of those buckets.  A walk per cell and the
+// repeats of rings that had come out too large cost 40 % of the pass.
+
+// The wave's shared bucket list: complete for every seed of instance inst
+// within sqrt(r2) of the wave's seeds.
+struct NearList {
+    int inst;  // -1: no list (each cell walks the tree)
+    int n;
+    float r2;
+};
+// radius of the list and of a first ring over the mean 4th nearest distance
+// among bucket mates
+constexpr float kNearList = 2.3f, kNearRing = 1.95f;
+
+// Mean distance to the 4th nearest bucket mate of 4 * passes seeds of the
+// bucket of seed c (0: none has four).
+VGC_HD float near_spacing(const ClipParams& P, int c, int inst, int passes) {
+    const LI lane = lane_id();
+    const int p0 = P.IL.p0[inst], n = P.IL.n[inst];
+    const int m0 = c - ((c - p0) & (kBucket - 1));
+    float sum = 0.0f, cnt = 0.0f;
+    const LI m = m0 + (lane & (kBucket - 1));
+    const LB in = m < p0 + n;
+    const SeedLanes q = lane_seed(P.pf, select(in, m, LI(m0)), in);
+    for (int k = 0; k < passes; ++k) {
+        // row r of 16 lanes takes seed 4 (k + c / 4) + r of the bucket
+        const LI s = m0 + ((((c - m0) & ~3) + 4 * k + (lane >> 4)) & (kBucket - 1));
+        const LB sin = s < p0 + n;
+        const SeedLanes p = lane_seed(P.pf, select(sin, s, LI(m0)), sin);
+        const LF dx = q.x - p.x, dy = q.y - p.y, dz = q.z - p.z;
+        const LB ok = in & sin & (m != s);
+        const LF d2 = select(ok, dx * dx + dy * dy + dz * dz, LF(INFINITY));
+        LI below = LI(0);
+#pragma unroll
+        for (int i = 1; i < kBucket; ++i) below = below + select(row_ror(d2, i) < d2, LI(1), LI(0));
+        uint64_t fourth = ballot((below == 3) & (d2 < INFINITY));
+        for (int r = 0; r < 4; ++r) {
+            const uint64_t f = fourth & (0xFFFFull << (16 * r));
+            if (!f) continue;
+            const float d = readlane(d2, ffs64(f));
+            sum += sqrtf(d);
+            cnt += 1.0f;
+        }
+    }
+    return cnt > 0.0f ? sum / cnt : 0.0f;
+}
+
+// The buckets of instance inst within sqrt(r2) of the box of the wave's
+// seeds (items [i0, i1) with their Morton positions c per lane) into
+// L.near_list; returns their number, -1 when they or the walk overflow.
+template <class LDS>
+VGC_HD int near_buckets(const ClipParams& P, LDS& L, int inst, const LI& c, const LB& has, float r2) {
+    const LI lane = lane_id();
+    const SeedLanes p = lane_seed(P.pf, c, has);
+    const float hx = wave_maxf(select(has, p.x, LF(-INFINITY))), lx = -wave_maxf(select(has, -p.x, LF(-INFINITY)));
+    const float hy = wave_maxf(select(has, p.y, LF(-INFINITY))), ly = -wave_maxf(select(has, -p.y, LF(-INFINITY)));
+    const float hz = wave_maxf(select(has, p.z, LF(-INFINITY))), lz = -wave_maxf(select(has, -p.z, LF(-INFINITY)));
+    const int nb = P.IL.nb[inst], Lv = P.IL.L[inst];
+    const bnode* T = P.nodes + P.IL.t0[inst];
+    lds_st(&L.front[0][0], LI(0), LI(1), lane == 0);
+    wave_sync();
+    int nf = 1, cur = 0, nbk = 0;
+    while (nf > 0) {
+        int nn = 0;
+        for (int base = 0; base < nf; base += kWave) {
+            const LI idx = base + lane;
+            const LB in = idx < nf;
+            const LI node = lds_ld(&L.front[cur][0], select(in, idx, LI(0)));
+            const BoxLanes B = load_box(T, node, in);
+            const LF dx = vmaxf(vmaxf(B.lx - hx, lx - B.hx), 0.0f);
+            const LF dy = vmaxf(vmaxf(B.ly - hy, ly - B.hy), 0.0f);
+            const LF dz = vmaxf(vmaxf(B.lz - hz, lz - B.hz), 0.0f);
+            // (the margin covers the rounding of a seed's own distances)
+            const LB hit = in & ((dx * dx + dy * dy + dz * dz) * 0.99999f <= r2);
+            const LB internal = node < Lv;
+            const LB push = hit & internal;
+            const LB leaf = hit & !internal & (node - Lv < nb);
+            const LB deep = push & (2 * node < Lv);
+            const uint64_t mp = ballot(push), md = ballot(deep), ml = ballot(leaf);
+            const LI rp = nn + 2 * mbcnt(mp) + 2 * mbcnt(md);
+            const LI first = select(deep, 4 * node, 2 * node);
+            const LB okp = push & (rp + select(deep, LI(3), LI(1)) < kFrontCap);
+            lds_st(&L.front[cur ^ 1][0], select(okp, rp, LI(0)), first, okp);
+            lds_st(&L.front[cur ^ 1][0], select(okp, rp + 1, LI(0)), first + 1, okp);
+            const LB okd = okp & deep;
+            lds_st(&L.front[cur ^ 1][0], select(okd, rp + 2, LI(0)), first + 2, okd);
+            lds_st(&L.front[cur ^ 1][0], select(okd, rp + 3, LI(0)), first + 3, okd);
+            const LI rl = nbk + mbcnt(ml);
+            lds_st(L.near_list, select(rl < kNearCap, rl, LI(0)), node - Lv, leaf & (rl < kNearCap));
+            nn += 2 * popc64(mp) + 2 * popc64(md);
+            nbk += popc64(ml);
+        }
+        wave_sync();
+        if (nn > kFrontCap || nbk > kNearCap) return -1;
+        nf = nn;
+        cur ^= 1;
+    }
+    return nbk;
+}
+
+// The listed seeds q with lo < d2 <= hi of the cells of the two halves
+// (seeds ca, cb at a, b; hi < 0: none wanted) into L.cand and L.cand_b as
+// (d2 bits << 32 | q), unsorted.  na, nb receive their numbers (only the
+// first kCandCap are stored).
+template <class LDS>
+VGC_HD void near_scan(const ClipParams& P, LDS& L, const NearList& N, int ca, int cb, const pf4& a,
+                      const pf4& b, float loa, float hia, float lob, float hib, int& na, int& nb) {
+    const LI lane = lane_id();
+    const int p0 = P.IL.p0[N.inst], n = P.IL.n[N.inst], Lv = P.IL.L[N.inst];
+    const bnode* T = P.nodes + P.IL.t0[N.inst];
+    int nbk = 0;
+    for (int base = 0; base < N.n; base += kWave) {
+        const LI idx = base + lane;
+        const LB in = idx < N.n;
+        const LI bk = lds_ld(L.near_list, select(in, idx, LI(0)));
+        const BoxLanes B = load_box(T, bk + Lv, in);
+        const LF ax = vmaxf(vmaxf(B.lx - a.x, a.x - B.hx), 0.0f);
+        const LF ay = vmaxf(vmaxf(B.ly - a.y, a.y - B.hy), 0.0f);
+        const LF az = vmaxf(vmaxf(B.lz - a.z, a.z - B.hz), 0.0f);
+        const LF bx = vmaxf(vmaxf(B.lx - b.x, b.x - B.hx), 0.0f);
+        const LF by = vmaxf(vmaxf(B.ly - b.y, b.y - B.hy), 0.0f);
+        const LF bz = vmaxf(vmaxf(B.lz - b.z, b.z - B.hz), 0.0f);
+        const LB hit = in & ((ax * ax + ay * ay + az * az <= hia) | (bx * bx + by * by + bz * bz <= hib));
+        const uint64_t m = ballot(hit);
+        const LI r = nbk + mbcnt(m);
+        lds_st(L.bucket, select(hit, r, LI(0)) & (kBucketCap - 1), bk, hit & (r < kBucketCap));
+        nbk += popc64(m);
+    }
+    wave_sync();
+    if (nbk > kBucketCap) {
+        // more than kBucketCap buckets around one cell: more seeds than a
+        // ring holds
+        na = nb = kBucketCap * kBucket;
+        return;
+    }
+    na = nb = 0;
+    for (int base = 0; base < nbk; base += kWave / kBucket) {
+        const LI bi = base + (lane >> 4);
+        const LB inb = bi < nbk;
+        const LI m = p0 + lds_ld(L.bucket, select(inb, bi, LI(0))) * kBucket + (lane & (kBucket - 1));
+        const LB ok = inb & (m < p0 + n);
+        const SeedLanes q = lane_seed(P.pf, select(ok, m, LI(p0)), ok);
+        const LF ax = q.x - a.x, ay = q.y - a.y, az = q.z - a.z;
+        const LF bx = q.x - b.x, by = q.y - b.y, bz = q.z - b.z;
+        const LF da = ax * ax + ay * ay + az * az, db = bx * bx + by * by + bz * bz;
+        const uint64_t ta = ballot(ok & (da > loa) & (da <= hia) & (m != ca));
+        const uint64_t tb = ballot(ok & (db > lob) & (db <= hib) & (m != cb));
+        const LU64 id = cvt<uint64_t>(cvt<uint32_t>(m));
+        const LI ra = na + mbcnt(ta), rb = nb + mbcnt(tb);
+        lds_st(L.cand, ra & (kCandCap - 1), (cvt<uint64_t>(fbits(da)) << LU64(32)) | id,
+               mask_bit(ta) & (ra < kCandCap));
+        lds_st(L.cand_b, rb & (kCandCap - 1), (cvt<uint64_t>(fbits(db)) << LU64(32)) | id,
+               mask_bit(tb) & (rb < kCandCap));
+        na += popc64(ta);
+        nb += popc64(tb);
+    }
+    wave_sync();
+}
+
+// The nearest of the ring's n <= kCandCap unsorted candidates src into out in
+// ascending order, at most kStageCap: of more, those within a lowered bound
+// that keeps 52 .. kStageCap of them where the distances allow (the others are
+// gathered again if the cell still needs them).  rhi2 is lowered to that
+// bound; returns the count, -1 when more than kStageCap share one distance.
+// Sorted by counting: a lane's rank is the number of keys below its own (two
+// instructions per key, against 21 rounds of compares and LDS traffic of a
+// bitonic network).
+VGC_HD int ring_sort(uint64_t* src, int n, float& rhi2, uint64_t* out) {
+    const LI lane = lane_id();
+    const LB in0 = lane < n;
+    LU64 a = lds_ld(src, select(in0, lane, LI(0)));
+    if (n > kStageCap) {
+        const LB in1 = lane + kWave < n;
+        const LU64 b = lds_ld(src, select(in1, lane + kWave, LI(0)));
+        const LF da = from_bits(cvt<uint32_t>(a >> LU64(32))), db = from_bits(cvt<uint32_t>(b >> LU64(32)));
+        float lo = 0.0f, hi = rhi2, best = 0.0f;
+        int keep = 0;
+        for (int it = 0; it < 32; ++it) {
+            const float t = it == 0 ? hi * (0.4f + 0.6f * 58.0f / float(n)) : 0.5f * (lo + hi);
+            const int k = popc64(ballot(in0 & (da <= t))) + popc64(ballot(in1 & (db <= t)));
+            if (k > kStageCap) {
+                hi = t;
+                continue;
+            }
+            lo = t;
+            if (k > keep) {
+                keep = k;
+                best = t;
+            }
+            if (k >= 52) break;
+        }
+        if (keep == 0) return -1;
+        rhi2 = uni(best);
+        // the kept ones together (every key read before the first write)
+        const LB ka = in0 & (da <= rhi2), kb = in1 & (db <= rhi2);
+        const uint64_t ma = ballot(ka), mb = ballot(kb);
+        wave_sync();
+        lds_st(src, select(ka, mbcnt(ma), LI(0)), a, ka);
+        lds_st(src, select(kb, popc64(ma) + mbcnt(mb), LI(0)), b, kb);
+        wave_sync();
+        n = keep;
+        a = lds_ld(src, select(lane < n, lane, LI(0)));
+    }
+    LI rank = LI(0);
+    for (int i = 0; i < n; ++i) rank = rank + select(lds_ld(src, LI(i)) < a, LI(1), LI(0));
+    lds_st(out, select(lane < n, rank, LI(0)), a, lane < n);
+    wave_sync();
+    return n;
+}
+
 // ------------------------------------------------------------- the pair
 
 // The next ring of half h, gathered and sorted into L.h[h].key (c: the seed;
 // first: no ring yet).  Returns the candidate count, -1 when the cell is
 // complete, -2 when the cell is left to the FP64 pass.
 template <bool W>
-VGC_HD int pair_ring(const ClipParams& P, PairLds& L, const PairState& st, int h, bool first) {
+VGC_HD int pair_ring(const ClipParams& P, PairLds& L, const PairState& st, const NearList& N, int h,
+                     bool first) {
     PairCtl& K = L.ctl[h];
     const int c = uni(K.c), inst = uni(K.inst);
     float rlo2 = uni(K.rlo2), rhi2 = uni(K.rhi2);
@@ -556,6 +743,17 @@ VGC_HD int pair_ring(const ClipParams& P, PairLds& L, const PairState& st, int h
         if (uni(need2 <= rhi2 || rhi2 >= all2)) return -1;
         rlo2 = rhi2;
         rhi2 = need2 < all2 ? need2 : all2;
+        if (uni(inst == N.inst && rhi2 <= N.r2)) {
+            int n, none;
+            near_scan(P, L, N, c, c, pq, pq, rlo2, rhi2, 0.0f, -1.0f, n, none);
+            if (n <= kCandCap) {
+                n = ring_sort(L.cand, n, rhi2, L.h[h].key);
+                K.rlo2 = rlo2;
+                K.rhi2 = rhi2;
+                wave_sync();
+                return n < 0 ? -2 : n;
+            }
+        }
         // filter of the partial cell: its corners by id over the wave
         CellRun<1, float> R;
         R.pc = pc;
@@ -591,19 +789,20 @@ VGC_HD int pair_ring(const ClipParams& P, PairLds& L, const PairState& st, int h
         if (uni(!(nh > lo * 1.000001f) || !(nh < rhi2))) return -2;
         rhi2 = nh;
     }
-    rank_cand(L, n, L.h[h].key);
+    n = ring_sort(L.cand, n, rhi2, L.h[h].key);
     K.rlo2 = rlo2;
     K.rhi2 = rhi2;
     K.nfilt = nfilt;
     K.ct_on = ct_on;
     wave_sync();
-    return n;
+    return n < 0 ? -2 : n;
 }
 
-// Items item0 and item0 + 1 (the second may be missing).
+// Items item0 and item0 + 1 (the second may be missing); near2: squared
+// radius of the first ring (0: unknown).
 template <bool W, bool COUNT>
-VGC_HD void process_pair(const ClipParams& P, int item0, PairLds& L) {
-    const LI lane = lane_id();
+VGC_HD void process_pair(const ClipParams& P, int item0, PairLds& L, const NearList& N, float near2) {
+    const LI lane = lane_id_here();
     const LB up = lane >= 32;
     const LI hl = lane & 31;
     wave_sync();  // the previous pair of this wave is done with the LDS
@@ -625,35 +824,18 @@ VGC_HD void process_pair(const ClipParams& P, int item0, PairLds& L) {
     uint64_t live = ballot(on);
     if (live == 0) return;
 
-    // first ring of each cell, about 56 seeds: 2.4 times the distance to the
-    // 4th nearest seed of its own bucket
+    // the first ring: the radius of the wave's bucket list (or, without one,
+    // the radius that holds about 60 seeds of a cloud spread over the box)
     LF scale;
     {
-        const LI p0 = gld(P.IL.p0, inst, LB(true)), n = gld(P.IL.n, inst, LB(true));
-        const SeedLanes p = lane_seed(P.pf, c, LB(true));
-        const LI m0 = c - ((c - p0) & (kBucket - 1));
-        const LI m = m0 + (lane & (kBucket - 1));
-        const LB ok = (m < p0 + n) & (m != c);
-        const SeedLanes q = lane_seed(P.pf, select(ok, m, m0), ok);
-        const LF dx = q.x - p.x, dy = q.y - p.y, dz = q.z - p.z;
-        const LF d2 = select(ok, dx * dx + dy * dy + dz * dz, LF(INFINITY));
-        LI below = LI(0);
-#pragma unroll
-        for (int k = 1; k < kBucket; ++k) below = below + select(row_ror(d2, k) < d2, LI(1), LI(0));
-        const uint64_t fourth = ballot((below == 3) & (d2 < INFINITY));
-        const uint64_t fa = fourth & kLoHalf, fb = fourth & kHiHalf;
-        const float ra = fa ? 5.8f * readlane(d2, ffs64(fa)) : 0.0f;
-        const float rb = fb ? 5.8f * readlane(d2, ffs64(fb)) : 0.0f;
-        LF rhi2 = select(up, LF(rb), LF(ra));
+        const LI n = gld(P.IL.n, inst, LB(true));
         const LI b6 = inst * 6;
         const LF bx = cvt<float>(gld(P.box, b6 + 3, LB(true)) - gld(P.box, b6 + 0, LB(true)));
         const LF by = cvt<float>(gld(P.box, b6 + 4, LB(true)) - gld(P.box, b6 + 1, LB(true)));
         const LF bz = cvt<float>(gld(P.box, b6 + 5, LB(true)) - gld(P.box, b6 + 2, LB(true)));
         const LF all2 = (bx * bx + by * by + bz * bz) * 1.0002f;
-        // (fewer than four other seeds in the bucket, or copies: the radius
-        // that holds as many of seeds spread over the box)
         const LF nf = cvt<float>(n);
-        rhi2 = select(rhi2 > 0.0f, rhi2, 1.9f * all2 / vcbrtf(nf * nf));
+        const LF rhi2 = near2 > 0.0f ? LF(near2) : 1.9f * all2 / vcbrtf(nf * nf);
         // the power of two that brings the ring's radius to 1 .. 2
         scale = pow2_inv_sqrt(rhi2);
         const LB m0l = hl == 0;
@@ -718,29 +900,57 @@ VGC_HD void process_pair(const ClipParams& P, int item0, PairLds& L) {
     // ------------------------------------------------ security-radius loop
     const uint64_t have_m = halves(st.valid[0]);
     uint64_t done = 0, empty = 0;  // halves finished; the others of have_m fail
-    LI cnt = LI(0), pos = LI(0);   // candidates of the ring; the next to stage
-    uint64_t first = kLoHalf | kHiHalf;
+    LI cnt = LI(0);                // candidates of the ring
+    uint64_t first = kLoHalf | kHiHalf, more = kLoHalf | kHiHalf;
     PairWork work{};
     const LI soff4 = select(up, LI(int(sizeof(PairStage)) / 16), LI(0));
     const LI soff2 = select(up, LI(int(sizeof(PairStage)) / 8), LI(0));
     const LI koff = select(up, LI(int(sizeof(PairHalf)) / 8), LI(0));
+    if (N.inst >= 0 && ballot(inst != N.inst) == 0) {
+        // both first rings in one scan of the wave's buckets
+        const int ca = uni(L.ctl[0].c), cb = uni(L.ctl[1].c);
+        int n2[2];
+        near_scan(P, L, N, ca, cb, P.pf[ca], P.pf[cb], -1.0f, (live & kLoHalf) ? near2 : -1.0f, -1.0f,
+                  (live & kHiHalf) ? near2 : -1.0f, n2[0], n2[1]);
+#pragma unroll 1
+        for (int h = 0; h < 2; ++h) {
+            if (!(live & half_mask(h))) continue;
+            float r2 = near2;
+            if (n2[h] > kCandCap) {
+                // too many: once more within the radius that holds about 64
+                const float f = cbrtf(64.0f / float(n2[h]));
+                r2 *= f * f;
+                int none;
+                const int ch = h ? cb : ca;
+                near_scan(P, L, N, ch, ch, P.pf[ch], P.pf[ch], -1.0f, h ? -1.0f : r2, -1.0f,
+                          h ? r2 : -1.0f, h ? none : n2[h], h ? n2[h] : none);
+                // (copies without an end: the cell's own walk)
+                if (n2[h] > kCandCap) continue;
+            }
+            const int k = ring_sort(h ? L.cand_b : L.cand, n2[h], r2, L.h[h].key);
+            L.ctl[h].rhi2 = r2;
+            if (k < 0) continue;
+            first &= ~half_mask(h);
+            more &= ~half_mask(h);
+            cnt = select(mask_bit(half_mask(h)), LI(k), cnt);
+        }
+        wave_sync();
+    }
     while (live) {
-        // candidates for every live half: the next batch of its ring, or the
-        // next ring
-        const uint64_t more = live & ballot(pos >= cnt);
+        // the next ring of every live half
 #pragma unroll 1
         for (int h = 0; h < 2; ++h) {
             const uint64_t hm = half_mask(h);
-            if (!(more & hm)) continue;
-            const int n = pair_ring<W>(P, L, st, h, (first & hm) != 0);
+            if (!(live & more & hm)) continue;
+            const int n = pair_ring<W>(P, L, st, N, h, (first & hm) != 0);
             first &= ~hm;
             if (n < 0) {
                 live &= ~hm;
                 if (n == -1) done |= hm;
             }
             cnt = select(mask_bit(hm), LI(n), cnt);
-            pos = select(mask_bit(hm), LI(0), pos);
         }
+        more = kLoHalf | kHiHalf;
         LI n = LI(0);  // staged now
 #pragma unroll 1
         for (int h = 0; h < 2; ++h) {
@@ -750,7 +960,7 @@ VGC_HD void process_pair(const ClipParams& P, int item0, PairLds& L) {
             const pt4 pc = P.pts[ch];
             const int k = pair_stage<W>(P, L, h, uni(L.ctl[h].scale), pc,
                                         W ? pc.w - P.wmax[uni(L.ctl[h].inst)] : 0.0,
-                                        readlane(pos, 32 * h), readlane(cnt, 32 * h));
+                                        readlane(cnt, 32 * h));
             if (k < 0) live &= ~hm;
             n = select(mask_bit(hm), LI(k), n);
         }
@@ -776,7 +986,7 @@ VGC_HD void process_pair(const ClipParams& P, int item0, PairLds& L) {
                 uu |= ~ballot(vabs(t1) > b1) & st.valid[1];
                 ss |= ballot(st.num[1] >= rho * st.den2[1]) & st.valid[1];
             }
-            // batch at its end, security radius reached, sign not certified,
+            // ring at its end, security radius reached, sign not certified,
             // plane cuts: in this order
             uint64_t rem = run & ballot(k < n);
             const uint64_t reach = rem & ~halves(ss);
@@ -801,7 +1011,7 @@ VGC_HD void process_pair(const ClipParams& P, int item0, PairLds& L) {
             k = k + select(mask_bit(run), LI(1), LI(0));
             if (run) continue;
             if (pend == 0) break;
-            const LI j = cvt<int>(cvt<uint32_t>(lds_ld(&L.h[0].key[0], koff + pos + ks)));
+            const LI j = cvt<int>(cvt<uint32_t>(lds_ld(&L.h[0].key[0], koff + ks)));
             if (COUNT) {
                 if (pend & kLoHalf) work.nclip[0]++;
                 if (pend & kHiHalf) work.nclip[1]++;
@@ -818,7 +1028,6 @@ VGC_HD void process_pair(const ClipParams& P, int item0, PairLds& L) {
             pend = 0;
             if (run == 0) break;
         }
-        pos = select(pos + kStageCap < cnt, pos + kStageCap, cnt);
     }
 
     if (COUNT && lane0()) {
@@ -1032,6 +1241,29 @@ VGC_HD void process_pair(const ClipParams& P, int item0, PairLds& L) {
     gst(P.nbr_cnt, ocl, select(up, LI(out[1]), LI(out[0])), w0);
     gst(P.flags, cl, LU(uint32_t(CELL_DONE)), w0);
     if (P.e2) gst(P.e2, ocl, half_sum(e2a), w0);
+}
+
+// Items first .. first + count - 1 (at most 16), two at a time, by one
+// wavefront.
+template <bool W, bool COUNT>
+VGC_HD void process_pairs(const ClipParams& P, int first, int count, PairLds& L) {
+    wave_sync();  // the previous cells of this wave are done with the LDS
+    NearList N;
+    const LI lane = lane_id();
+    const LB has = lane < count;
+    const LI item = first + select(has, lane, LI(0));
+    const LI c = P.items ? gld(P.items, item, LB(true)) : item;
+    const int c0 = readlane(c, 0);
+    const int inst = P.inst_of ? P.inst_of[c0] : 0;
+    N.inst = inst;
+    const float d4 = uni(near_spacing(P, c0, inst, count > 2 ? kBucket / 4 : 1));
+    const float ring2 = (kNearRing * d4) * (kNearRing * d4);
+    N.r2 = (kNearList * d4) * (kNearList * d4);
+    bool one = d4 > 0.0f;
+    if (P.inst_of) one = one && ballot(gld(P.inst_of, c, LB(true)) != inst) == 0;
+    N.n = one ? near_buckets(P, L, inst, c, has, N.r2) : -1;
+    if (N.n < 0) N.inst = -1;
+    for (int k = 0; k < count; k += 2) process_pair<W, COUNT>(P, first + k, L, N, ring2);
 }
 
 }  // namespace vgc

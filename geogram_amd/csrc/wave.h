@@ -293,6 +293,8 @@ inline LI lane_id() {
     return r;
 }
 
+inline LI lane_id_here() { return lane_id(); }
+
 inline uint64_t ballot(const LB& b) {
     uint64_t m = 0;
     for (int i = 0; i < kWave; ++i)
@@ -494,6 +496,13 @@ VGC_HD T gld(const T* base, int idx, bool m) {
 }
 
 VGC_HD int lane_id() { return __lane_id(); }
+// the same, opaque to the optimiser: what a loop derives from it is formed
+// in each turn instead of being kept in registers across the loop
+VGC_HD int lane_id_here() {
+    int l = __lane_id();
+    asm volatile("" : "+v"(l));
+    return l;
+}
 
 VGC_HD uint64_t ballot(bool b) { return __ballot(b); }
 
