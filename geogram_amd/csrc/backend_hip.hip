@@ -215,7 +215,7 @@ __global__ void k_radius_fill(const pf4* __restrict__ pf, const bnode* __restric
     wide[t] = c < 0 ? 1 : 0;
 }
 
-// The flagged radius queries, one wavefront each (a grid of waves strides
+// The flagged radius queries (all of them if wide is null), one wavefront each (a grid of waves strides
 // over the queries): the tree level by level, 64 nodes per step, each
 // level's passing nodes kept in order in the wave's scratch (two buffers of
 // fstride >= L nodes), then the seeds of the passing leaves, four leaves
@@ -236,7 +236,7 @@ __global__ __launch_bounds__(64) void k_radius_wide(const pf4* __restrict__ pf,
     int* fa = front + (long long)blockIdx.x * 2 * fstride;
     int* fb = fa + fstride;
     for (int t = blockIdx.x; t < ni; t += gridDim.x) {
-        if (!wide[t]) continue;  // uniform over the wave
+        if (wide && !wide[t]) continue;  // uniform over the wave
         const int q = items[t];
         const int inst = IL.inst_of ? IL.inst_of[q] : 0;
         const pf4 pq = pf[q];
@@ -1672,6 +1672,11 @@ struct HipBackend {
     void radius_count(const pf4* pf, const bnode* nodes, const InstLayout& IL, const int* items,
                       int ni, const float* rho2, const PowerFilter* filt, int* cnt) {
         if (ni <= 0) return;
+        if (ni <= wide_waves()) {
+            radius_wide(pf, nodes, IL, items, ni, rho2, filt, nullptr, cnt, nullptr, 0, nullptr, nullptr);
+            check();
+            return;
+        }
         unsigned char* wide = wide_flags(ni);
         k_radius_count<<<blocks_for(ni, 64), 64, 0, stream_>>>(pf, nodes, IL, items, ni, rho2, filt,
                                                                cnt, wide);
@@ -1682,20 +1687,32 @@ struct HipBackend {
                      int ni, const float* rho2, const PowerFilter* filt, const long long* off,
                      long long base, int* list, float* d2) {
         if (ni <= 0) return;
+        if (ni <= wide_waves()) {
+            radius_wide(pf, nodes, IL, items, ni, rho2, filt, nullptr, nullptr, off, base, list, d2);
+            check();
+            return;
+        }
         unsigned char* wide = wide_flags(ni);
         k_radius_fill<<<blocks_for(ni, 64), 64, 0, stream_>>>(pf, nodes, IL, items, ni, rho2, filt,
                                                               off, base, list, d2, wide);
         radius_wide(pf, nodes, IL, items, ni, rho2, filt, wide, nullptr, off, base, list, d2);
         check();
     }
-    // the flagged queries by k_radius_wide: up to 64 waves, each with two
-    // frontier buffers of tree_leaves_ nodes (at most 256 MB in all)
+    // wavefronts of k_radius_wide at most: each has two frontier buffers of
+    // tree_leaves_ nodes, 256 MB in all.  Up to that many queries are walked
+    // by a wavefront each from the start: a lane's walk of 512 nodes is one
+    // chain of dependent loads (0.7 ms for the two queries of the 2M mixture,
+    // by wavefronts 0.05 ms; the lists are the same).
+    long long wide_waves() const {
+        const long long g = (256ll << 20) / (2 * sizeof(int) * std::max(1ll, (long long)tree_leaves_));
+        return std::max(1ll, std::min(g, 256ll));
+    }
+    // the flagged queries by k_radius_wide
     void radius_wide(const pf4* pf, const bnode* nodes, const InstLayout& IL, const int* items,
                      int ni, const float* rho2, const PowerFilter* filt, const unsigned char* wide,
                      int* cnt, const long long* off, long long base, int* list, float* d2) {
         const long long fstride = std::max(1, tree_leaves_);
-        long long g = (256ll << 20) / (2 * sizeof(int) * fstride);
-        g = std::max(1ll, std::min(g, std::min(64ll, (long long)ni)));
+        const long long g = std::min(wide_waves(), (long long)ni);
         const long long need = g * 2 * fstride;
         if (wide_front_cap_ < need) {
             if (wide_front_) VGC_HIP_CHECK(hipFree(wide_front_));

@@ -187,6 +187,9 @@ struct ClipParams {
     // its cells per wavefront (even, at most 16)
     int fp32;
     int group;
+    // the FP32 first pass: neighbour ids and facet areas wanted (else only
+    // their number)
+    int faces;
 };
 
 template <int S>

@@ -1117,13 +1117,26 @@ VGC_HD void process_pair(const ClipParams& P, int item0, PairLds& L, const NearL
 #pragma unroll
             for (int a = 0; a < 4; ++a) e[k][a] = lds_ld(&L.in[0].row[0][0], o8 + p3[k] * 4 + a);
         }
-        const Corner C = make_corner(e[0][0], e[0][1], e[0][2], e[0][3], e[1][0], e[1][1], e[1][2],
-                                             e[1][3], e[2][0], e[2][1], e[2][2], e[2][3]);
-        r2f = vmax(r2f, select(vs, C.r2, LD(0.0)));
-        const LD inv = 1.0 / select(vs, C.d, LD(1.0));
-        lds_st(&L.in[0].q[0][0], o8 + cid * 3 + 0, C.nx * inv, vs);
-        lds_st(&L.in[0].q[0][0], o8 + cid * 3 + 1, C.ny * inv, vs);
-        lds_st(&L.in[0].q[0][0], o8 + cid * 3 + 2, C.nz * inv, vs);
+        // N and D as make_corner forms them (FP32 certified that the corner
+        // is not degenerate: no magnitudes here, and one division)
+        const LD bcx = vfma(e[1][1], e[2][2], -(e[1][2] * e[2][1])),
+                 bcy = vfma(e[1][2], e[2][0], -(e[1][0] * e[2][2])),
+                 bcz = vfma(e[1][0], e[2][1], -(e[1][1] * e[2][0]));
+        const LD cax = vfma(e[2][1], e[0][2], -(e[2][2] * e[0][1])),
+                 cay = vfma(e[2][2], e[0][0], -(e[2][0] * e[0][2])),
+                 caz = vfma(e[2][0], e[0][1], -(e[2][1] * e[0][0]));
+        const LD abx = vfma(e[0][1], e[1][2], -(e[0][2] * e[1][1])),
+                 aby = vfma(e[0][2], e[1][0], -(e[0][0] * e[1][2])),
+                 abz = vfma(e[0][0], e[1][1], -(e[0][1] * e[1][0]));
+        const LD nx = vfma(e[0][3], bcx, vfma(e[1][3], cax, e[2][3] * abx));
+        const LD ny = vfma(e[0][3], bcy, vfma(e[1][3], cay, e[2][3] * aby));
+        const LD nz = vfma(e[0][3], bcz, vfma(e[1][3], caz, e[2][3] * abz));
+        const LD inv = 1.0 / vfma(e[0][0], bcx, vfma(e[0][1], bcy, e[0][2] * bcz));
+        const LD qx = nx * inv, qy = ny * inv, qz = nz * inv;
+        r2f = vmax(r2f, select(vs, vfma(qx, qx, vfma(qy, qy, qz * qz)), LD(0.0)));
+        lds_st(&L.in[0].q[0][0], o8 + cid * 3 + 0, qx, vs);
+        lds_st(&L.in[0].q[0][0], o8 + cid * 3 + 1, qy, vs);
+        lds_st(&L.in[0].q[0][0], o8 + cid * 3 + 2, qz, vs);
         lds_st(L.in[0].cpl, o4 + cid, st.pl[s], vs);
         lds_st(L.in[0].cadj, o4 + cid, st.adj[s], vs);
 #pragma unroll
@@ -1151,7 +1164,9 @@ VGC_HD void process_pair(const ClipParams& P, int item0, PairLds& L, const NearL
         const LI fs = select(inr, f, LI(0));
         LI t0 = lds_ld(L.in[0].v2t, o4 + fs);
         const LB act = finl & inr & (t0 != LI(0x7FFFFFFF));
-        t0 = select(act, t0, LI(0)) & 63;
+        // (lanes without a face walk from the apex, adding zeros: every point
+        // they read is one of the cell)
+        t0 = select(act, t0, apex) & 63;
         const LU fu = cvt<uint32_t>(fs);
         auto nxt = [&](const LI& t) -> LI {
             const LU plt = lds_ld(L.in[0].cpl, o4 + t);
@@ -1167,35 +1182,46 @@ VGC_HD void process_pair(const ClipParams& P, int item0, PairLds& L, const NearL
            q1z = lds_ld(Q, o8 + t1 * 3 + 2);
         LD area = LD(0.0), fv = LD(0.0), fmx = LD(0.0), fmy = LD(0.0), fmz = LD(0.0), fe = LD(0.0);
         const LD oq0 = (ox * ox + oy * oy + oz * oz) + (q0x * q0x + q0y * q0y + q0z * q0z);
+        const LD ux = q0x - ox, uy = q0y - oy, uz = q0z - oz;
+        const LD rx = ox + q0x, ry = oy + q0y, rz = oz + q0z;
+        LD vx = q1x - ox, vy = q1y - oy, vz = q1z - oz;
+        LD ax = q1x - q0x, ay = q1y - q0y, az = q1z - q0z;
         LB go = act & (t != t0);
         for (int guard = 0; guard < 64 && any(go); ++guard) {
             const LD qx = lds_ld(Q, o8 + t * 3 + 0), qy = lds_ld(Q, o8 + t * 3 + 1),
                      qz = lds_ld(Q, o8 + t * 3 + 2);
-            // tetrahedron and triangle terms exactly as in process_cell
-            const LD ux = q0x - ox, uy = q0y - oy, uz = q0z - oz;
-            const LD vx = q1x - ox, vy = q1y - oy, vz = q1z - oz;
+            // tetrahedron and triangle terms exactly as in process_cell, the
+            // differences of the previous point carried along; a lane whose
+            // face is done adds zeros
             const LD wx = qx - ox, wy = qy - oy, wz = qz - oz;
             const LD cx = uy * vz - uz * vy, cy = uz * vx - ux * vz, cz = ux * vy - uy * vx;
-            const LD tv = vabs(cx * wx + cy * wy + cz * wz) * (1.0 / 6.0);
-            const LD ax = q1x - q0x, ay = q1y - q0y, az = q1z - q0z;
-            const LD bx = qx - q0x, by = qy - q0y, bz = qz - q0z;
-            const LD wx2 = ay * bz - az * by, wy2 = az * bx - ax * bz, wz2 = ax * by - ay * bx;
-            const LD ta = 0.5 * vsqrt(wx2 * wx2 + wy2 * wy2 + wz2 * wz2);
+            const LD tv = select(go, vabs(cx * wx + cy * wy + cz * wz) * (1.0 / 6.0), LD(0.0));
             if (COUNT) ntet = ntet + select(go, LI(1), LI(0));
-            fv = select(go, fv + tv, fv);
-            const LD sx = ox + q0x + q1x + qx, sy = oy + q0y + q1y + qy, sz = oz + q0z + q1z + qz;
-            fmx = select(go, fmx + tv * sx / 4.0, fmx);
-            fmy = select(go, fmy + tv * sy / 4.0, fmy);
-            fmz = select(go, fmz + tv * sz / 4.0, fmz);
+            fv = fv + tv;
+            const LD sx = rx + q1x + qx, sy = ry + q1y + qy, sz = rz + q1z + qz;
+            fmx = fmx + tv * sx / 4.0;
+            fmy = fmy + tv * sy / 4.0;
+            fmz = fmz + tv * sz / 4.0;
             if (P.e2) {
                 const LD nn = oq0 + (q1x * q1x + q1y * q1y + q1z * q1z) + (qx * qx + qy * qy + qz * qz) +
                               (sx * sx + sy * sy + sz * sz);
-                fe = select(go, fe + tv * nn * (1.0 / 20.0), fe);
+                fe = fe + tv * nn * (1.0 / 20.0);
             }
-            area = select(go, area + ta, area);
-            q1x = select(go, qx, q1x);
-            q1y = select(go, qy, q1y);
-            q1z = select(go, qz, q1z);
+            if (P.faces) {
+                const LD bx = qx - q0x, by = qy - q0y, bz = qz - q0z;
+                const LD wx2 = ay * bz - az * by, wy2 = az * bx - ax * bz, wz2 = ax * by - ay * bx;
+                const LD ta = 0.5 * vsqrt(wx2 * wx2 + wy2 * wy2 + wz2 * wz2);
+                area = area + select(go, ta, LD(0.0));
+                ax = bx;
+                ay = by;
+                az = bz;
+            }
+            q1x = qx;
+            q1y = qy;
+            q1z = qz;
+            vx = wx;
+            vy = wy;
+            vz = wz;
             const LI tn = nxt(t);
             t = select(go, tn, t);
             go = go & (t != t0);
@@ -1213,12 +1239,14 @@ VGC_HD void process_pair(const ClipParams& P, int item0, PairLds& L, const NearL
         const LI pg = s == 0 ? pgv[0] : pgv[1];
         const LB outm = act & (pg >= 0);
         const uint64_t om = ballot(outm);
-        const LI rank = half_rank(om, out[0], out[1], up);
-        const LI oj0 = gld(P.orig, select(outm, pg, LI(0)), outm);
-        const LI oj = P.src ? gld(P.src, select(outm, oj0, LI(0)), outm) : oj0;
-        const Lane<long long> at = obase + cvt<long long>(rank);
-        gst(P.nbr_tmp, at, oj, outm);
-        gst(P.area_tmp, at, area, outm);
+        if (P.faces) {
+            const LI rank = half_rank(om, out[0], out[1], up);
+            const LI oj0 = gld(P.orig, select(outm, pg, LI(0)), outm);
+            const LI oj = P.src ? gld(P.src, select(outm, oj0, LI(0)), outm) : oj0;
+            const Lane<long long> at = obase + cvt<long long>(rank);
+            gst(P.nbr_tmp, at, oj, outm);
+            gst(P.area_tmp, at, area, outm);
+        }
         out[0] += popc_half(om, 0);
         out[1] += popc_half(om, 1);
     }

@@ -522,6 +522,7 @@ public:
         P.nbr_tmp = d_nbr_tmp;
         P.area_tmp = d_area_tmp;
         P.face_stride = kFaceStride;
+        P.faces = pb.want_neighbors ? 1 : 0;
         P.flags = d_flags;
         P.r2 = d_r2;
         P.ball = (fball*)slot(S_BALL, sizeof(fball) * (size_t)n_);
