@@ -10,12 +10,14 @@ from __future__ import annotations
 import os
 import subprocess
 import sys
+import tempfile
+from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 
 HIP_FLAGS = [
-    "-std=c++17", "-O3", "--offload-arch=gfx950", "-fPIC", "-shared",
+    "-std=c++17", "-O3", "--offload-arch=gfx950", "-fPIC",
     # no implicit FMA contraction: the error bounds of the sign tests and the
     # bit-for-bit agreement with the emulation assume the written operations
     "-ffp-contract=off",
@@ -29,9 +31,19 @@ def _run(cmd):
     subprocess.run(cmd, check=True, cwd=CSRC)
 
 
+# translation units of libvgc.so (the clipping kernels in parts)
+HIP_UNITS = [("backend", "backend_hip.hip", [])] + [
+    (f"clip{k}", "clip_kernels.hip", [f"-DVGC_CLIP_PART={k}"]) for k in range(5)]
+
+
 def build_gpu():
     out = os.path.join(HERE, "libvgc.so")
-    _run(["hipcc", *HIP_FLAGS, "-o", out + ".tmp", "backend_hip.hip"])
+    with tempfile.TemporaryDirectory() as tmp:
+        objs = [os.path.join(tmp, name + ".o") for name, _, _ in HIP_UNITS]
+        with ThreadPoolExecutor(len(HIP_UNITS)) as ex:
+            list(ex.map(_run, [["hipcc", *HIP_FLAGS, *defs, "-c", "-o", obj, src]
+                               for (_, src, defs), obj in zip(HIP_UNITS, objs)]))
+        _run(["hipcc", "--offload-arch=gfx950", "-shared", "-o", out + ".tmp", *objs])
     os.replace(out + ".tmp", out)
     return out
 

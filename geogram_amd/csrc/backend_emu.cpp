@@ -808,9 +808,22 @@ struct EmuBackend {
         }
     }
     void knn_seed_radius(const pf4* pf, const bnode* nodes, const InstLayout& IL, const pf4* qf,
-                         const int* qpos, int nq, int kk, double e, float* rr) {
+                         const int* qpos, const int* items, int nq, int kk, double e, float* rr) {
 #pragma omp parallel for schedule(dynamic, 64)
-        for (int t = 0; t < nq; ++t) rr[t] = knn_seed_radius_row(pf, nodes, IL, qf, qpos, t, kk, e);
+        for (int i = 0; i < nq; ++i) {
+            const int t = items ? items[i] : i;
+            rr[t] = knn_seed_radius_row(pf, nodes, IL, qf, qpos, t, kk, e);
+        }
+    }
+    void knn_wave(const KnnParams& K) {
+#pragma omp parallel
+        {
+            std::unique_ptr<KnnLds> L(new KnnLds());
+            std::memset(L.get(), 0, sizeof(KnnLds));
+#pragma omp for schedule(dynamic, 8)
+            for (int t = 0; t < K.nq; t += kKnnGroup)
+                process_knn(K, t, std::min(kKnnGroup, K.nq - t), *L);
+        }
     }
     void knn_count(const pf4* pf, const bnode* nodes, const InstLayout& IL, const pf4* qf,
                    const int* items, int ni, const float* rr, int* cnt) {

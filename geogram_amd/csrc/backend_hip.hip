@@ -21,6 +21,7 @@
 #include <string>
 
 #include "api_impl.h"
+#include "clip_launch.h"
 #include "mlp.h"
 #include "ot_kernels.h"
 
@@ -135,42 +136,6 @@ __global__ __launch_bounds__(256) void k_knn(const pf4* __restrict__ pf,
     if (t >= nq) return;
     int q = queries ? queries[t] : t;
     knn_query<K>(pf, nodes, IL, q, out + (size_t)t * K, out_d2 ? out_d2 + (size_t)t * K : nullptr);
-}
-
-// Work-groups go to the 8 XCDs of the chip in turn; renumber them so that
-// each XCD takes one contiguous range of work-groups (cells in Morton order:
-// neighbouring cells read the same seeds and tree nodes, from that XCD's L2).
-// A bijection of [0, gridDim.x).
-constexpr int kXcds = 8;
-__device__ __forceinline__ int xcd_block() {
-    const int nb = gridDim.x, b = blockIdx.x;
-    const int q = nb / kXcds, r = nb % kXcds, x = b % kXcds;
-    return x * q + (x < r ? x : r) + b / kXcds;
-}
-
-// S = 1 with FP64 signs (every cell's first pass, and the second gather):
-// registers capped at 128 for 4 waves per SIMD (some spill to scratch); with
-// one-wave work-groups that measured 7 % faster than 168 registers and 3
-// waves — the wait for dependent LDS and memory round trips is hidden by
-// occupancy.  The exact re-clip (a few cells) keeps its registers.
-template <int S, int WAVES, bool EXACT, bool GATHER, bool W, bool CORNER = W>
-__global__ __launch_bounds__(64 * WAVES, (S == 1 && !EXACT) ? 4 : 1) void k_clip(ClipParams P) {
-    __shared__ CellLds<S> lds[WAVES];
-    const int wave = WAVES == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int item = xcd_block() * WAVES + wave;
-    if (item >= P.n_items) return;  // whole wavefront
-    process_cell<S, EXACT, GATHER, W, CORNER>(P, item, lds[wave]);
-}
-
-// The first pass with FP32 corner state: two cells per wavefront
-// (pair_cell.h).
-template <int WAVES, bool W, bool COUNT>
-__global__ __launch_bounds__(64 * WAVES, 4) void k_pair(ClipParams P) {
-    __shared__ PairLds lds[WAVES];
-    const int wave = WAVES == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int first = P.group * (xcd_block() * WAVES + wave);
-    if (first >= P.n_items) return;  // whole wavefront
-    process_pairs<W, COUNT>(P, first, min(P.group, P.n_items - first), lds[wave]);
 }
 
 __global__ void k_radius_r2(const int* __restrict__ items, int ni, const pt4* __restrict__ pts,
@@ -456,10 +421,23 @@ template <int W>
 __global__ __launch_bounds__(256) void k_knn_seed_radius(const pf4* __restrict__ pf,
                                                          const bnode* __restrict__ nodes,
                                                          InstLayout IL, const pf4* __restrict__ qf,
-                                                         const int* __restrict__ qpos, int nq,
+                                                         const int* __restrict__ qpos,
+                                                         const int* __restrict__ items, int nq,
                                                          int kk, double e, float* rr) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < nq) rr[t] = knn_seed_radius_row<W>(pf, nodes, IL, qf, qpos, t, kk, e);
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= nq) return;
+    const int t = items ? items[i] : i;
+    rr[t] = knn_seed_radius_row<W>(pf, nodes, IL, qf, qpos, t, kk, e);
+}
+
+// Exact kNN by a wavefront per kKnnGroup queries (knn_wave.h).  Against a lane
+// per query (radius by a top-8 walk, count and fill walks, two segmented
+// sorts): 100k points, k = 16: 7.0 -> 0.6 ms of kernels; the lane walks were
+// chains of dependent loads on 1.5 wavefronts per SIMD.
+__global__ __launch_bounds__(64, 4) void k_knn_wave(KnnParams K) {
+    __shared__ KnnLds lds;
+    const int first = kKnnGroup * xcd_block();
+    process_knn(K, first, min(kKnnGroup, K.nq - first), lds);
 }
 
 __global__ void k_knn_count(const pf4* __restrict__ pf, const bnode* __restrict__ nodes,
@@ -1589,75 +1567,19 @@ struct HipBackend {
         }
         check();
     }
-    template <bool E, bool G, bool W>
-    void clip_egw(int S, const ClipParams& P) {
-        const unsigned g4 = blocks_for(P.n_items, 4), g1 = blocks_for(P.n_items, 1);
-        if (S == 1) {
-            if constexpr (G && !W) {
-                if (P.corner) {
-                    // second gather of Voronoi cells, with the corner test
-                    k_clip<1, 1, E, G, W, true><<<g1, 64, 0, stream_>>>(P);
-                    return;
-                }
-            }
-            if (waves_ == 1)
-                k_clip<1, 1, E, G, W><<<g1, 64, 0, stream_>>>(P);
-            else
-                k_clip<1, 4, E, G, W><<<g4, 256, 0, stream_>>>(P);
-        } else if (S == 2) {
-            k_clip<2, 4, E, G, W><<<g4, 256, 0, stream_>>>(P);
-        } else if (S == 4) {
-            k_clip<4, 1, E, G, W><<<g1, 64, 0, stream_>>>(P);
-        } else {
-            // 512 corners: list mode only (the last tier)
-            if constexpr (!G)
-                k_clip<8, 1, E, false, W><<<g1, 64, 0, stream_>>>(P);
-            else
-                throw std::runtime_error("clip: 512-corner cells run from lists only");
-        }
-    }
-    // Cells per wavefront of k_pair: 8, which share one walk of the tree, once
-    // that leaves enough wavefronts for the 4096 resident ones to even out,
-    // else 4 or 2.
-    static int pair_group(int n) { return n >= 400000 ? 8 : n >= 150000 ? 4 : 2; }
-    template <bool W, bool COUNT>
-    void clip_pairs(const ClipParams& P) {
-        ClipParams Q = P;
-        Q.group = pair_group(P.n_items);
-        if (waves_ == 1)
-            k_pair<1, W, COUNT><<<blocks_for(Q.n_items, Q.group), 64, 0, stream_>>>(Q);
-        else
-            k_pair<4, W, COUNT><<<blocks_for(Q.n_items, 4 * Q.group), 256, 0, stream_>>>(Q);
-    }
-    template <bool E, bool G>
-    void clip_eg(int S, const ClipParams& P) {
-        if (P.weighted)
-            clip_egw<E, G, true>(S, P);
-        else
-            clip_egw<E, G, false>(S, P);
-    }
     // wavefronts per work-group of the S = 1 kernels (1 or 4); the cells'
     // results do not depend on it
     void set_clip_waves(int w) { waves_ = w == 1 ? 1 : 4; }
     int clip_waves() const { return waves_; }
     void clip(int S, bool exact, bool gather, const ClipParams& P) {
         if (P.n_items <= 0) return;
-        if (P.fp32) {
-            if (P.weighted)
-                P.counters ? clip_pairs<true, true>(P) : clip_pairs<true, false>(P);
-            else
-                P.counters ? clip_pairs<false, true>(P) : clip_pairs<false, false>(P);
-        } else if (exact) {
-            if (gather)
-                clip_eg<true, true>(S, P);
-            else
-                clip_eg<true, false>(S, P);
-        } else {
-            if (gather)
-                clip_eg<false, true>(S, P);
-            else
-                clip_eg<false, false>(S, P);
-        }
+        if (P.fp32)
+            launch_pairs(P, waves_, stream_);
+        else if (exact)
+            gather ? launch_clip_exact_gather(S, P, waves_, stream_)
+                   : launch_clip_exact_list(S, P, waves_, stream_);
+        else
+            gather ? launch_clip_gather(S, P, waves_, stream_) : launch_clip_list(S, P, waves_, stream_);
         check();
     }
     void radius_r2(const int* items, int ni, const pt4* pts, const double* r2, const int* inst_of,
@@ -2153,23 +2075,26 @@ struct HipBackend {
         if (nq > 0) k_lower_bound_u64<<<blocks_for(nq, 256), 256, 0, stream_>>>(keys, n, q, nq, out);
         check();
     }
+    // items: the queries wanted (nullptr: all nq)
     void knn_seed_radius(const pf4* pf, const bnode* nodes, const InstLayout& IL, const pf4* qf,
-                         const int* qpos, int nq, int kk, double e, float* rr) {
+                         const int* qpos, const int* items, int nq, int kk, double e, float* rr) {
         // kk <= 8: the narrowest walk that holds kk (the radius of the
         // 16-wide walk); kk > 16: the 8th nearest scaled, a first guess like
-        // the scaled 16th (the lists are exact either way).  On the surface
-        // leg (327,680 triangles, 100k seeds, 33-NN lists) the call took
-        // 47 ms with the 16th, 27 ms with the 8th, 31 ms with the 4th.
+        // the scaled 16th (the lists are exact either way).
         const unsigned g = blocks_for(nq, 256);
         if (kk == 1)
-            k_knn_seed_radius<1><<<g, 256, 0, stream_>>>(pf, nodes, IL, qf, qpos, nq, kk, e, rr);
+            k_knn_seed_radius<1><<<g, 256, 0, stream_>>>(pf, nodes, IL, qf, qpos, items, nq, kk, e, rr);
         else if (kk <= 4)
-            k_knn_seed_radius<4><<<g, 256, 0, stream_>>>(pf, nodes, IL, qf, qpos, nq, kk, e, rr);
+            k_knn_seed_radius<4><<<g, 256, 0, stream_>>>(pf, nodes, IL, qf, qpos, items, nq, kk, e, rr);
         else if (kk <= 8 || kk > kKnnSeedK)
-            k_knn_seed_radius<8><<<g, 256, 0, stream_>>>(pf, nodes, IL, qf, qpos, nq, kk, e, rr);
+            k_knn_seed_radius<8><<<g, 256, 0, stream_>>>(pf, nodes, IL, qf, qpos, items, nq, kk, e, rr);
         else
-            k_knn_seed_radius<kKnnSeedK><<<g, 256, 0, stream_>>>(pf, nodes, IL, qf, qpos, nq, kk, e,
-                                                                 rr);
+            k_knn_seed_radius<kKnnSeedK><<<g, 256, 0, stream_>>>(pf, nodes, IL, qf, qpos, items, nq,
+                                                                 kk, e, rr);
+        check();
+    }
+    void knn_wave(const KnnParams& K) {
+        if (K.nq > 0) k_knn_wave<<<blocks_for(K.nq, kKnnGroup), 64, 0, stream_>>>(K);
         check();
     }
     void knn_count(const pf4* pf, const bnode* nodes, const InstLayout& IL, const pf4* qf,

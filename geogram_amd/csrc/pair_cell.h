@@ -548,13 +548,13 @@ VGC_HD float near_spacing(const ClipParams& P, int c, int inst, int passes) {
     return cnt > 0.0f ? sum / cnt : 0.0f;
 }
 
-// The buckets of instance inst within sqrt(r2) of the box of the wave's
-// seeds (items [i0, i1) with their Morton positions c per lane) into
-// L.near_list; returns their number, -1 when they or the walk overflow.
+// The buckets of instance inst within sqrt(r2) of the box of the points p of
+// the lanes in `has` into L.near_list; returns their number, -1 when they or
+// the walk overflow.
 template <class LDS>
-VGC_HD int near_buckets(const ClipParams& P, LDS& L, int inst, const LI& c, const LB& has, float r2) {
+VGC_HD int near_buckets(const ClipParams& P, LDS& L, int inst, const SeedLanes& p, const LB& has,
+                        float r2) {
     const LI lane = lane_id();
-    const SeedLanes p = lane_seed(P.pf, c, has);
     const float hx = wave_maxf(select(has, p.x, LF(-INFINITY))), lx = -wave_maxf(select(has, -p.x, LF(-INFINITY)));
     const float hy = wave_maxf(select(has, p.y, LF(-INFINITY))), ly = -wave_maxf(select(has, -p.y, LF(-INFINITY)));
     const float hz = wave_maxf(select(has, p.z, LF(-INFINITY))), lz = -wave_maxf(select(has, -p.z, LF(-INFINITY)));
@@ -1289,7 +1289,7 @@ VGC_HD void process_pairs(const ClipParams& P, int first, int count, PairLds& L)
     N.r2 = (kNearList * d4) * (kNearList * d4);
     bool one = d4 > 0.0f;
     if (P.inst_of) one = one && ballot(gld(P.inst_of, c, LB(true)) != inst) == 0;
-    N.n = one ? near_buckets(P, L, inst, c, has, N.r2) : -1;
+    N.n = one ? near_buckets(P, L, inst, lane_seed(P.pf, c, has), has, N.r2) : -1;
     if (N.n < 0) N.inst = -1;
     for (int k = 0; k < count; k += 2) process_pair<W, COUNT>(P, first + k, L, N, ring2);
 }

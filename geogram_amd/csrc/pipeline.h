@@ -32,6 +32,7 @@
 #include <vector>
 
 #include "common.h"
+#include "knn_wave.h"
 
 namespace vgc {
 
@@ -328,11 +329,48 @@ public:
         }
         const double e = knn_vec_err(S);
         float* rr = (float*)slot(S_QR2, sizeof(float) * (size_t)nq);
-        be_.knn_seed_radius(d_pf, d_nodes, IL, qf, qpos, nq, kk, e, rr);
         std::vector<int> items;
         bool all = true;
         int* d_redo = (int*)slot(S_QREDO, sizeof(int) * (size_t)nq);
         unsigned* d_nredo = (unsigned*)slot(S_CENS_N, sizeof(unsigned));
+        if (kk <= kKnnWaveMax) {
+            // a wavefront per few queries; those it leaves go through the
+            // lists below
+            KnnParams K{};
+            K.C.pts = d_pts;
+            K.C.orig = d_orig;
+            K.C.pf = d_pf;
+            K.C.nodes = d_nodes;
+            K.C.IL = IL;
+            K.qp = qp;
+            K.qf = qf;
+            K.qpos = qpos;
+            K.qrow = qrow;
+            K.nq = nq;
+            K.kk = kk;
+            K.n = n_;
+            K.self_rule = self_rule ? 1 : 0;
+            K.e = e;
+            K.out_idx = d_idx;
+            K.out_d2 = d_d2;
+            K.fail = d_redo;
+            K.nfail = d_nredo;
+            be_.dzero(d_nredo, sizeof(unsigned));
+            be_.knn_wave(K);
+            unsigned nf = 0;
+            be_.d2h(&nf, d_nredo, sizeof(unsigned));
+            items.resize(nf);
+            if (nf) be_.d2h(items.data(), d_redo, sizeof(int) * nf);
+            std::sort(items.begin(), items.end());
+            all = false;
+            if (nf) {
+                int* d_items = (int*)slot(S_ITEMS, sizeof(int) * (size_t)nf);
+                be_.h2d(d_items, items.data(), sizeof(int) * (size_t)nf);
+                be_.knn_seed_radius(d_pf, d_nodes, IL, qf, qpos, d_items, (int)nf, kk, e, rr);
+            }
+        } else {
+            be_.knn_seed_radius(d_pf, d_nodes, IL, qf, qpos, nullptr, nq, kk, e, rr);
+        }
         for (int round = 0;; ++round) {
             const int ni = all ? nq : (int)items.size();
             if (ni == 0) break;
