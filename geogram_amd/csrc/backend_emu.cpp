@@ -140,14 +140,14 @@ struct EmuBackend {
 
     // the first pass with FP32 corner state, two cells per wavefront
     void clip_pairs(const ClipParams& P) {
-        constexpr int kGroup = 16;  // cells per wavefront (the results do not depend on it)
+        const int group = pair_group(P.n_items);
 #pragma omp parallel
         {
             std::unique_ptr<PairLds> L(new PairLds());
             std::memset(L.get(), 0, sizeof(PairLds));
 #pragma omp for schedule(dynamic, 8)
-            for (int it = 0; it < P.n_items; it += kGroup) {
-                const int m = std::min(kGroup, P.n_items - it);
+            for (int it = 0; it < P.n_items; it += group) {
+                const int m = std::min(group, P.n_items - it);
                 if (P.weighted) {
                     if (P.counters)
                         process_pairs<true, true>(P, it, m, *L);

@@ -432,7 +432,7 @@ __global__ __launch_bounds__(256) void k_knn_seed_radius(const pf4* __restrict__
 
 // Exact kNN by a wavefront per kKnnGroup queries (knn_wave.h).  Against a lane
 // per query (radius by a top-8 walk, count and fill walks, two segmented
-// sorts): 100k points, k = 16: 7.0 -> 0.6 ms of kernels; the lane walks were
+// sorts): 100k points, k = 16: 7.0 -> 0.43 ms of kernels; the lane walks were
 // chains of dependent loads on 1.5 wavefronts per SIMD.
 __global__ __launch_bounds__(64, 4) void k_knn_wave(KnnParams K) {
     __shared__ KnnLds lds;

@@ -91,6 +91,11 @@ constexpr int kMaxFilteredRings = 48;  // power-filtered rings of the first pass
 // a second gather with the corner test (clustered seeds: large cells beside
 // dense clusters, whose balls hold thousands of seeds that cannot cut)
 constexpr int kMaxVoronoiRings = 16;
+// the same of the FP32 first pass, whose cells go straight to the second
+// gather: a cell of many rings beside a dense cluster holds up its whole
+// launch.
+constexpr int kMaxPairRings = 4;
+constexpr int kMaxPairRingsW = 12;
 constexpr double kGamma9 = 1.2e-15;  // > gamma_9 for the conflict determinant
 constexpr double kGamma5 = 0.8e-15;  // > gamma_5 for the corner determinant D
 
@@ -187,6 +192,7 @@ struct ClipParams {
     // its cells per wavefront (even, at most 16)
     int fp32;
     int group;
+    int pair_rings;  // its filtered rings before the cell goes to the second gather
     // the FP32 first pass: neighbour ids and facet areas wanted (else only
     // their number)
     int faces;

@@ -88,10 +88,6 @@ __global__ __launch_bounds__(64 * WAVES, 4) void k_pair(ClipParams P) {
     process_pairs<W, COUNT>(P, first, min(P.group, P.n_items - first), lds[wave]);
 }
 
-// Cells per wavefront of k_pair: 8, which share one walk of the tree, once
-// that leaves enough wavefronts for the 4096 resident ones to even out,
-// else 4 or 2.
-static inline int pair_group(int n) { return n >= 400000 ? 8 : n >= 150000 ? 4 : 2; }
 template <bool W, bool COUNT>
 static void clip_pairs(const ClipParams& P, int waves, hipStream_t stream) {
     ClipParams Q = P;

@@ -12,7 +12,7 @@
 
 namespace vgc {
 
-constexpr int kKnnWaveMax = 64;
+constexpr int kKnnWaveMax = 96;
 constexpr int kKnnGroup = 8;
 constexpr int kKnnTries = 8;
 
@@ -71,8 +71,8 @@ VGC_HD void knn_wave_query(const KnnParams& K, KnnLds& L, const NearList& N, int
             continue;
         }
         if (n < K.kk && n < K.n) {
-            const float f = cbrtf((1.4f * K.kk + 4.0f) / float(n > 0 ? n : 1));
-            r2 = uni(r2 * f * f * 1.1f);
+            const float f = cbrtf((1.2f * K.kk + 4.0f) / float(n > 0 ? n : 1));
+            r2 = uni(r2 * f * f);
             continue;
         }
         // FP64 distances and caller's indices of the listed points
@@ -132,9 +132,12 @@ VGC_HD void knn_wave_query(const KnnParams& K, KnnLds& L, const NearList& N, int
         }
         const int have = empty ? 0 : K.kk - skip;
         if (have < kout) {
-            const LB pad = (lane >= have) & (lane < kout);
-            gst(K.out_idx, base + cvt<long long>(lane), LI(-1), pad);
-            gst(K.out_d2, base + cvt<long long>(lane), LD(-1.0), pad);
+            for (int k0 = 0; k0 < kout; k0 += kWave) {
+                const LI k = lane + k0;
+                const LB pad = (k >= have) & (k < kout);
+                gst(K.out_idx, base + cvt<long long>(k), LI(-1), pad);
+                gst(K.out_d2, base + cvt<long long>(k), LD(-1.0), pad);
+            }
         }
         return;
     }
@@ -148,8 +151,10 @@ VGC_HD void process_knn(const KnnParams& K, int first, int count, KnnLds& L) {
     const LI t = first + select(has, lane, LI(0));
     const int c0 = K.qpos ? K.qpos[first] : first;
     const float d4 = uni(near_spacing(K.C, c0, 0, 1));
-    // kNearRing spacings hold about 60 points; a quarter more than wanted
-    const float r = kNearRing * d4 * cbrtf((1.25f * K.kk + 8.0f) * (1.0f / 60.0f));
+    // kNearRing spacings hold about 60 points; a quarter more than wanted, and
+    // within the candidate buffer
+    const float want = fminf(1.25f * K.kk + 8.0f, 108.0f);
+    const float r = kNearRing * d4 * cbrtf(want * (1.0f / 60.0f));
     NearList N;
     N.inst = 0;
     N.r2 = (1.25f * r) * (1.25f * r);

@@ -28,8 +28,9 @@
 //
 // A cell that needs anything rare (a sign or corner that FP32 cannot certify,
 // more than 64 corners or planes, a coincident or duplicate seed, a walk that
-// outgrows its buffers, the ring limit) is flagged CELL_UNCERTAIN without
-// outputs; the FP64 first pass redoes it from the start.
+// outgrows its buffers) is flagged CELL_UNCERTAIN without outputs; the FP64
+// first pass redoes it from the start.  One that uses up its rings goes to the
+// second gather.
 #pragma once
 
 #include "clip_cell.h"
@@ -715,7 +716,8 @@ VGC_HD int ring_sort(uint64_t* src, int n, float& rhi2, uint64_t* out) {
 
 // The next ring of half h, gathered and sorted into L.h[h].key (c: the seed;
 // first: no ring yet).  Returns the candidate count, -1 when the cell is
-// complete, -2 when the cell is left to the FP64 pass.
+// complete, -2 when the cell is left to the FP64 pass, -3 when it has used up
+// its rings.
 template <bool W>
 VGC_HD int pair_ring(const ClipParams& P, PairLds& L, const PairState& st, const NearList& N, int h,
                      bool first) {
@@ -777,7 +779,7 @@ VGC_HD int pair_ring(const ClipParams& P, PairLds& L, const PairState& st, const
     while (true) {
         n = first ? gather_ring(P, L, c, inst, pq.x, pq.y, pq.z, rlo2, rhi2, F)
                   : gather_dfs<W>(P, L, c, inst, pq.x, pq.y, pq.z, rlo2, rhi2, F, CT, ct_on);
-        if (F.on && ++nfilt > P.ring_limit) return -2;
+        if (F.on && ++nfilt > P.pair_rings) return -3;
         if (n >= 0 && n <= kCandCap) break;
         // too many seeds (or tree nodes): narrow the ring, same shell-volume
         // fraction in r^3, and gather again
@@ -900,6 +902,7 @@ VGC_HD void process_pair(const ClipParams& P, int item0, PairLds& L, const NearL
     // ------------------------------------------------ security-radius loop
     const uint64_t have_m = halves(st.valid[0]);
     uint64_t done = 0, empty = 0;  // halves finished; the others of have_m fail
+    uint64_t rings = 0;            // of those: out of rings
     LI cnt = LI(0);                // candidates of the ring
     uint64_t first = kLoHalf | kHiHalf, more = kLoHalf | kHiHalf;
     PairWork work{};
@@ -947,6 +950,7 @@ VGC_HD void process_pair(const ClipParams& P, int item0, PairLds& L, const NearL
             if (n < 0) {
                 live &= ~hm;
                 if (n == -1) done |= hm;
+                if (n == -3) rings |= hm;
             }
             cnt = select(mask_bit(hm), LI(n), cnt);
         }
@@ -1043,7 +1047,9 @@ VGC_HD void process_pair(const ClipParams& P, int item0, PairLds& L, const NearL
     const LB lead = hl == 0;
     {
         const LB failed = mask_bit(have_m & ~(done | empty)) & lead;
-        gst(P.flags, cl, LU(uint32_t(CELL_UNCERTAIN)), failed);
+        gst(P.flags, cl,
+            select(mask_bit(rings), LU(uint32_t(CELL_NEED_K | CELL_WHY_RINGS)), LU(uint32_t(CELL_UNCERTAIN))),
+            failed);
         const LB em = mask_bit(empty) & lead;
         gst(P.r2, cl, LD(0.0), failed | em);
         if (empty) {
@@ -1293,5 +1299,10 @@ VGC_HD void process_pairs(const ClipParams& P, int first, int count, PairLds& L)
     if (N.n < 0) N.inst = -1;
     for (int k = 0; k < count; k += 2) process_pair<W, COUNT>(P, first + k, L, N, ring2);
 }
+
+// Cells per wavefront of k_pair: 8, which share one walk of the tree, once
+// that leaves enough wavefronts for the 4096 resident ones to even out,
+// else 4 or 2.
+static inline int pair_group(int n) { return n >= 400000 ? 8 : n >= 150000 ? 4 : 2; }
 
 }  // namespace vgc

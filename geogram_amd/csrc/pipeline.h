@@ -598,12 +598,13 @@ public:
         P.list_stride = K0;
         P.list_complete = 0;
         P.ring_limit = weighted_ ? kMaxFilteredRings : kMaxVoronoiRings;
+        P.pair_rings = weighted_ ? kMaxPairRingsW : kMaxPairRings;
         P.corner = 0;
         // FP32 corner state for the first pass, except for cell meshes (those
         // are emitted by the FP64 pass) and for a few passes after one that
-        // had to redo more than 5 % of its cells in FP64 (large Laguerre
-        // weights: there the FP64 pass alone is faster; the outputs are the
-        // same either way)
+        // had to redo more than half of its cells in FP64 (ties everywhere,
+        // as on lattices; the FP32 pass costs less than half of the FP64
+        // one, and the outputs are the same either way)
         P.fp32 = (gather && !fp64_first && !pb.mesh_mode && fp32_skip_ == 0) ? 1 : 0;
         if (fp32_skip_ > 0) --fp32_skip_;
         if (pb.abort_on_empty) {
@@ -697,7 +698,7 @@ public:
                 if (cf[i] & CELL_UNCERTAIN) redo.push_back(cc[i]);
             std::sort(redo.begin(), redo.end());
             st.nb_fp64_redo += redo.size();
-            if (redo.size() * 20 > (size_t)P.n_items) fp32_skip_ = kFp32Skip;
+            if (redo.size() * 2 > (size_t)P.n_items) fp32_skip_ = kFp32Skip;
             if (!redo.empty()) {
                 int* d_items = (int*)slot(S_ITEMS, sizeof(int) * redo.size());
                 be_.h2d(d_items, redo.data(), sizeof(int) * redo.size());
@@ -1278,7 +1279,7 @@ private:
     double* d_r2_ = nullptr;  // squared radius per cell of the last pass (Morton order)
     std::vector<int> h_p0_, h_n_, h_b0_, h_nb_, h_L_;
     // first passes left to run with FP64 corners (after an FP32 pass that
-    // redid more than 5 % of its cells)
+    // redid more than half of its cells)
     static constexpr int kFp32Skip = 8;
     int fp32_skip_ = 0;
     std::vector<int> piece_cells_;  // cells of this pass computed in pieces
