@@ -800,17 +800,18 @@ VGC_HD int pair_ring(const ClipParams& P, PairLds& L, const PairState& st, const
     return n < 0 ? -2 : n;
 }
 
-// Items item0 and item0 + 1 (the second may be missing); near2: squared
+// Items item0 and item0 + 1 (the second only if below end); near2: squared
 // radius of the first ring (0: unknown).
 template <bool W, bool COUNT>
-VGC_HD void process_pair(const ClipParams& P, int item0, PairLds& L, const NearList& N, float near2) {
+VGC_HD void process_pair(const ClipParams& P, int item0, int end, PairLds& L, const NearList& N,
+                         float near2) {
     const LI lane = lane_id_here();
     const LB up = lane >= 32;
     const LI hl = lane & 31;
     wave_sync();  // the previous pair of this wave is done with the LDS
     // a cell's scalars are held by every lane of its half
     const LI item = select(up, LI(item0 + 1), LI(item0));
-    const LB have = item < P.n_items;
+    const LB have = item < end;
     const LI items = select(have, item, LI(item0));
     const LI c = P.items ? gld(P.items, items, LB(true)) : items;
     const LI inst = P.inst_of ? gld(P.inst_of, c, LB(true)) : LI(0);
@@ -1297,12 +1298,13 @@ VGC_HD void process_pairs(const ClipParams& P, int first, int count, PairLds& L)
     if (P.inst_of) one = one && ballot(gld(P.inst_of, c, LB(true)) != inst) == 0;
     N.n = one ? near_buckets(P, L, inst, lane_seed(P.pf, c, has), has, N.r2) : -1;
     if (N.n < 0) N.inst = -1;
-    for (int k = 0; k < count; k += 2) process_pair<W, COUNT>(P, first + k, L, N, ring2);
+    for (int k = 0; k < count; k += 2) process_pair<W, COUNT>(P, first + k, first + count, L, N, ring2);
 }
 
 // Cells per wavefront of k_pair: 8, which share one walk of the tree, once
 // that leaves enough wavefronts for the 4096 resident ones to even out,
-// else 4 or 2.
-static inline int pair_group(int n) { return n >= 400000 ? 8 : n >= 150000 ? 4 : 2; }
+// else 4 or 2; 1 where the chip stays half empty anyway and the time is that
+// of one wavefront.
+static inline int pair_group(int n) { return n >= 400000 ? 8 : n >= 150000 ? 4 : n > 4096 ? 2 : 1; }
 
 }  // namespace vgc
