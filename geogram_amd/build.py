@@ -33,7 +33,7 @@ def _run(cmd):
 
 # translation units of libvgc.so (the clipping kernels in parts)
 HIP_UNITS = [("backend", "backend_hip.hip", [])] + [
-    (f"clip{k}", "clip_kernels.hip", [f"-DVGC_CLIP_PART={k}"]) for k in range(5)]
+    (f"clip{k}", "clip_kernels.hip", [f"-DVGC_CLIP_PART={k}"]) for k in range(6)]
 
 
 def build_gpu():

@@ -151,6 +151,15 @@ int api_cells(Ctx<B>* ctx, const double* xyz, const double* w, const uint32_t* i
                 pb.d_w = dw;
             }
         }
+        if (dev && !pb.periodic) {
+            // straight into the caller's arrays
+            pb.out_vol = vol;
+            pb.out_mg = mg;
+            pb.out_ptr = (long long*)nbr_ptr;
+            pb.out_nbr = nbr;
+            pb.out_area = farea;
+            pb.out_cap = (long long)std::min<uint64_t>(cap, 1ull << 62);
+        }
         EngineStats es;
         ctx->eng.autotune = (flags & VGC_AUTOTUNE) != 0;
         ctx->eng.waves4 = (flags & VGC_WAVES4) != 0;
@@ -162,7 +171,7 @@ int api_cells(Ctx<B>* ctx, const double* xyz, const double* w, const uint32_t* i
         }
         Engine<B>& E = ctx->eng;
         auto out = [&](void* dst, const void* src, size_t bytes) {
-            if (!dst) return;
+            if (!dst || dst == src) return;
             if (dev)
                 be.d2d(dst, src, bytes);
             else
@@ -174,6 +183,7 @@ int api_cells(Ctx<B>* ctx, const double* xyz, const double* w, const uint32_t* i
         fill_stats(es, stats);
         if (nbr || farea) {
             if ((uint64_t)E.total_neighbors > cap) {
+                be.sync();
                 ctx->err = "vgc_cells: neighbour capacity too small";
                 return VGC_ERR_CAPACITY;
             }
@@ -265,24 +275,28 @@ int api_cvt_func_grad(Ctx<B>* ctx, const double* xyz, uint32_t n, const double* 
     }
 }
 
-// Bounding box of n FP64 points (device memory copied to the host when
-// dev) for the Morton quantisation, and their largest coordinate magnitude.
+// Bounding box of n FP64 points (reduced on the device when dev) for the
+// Morton quantisation, and their largest coordinate magnitude.
 template <class B>
-void host_extent(B& be, const double* xyz, uint32_t n, bool dev, double lo[3], double hi[3],
-                 double& S) {
-    std::vector<double> hx;
-    const double* hp = xyz;
+void point_extent(Ctx<B>* ctx, const double* xyz, uint32_t n, bool dev, double lo[3], double hi[3],
+                  double& S) {
     if (dev) {
-        hx.resize(3 * (size_t)n);
-        be.d2h(hx.data(), xyz, sizeof(double) * 3 * (size_t)n);
-        hp = hx.data();
-    }
-    for (int c = 0; c < 3; ++c) lo[c] = hi[c] = hp[c];
-    for (uint32_t i = 0; i < n; ++i)
+        double* d = (double*)ctx->staging(7, sizeof(double) * 6);
+        ctx->be.extent(xyz, (long long)n, d);
+        double h[6];
+        ctx->be.d2h(h, d, sizeof(h));
         for (int c = 0; c < 3; ++c) {
-            lo[c] = std::min(lo[c], hp[3 * (size_t)i + c]);
-            hi[c] = std::max(hi[c], hp[3 * (size_t)i + c]);
+            lo[c] = h[c];
+            hi[c] = h[3 + c];
         }
+    } else {
+        for (int c = 0; c < 3; ++c) lo[c] = hi[c] = xyz[c];
+        for (uint32_t i = 0; i < n; ++i)
+            for (int c = 0; c < 3; ++c) {
+                lo[c] = std::min(lo[c], xyz[3 * (size_t)i + c]);
+                hi[c] = std::max(hi[c], xyz[3 * (size_t)i + c]);
+            }
+    }
     S = 0.0;
     for (int c = 0; c < 3; ++c) S = std::max(S, std::max(std::fabs(lo[c]), std::fabs(hi[c])));
 }
@@ -316,10 +330,10 @@ int knn_common(Ctx<B>* ctx, const char* name, const double* xyz, uint32_t n, con
         pb.n_inst = 1;
         pb.inst_n = {(int)n};
         double lo[3], hi[3], S;
-        host_extent(be, xyz, n, dev, lo, hi, S);
+        point_extent(ctx, xyz, n, dev, lo, hi, S);
         if (!self) {
             double qlo[3], qhi[3], qS;
-            host_extent(be, q, nq, dev, qlo, qhi, qS);
+            point_extent(ctx, q, nq, dev, qlo, qhi, qS);
             S = std::max(S, qS);
         }
         if (!(S < 1e300)) {
@@ -1235,7 +1249,7 @@ int nearest_masses(Ctx<B>* ctx, const double* dx, const std::vector<double>& hnu
     B& be = ctx->be;
     Engine<B>& E = ctx->eng;
     double lo[3], hi[3], S;
-    host_extent(be, dx, n, true, lo, hi, S);
+    point_extent(ctx, dx, n, true, lo, hi, S);
     if (!(S < 1e300)) {
         E.error = "coordinates must be finite";
         return 1;
@@ -1448,8 +1462,8 @@ int api_surface_centroids(Ctx<B>* ctx, const double* xyz, uint32_t n, const doub
         pb.n_inst = 1;
         pb.inst_n = {(int)n};
         double lo[3], hi[3], S, vlo[3], vhi[3], vS;
-        host_extent(be, xyz, n, dev, lo, hi, S);
-        host_extent(be, vtx, nv, dev, vlo, vhi, vS);
+        point_extent(ctx, xyz, n, dev, lo, hi, S);
+        point_extent(ctx, vtx, nv, dev, vlo, vhi, vS);
         S = std::max(S, vS);
         if (!(S < 1e300)) {
             ctx->err = std::string(name) + ": coordinates must be finite";

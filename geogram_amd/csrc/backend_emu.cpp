@@ -30,6 +30,10 @@ struct EmuBackend {
     void dfree(void* p) { std::free(p); }
     void h2d(void* d, const void* s, size_t b) { std::memcpy(d, s, b); }
     void d2h(void* d, const void* s, size_t b) { std::memcpy(d, s, b); }
+    void d2h2(void* d, const void* s, size_t b, void* d2, const void* s2, size_t b2) {
+        std::memcpy(d, s, b);
+        std::memcpy(d2, s2, b2);
+    }
     void d2d(void* d, const void* s, size_t b) { std::memmove(d, s, b); }
     void dzero(void* d, size_t b) { std::memset(d, 0, b); }
     void sync() {}
@@ -94,26 +98,35 @@ struct EmuBackend {
         }
     }
 
-    void bvh_leaves(const pt4* pts, const InstLayout& IL, bnode* nodes, const long long* leaf_off,
-                    int ni, long long) {
-        for (int inst = 0; inst < ni; ++inst)
-            for (long long l = 0; l < leaf_off[inst + 1] - leaf_off[inst]; ++l)
-                bvh_leaf(pts, IL, nodes, inst, (int)l);
-    }
-
-    void bvh_level(const InstLayout& IL, bnode* nodes, const long long*, int ni, long long, int h) {
+    void bvh_build(const pt4* pts, const InstLayout& IL, bnode* nodes, const long long*, int ni,
+                   long long, int) {
         for (int inst = 0; inst < ni; ++inst) {
-            int L = IL.L[inst];
-            for (int k = L >> h; k < (2 * L) >> h; ++k) bvh_merge(nodes, IL.t0[inst], k);
+            const int L = IL.L[inst];
+            for (int l = 0; l < L; ++l) bvh_leaf(pts, IL, nodes, inst, l);
+            for (int k = L - 1; k > 0; --k) bvh_merge(nodes, IL.t0[inst], k);
         }
     }
 
-    void wmax(const pt4* pts, const InstLayout& IL, int ni, double* out) {
+    void wmax(const pt4* pts, const InstLayout& IL, int ni, int, double* out) {
         for (int inst = 0; inst < ni; ++inst) {
             double m = -INFINITY;
             for (int s = IL.p0[inst]; s < IL.p0[inst] + IL.n[inst]; ++s) m = std::fmax(m, pts[s].w);
             out[inst] = m;
         }
+    }
+
+    void extent(const double* xyz, long long n, double* out) {
+        for (int c = 0; c < 3; ++c) {
+            out[c] = INFINITY;
+            out[3 + c] = -INFINITY;
+        }
+        for (long long i = 0; i < n; ++i)
+            for (int c = 0; c < 3; ++c) {
+                out[c] = std::fmin(out[c], xyz[3 * i + c]);
+                out[3 + c] = std::fmax(out[3 + c], xyz[3 * i + c]);
+            }
+        for (int c = 0; c < 6; ++c)
+            if (std::isnan(xyz[c % 3])) out[c] = xyz[c % 3];
     }
 
     template <int K>
@@ -218,6 +231,13 @@ struct EmuBackend {
         }
     }
 
+    void clip_listed(const ClipParams& P, const int* items, const unsigned* d_count) {
+        ClipParams Q = P;
+        Q.items = items;
+        Q.n_items = (int)*d_count;
+        clip(1, false, true, Q);
+    }
+
     int det4_sign(const double* r) { return det4_sign_exact(r, r + 4, r + 8, r + 12); }
 
     void radius_r2(const int* items, int ni, const pt4* pts, const double* r2, const int* inst_of,
@@ -253,22 +273,22 @@ struct EmuBackend {
         for (int t = 0; t < n; ++t) out[t] = off[t] - base;
     }
 
-    unsigned census(const int* items, int n_items, const uint32_t* flags, uint32_t mask,
-                    const unsigned* skip, const int* inst_of, int* out_cell, uint32_t* out_flag,
-                    unsigned* d_count) {
-        unsigned k = 0;
+    void census(const int* items, int n_items, const uint32_t* flags, uint32_t any, uint32_t all,
+                const unsigned* skip, const int* inst_of, int* out_cell, unsigned* out_pair,
+                unsigned* d_count) {
         for (int t = 0; t < n_items; ++t) {
             const int c = items ? items[t] : t;
             if (skip && skip[inst_of ? inst_of[c] : 0]) continue;
             const uint32_t f = flags[c];
-            if ((f & mask) || !(f & CELL_DONE)) {
-                out_cell[k] = c;
-                out_flag[k] = f;
-                ++k;
+            if ((f & any) || (f & all) != all) {
+                const size_t k = (*d_count)++;
+                if (out_cell) out_cell[k] = c;
+                if (out_pair) {
+                    out_pair[2 * k] = (unsigned)c;
+                    out_pair[2 * k + 1] = f;
+                }
             }
         }
-        *d_count = k;
-        return k;
     }
     void piece_setup(int nq, const int* cells, const pt4* pts, const int* inst_of,
                      const double* box, double* p_box) {

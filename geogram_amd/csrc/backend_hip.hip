@@ -2,7 +2,7 @@
 //
 // Kernels:
 //   k_morton / rocPRIM radix sort / k_gather   Morton order of the seeds
-//   k_bvh_leaves, k_bvh_level                  implicit tree over buckets
+//   k_tree_base, k_tree_top                    implicit tree over buckets
 //   k_knn<K>                                   lane-per-query kNN, FP32 ranking
 //   k_clip<S>                                  wavefront-per-cell clipping and
 //                                              FP64 integration (clip_cell.h)
@@ -95,36 +95,80 @@ __global__ void k_gather(const double* __restrict__ xyz, const double* __restric
     if (inst_of) inst_of[s] = inst_orig ? inst_orig[i] : 0;
 }
 
-__global__ void k_bvh_leaves(const pt4* __restrict__ pts, InstLayout IL, bnode* nodes,
-                             const long long* __restrict__ leaf_off, int ni, long long total) {
-    long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= total) return;
-    int inst = find_inst(leaf_off, ni, t);
-    bvh_leaf(pts, IL, nodes, inst, (int)(t - leaf_off[inst]));
+// The tree in two launches: each work-group builds kTreeLeaves leaves and the
+// levels above them while they are in its cache, then one work-group per
+// instance the rest: 12 + 4 us for 40k seeds, where a launch per level (12,
+// most of them a few wavefronts) paid its start and a table copy each time.
+__global__ __launch_bounds__(kTreeLeaves) void k_tree_base(const pt4* __restrict__ pts,
+                                                           InstLayout IL, bnode* nodes,
+                                                           const long long* __restrict__ blk_off,
+                                                           int ni) {
+    const int inst = find_inst(blk_off, ni, blockIdx.x);
+    const int L = IL.L[inst], l0 = (int)(blockIdx.x - blk_off[inst]) * kTreeLeaves;
+    const int m = min(kTreeLeaves, L - l0);  // a power of two
+    const int t = threadIdx.x;
+    if (t < m) bvh_leaf(pts, IL, nodes, inst, l0 + t);
+    for (int h = 1; (m >> h) > 0; ++h) {
+        __syncthreads();
+        if (t < (m >> h)) bvh_merge(nodes, IL.t0[inst], ((L + l0) >> h) + t);
+    }
 }
 
-__global__ void k_bvh_level(InstLayout IL, bnode* nodes, const long long* __restrict__ lvl_off,
-                            int ni, long long total, int h) {
-    long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= total) return;
-    int inst = find_inst(lvl_off, ni, t);
-    int k = (IL.L[inst] >> h) + (int)(t - lvl_off[inst]);
-    bvh_merge(nodes, IL.t0[inst], k);
+__global__ __launch_bounds__(1024) void k_tree_top(InstLayout IL, bnode* nodes) {
+    const int inst = blockIdx.x;
+    for (int k0 = IL.L[inst] / kTreeLeaves / 2; k0 > 0; k0 >>= 1) {
+        for (int k = k0 + threadIdx.x; k < 2 * k0; k += blockDim.x) bvh_merge(nodes, IL.t0[inst], k);
+        __syncthreads();
+    }
 }
 
-__global__ void k_wmax(const pt4* __restrict__ pts, InstLayout IL, double* out) {
+// Largest weight of each instance, by gridDim.y work-groups each (part: their
+// maxima, reduced by a second launch; the single work-group of before read
+// 120k weights in 112 us).
+__global__ void k_wmax(const pt4* __restrict__ pts, InstLayout IL, const double* __restrict__ part,
+                       int nparts, double* out) {
     __shared__ double red[256];
-    int inst = blockIdx.x;
-    int p0 = IL.p0[inst], n = IL.n[inst];
+    const int inst = blockIdx.x;
+    const int p0 = IL.p0[inst], n = part ? nparts : IL.n[inst];
     double m = -INFINITY;
-    for (int s = p0 + threadIdx.x; s < p0 + n; s += blockDim.x) m = fmax(m, pts[s].w);
+    for (int s = blockIdx.y * blockDim.x + threadIdx.x; s < n; s += blockDim.x * gridDim.y)
+        m = fmax(m, part ? part[(size_t)inst * nparts + s] : pts[p0 + s].w);
     red[threadIdx.x] = m;
     __syncthreads();
     for (int off = blockDim.x / 2; off > 0; off >>= 1) {
         if ((int)threadIdx.x < off) red[threadIdx.x] = fmax(red[threadIdx.x], red[threadIdx.x + off]);
         __syncthreads();
     }
-    if (threadIdx.x == 0) out[inst] = red[0];
+    if (threadIdx.x == 0) out[(size_t)inst * gridDim.y + blockIdx.y] = red[0];
+}
+
+// Bounding box of n points: minima in out[6 b .. +2], maxima in +3 .. +5 of
+// work-group b; rows (if not null): the partial boxes of an earlier launch.
+__global__ __launch_bounds__(256) void k_extent(const double* __restrict__ xyz,
+                                                const double* __restrict__ rows, long long n,
+                                                double* out) {
+    __shared__ double red[6][256];
+    double v[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
+    for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += 256ll * gridDim.x)
+        for (int c = 0; c < 3; ++c) {
+            v[c] = fmin(v[c], rows ? rows[6 * i + c] : xyz[3 * i + c]);
+            v[3 + c] = fmax(v[3 + c], rows ? rows[6 * i + 3 + c] : xyz[3 * i + c]);
+        }
+    for (int c = 0; c < 6; ++c) red[c][threadIdx.x] = v[c];
+    __syncthreads();
+    for (int off = 128; off > 0; off >>= 1) {
+        if ((int)threadIdx.x < off)
+            for (int c = 0; c < 6; ++c) {
+                const double a = red[c][threadIdx.x], b = red[c][threadIdx.x + off];
+                red[c][threadIdx.x] = c < 3 ? fmin(a, b) : fmax(a, b);
+            }
+        __syncthreads();
+    }
+    if (threadIdx.x == 0)
+        for (int c = 0; c < 6; ++c)
+            // (a first point that is NaN stays, as in a sequential min)
+            out[6 * (size_t)blockIdx.x + c] =
+                gridDim.x == 1 && isnan(xyz[c % 3]) ? xyz[c % 3] : red[c][0];
 }
 
 template <int K>
@@ -1409,23 +1453,26 @@ __global__ void k_power_nearest(const pt4* __restrict__ pts, const bnode* __rest
     wout[t] = pts[j].w;
 }
 
-// Cells of `items` (all n_items cells if null) that are not plainly done —
-// not CELL_DONE, or carrying a flag of `mask` — appended with their flags
-// (unordered; the host sorts them).  Cells of the instances marked in
-// `skip` (by inst_of; instance 0 if null) are left out.
+// Cells of `items` (all n_items cells if null) whose flags have a bit of
+// `any` or lack one of `all`, appended (unordered) to out_cell, or with their
+// flags to out_pair.  Cells of the instances marked in `skip` (by inst_of;
+// instance 0 if null) are left out.
 __global__ void k_census(const int* __restrict__ items, int n_items,
-                         const uint32_t* __restrict__ flags, uint32_t mask,
+                         const uint32_t* __restrict__ flags, uint32_t any, uint32_t all,
                          const unsigned* __restrict__ skip, const int* __restrict__ inst_of,
-                         int* out_cell, uint32_t* out_flag, unsigned* count) {
+                         int* out_cell, unsigned* out_pair, unsigned* count) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= n_items) return;
     const int c = items ? items[t] : t;
     if (skip && skip[inst_of ? inst_of[c] : 0]) return;
     const uint32_t f = flags[c];
-    if ((f & mask) || !(f & CELL_DONE)) {
-        const unsigned k = atomicAdd(count, 1u);
-        out_cell[k] = c;
-        out_flag[k] = f;
+    if ((f & any) || (f & all) != all) {
+        const size_t k = atomicAdd(count, 1u);
+        if (out_cell) out_cell[k] = c;
+        if (out_pair) {
+            out_pair[2 * k] = (unsigned)c;
+            out_pair[2 * k + 1] = f;
+        }
     }
 }
 
@@ -1458,6 +1505,7 @@ struct HipBackend {
         if (seg_part_) (void)hipFree(seg_part_);
         if (wide_) (void)hipFree(wide_);
         if (wide_front_) (void)hipFree(wide_front_);
+        if (pin_) (void)hipHostFree(pin_);
         if (enter_ev_) (void)hipEventDestroy(enter_ev_);
         if (stream_) (void)hipStreamDestroy(stream_);
     }
@@ -1478,20 +1526,50 @@ struct HipBackend {
         return p;
     }
     void dfree(void* p) { (void)hipFree(p); }
+    // Small copies go through a pinned buffer of the context: to the device
+    // without a wait (their place is reused only after a wait for the stream),
+    // back with one wait.  Larger ones, and the caller's arrays, as they are.
     void h2d(void* d, const void* s, size_t b) {
+        if (char* p = pinned(b)) {
+            std::memcpy(p, s, b);
+            VGC_HIP_CHECK(hipMemcpyAsync(d, p, b, hipMemcpyHostToDevice, stream_));
+            return;
+        }
         VGC_HIP_CHECK(hipMemcpyAsync(d, s, b, hipMemcpyHostToDevice, stream_));
-        VGC_HIP_CHECK(hipStreamSynchronize(stream_));
+        sync();
     }
-    void d2h(void* d, const void* s, size_t b) {
-        VGC_HIP_CHECK(hipMemcpyAsync(d, s, b, hipMemcpyDeviceToHost, stream_));
-        VGC_HIP_CHECK(hipStreamSynchronize(stream_));
+    void d2h(void* d, const void* s, size_t b) { d2h2(d, s, b, nullptr, nullptr, 0); }
+    // two copies, one wait
+    void d2h2(void* d, const void* s, size_t b, void* d2, const void* s2, size_t b2) {
+        const size_t a = (b + 15) / 16 * 16;
+        char* p = pinned(a + b2);
+        VGC_HIP_CHECK(hipMemcpyAsync(p ? p : d, s, b, hipMemcpyDeviceToHost, stream_));
+        if (b2) VGC_HIP_CHECK(hipMemcpyAsync(p ? p + a : d2, s2, b2, hipMemcpyDeviceToHost, stream_));
+        sync();
+        if (p) {
+            std::memcpy(d, p, b);
+            if (b2) std::memcpy(d2, p + a, b2);
+        }
+    }
+    // b bytes of the pinned buffer, or null if that is too large for it
+    char* pinned(size_t b) {
+        if (b == 0 || b > kPinChunk) return nullptr;
+        if (!pin_) VGC_HIP_CHECK(hipHostMalloc((void**)&pin_, kPinBytes, hipHostMallocDefault));
+        if (pin_used_ + b > kPinBytes) sync();
+        char* p = pin_ + pin_used_;
+        pin_used_ += (b + 63) / 64 * 64;
+        return p;
     }
     void d2d(void* d, const void* s, size_t b) {
         VGC_HIP_CHECK(hipMemcpyAsync(d, s, b, hipMemcpyDeviceToDevice, stream_));
     }
     void dzero(void* d, size_t b) { VGC_HIP_CHECK(hipMemsetAsync(d, 0, b, stream_)); }
-    void sync() { VGC_HIP_CHECK(hipStreamSynchronize(stream_)); }
-    // HIP events on the launch stream around a phase (slot 0: kNN, 1: pass A)
+    void sync() {
+        VGC_HIP_CHECK(hipStreamSynchronize(stream_));
+        pin_used_ = 0;
+    }
+    // HIP events on the launch stream around a phase (slot 0: kNN, 1: pass A,
+    // 2: its FP64 redo)
     void event_begin(int k) {
         if (!ev_[k][0]) {
             VGC_HIP_CHECK(hipEventCreate(&ev_[k][0]));
@@ -1540,18 +1618,27 @@ struct HipBackend {
                                                           inst_of);
         check();
     }
-    void bvh_leaves(const pt4* pts, const InstLayout& IL, bnode* nodes, const long long* leaf_off,
-                    int ni, long long total) {
-        k_bvh_leaves<<<blocks_for(total, 256), 256, 0, stream_>>>(pts, IL, nodes, leaf_off, ni, total);
+    // blk_off: the instances' work-groups of kTreeLeaves leaves, nblk in all;
+    // max_h: levels of the deepest tree
+    void bvh_build(const pt4* pts, const InstLayout& IL, bnode* nodes, const long long* blk_off,
+                   int ni, long long nblk, int max_h) {
+        k_tree_base<<<(unsigned)nblk, kTreeLeaves, 0, stream_>>>(pts, IL, nodes, blk_off, ni);
+        if ((1ll << max_h) > kTreeLeaves) k_tree_top<<<ni, 1024, 0, stream_>>>(IL, nodes);
         check();
     }
-    void bvh_level(const InstLayout& IL, bnode* nodes, const long long* lvl_off, int ni,
-                   long long total, int h) {
-        k_bvh_level<<<blocks_for(total, 256), 256, 0, stream_>>>(IL, nodes, lvl_off, ni, total, h);
+    void wmax(const pt4* pts, const InstLayout& IL, int ni, int nmax, double* out) {
+        const unsigned parts = (unsigned)std::min(64, 1 + nmax / 4096);
+        double* part = parts > 1 ? (double*)temp(sizeof(double) * (size_t)ni * parts) : out;
+        k_wmax<<<dim3(ni, parts), 256, 0, stream_>>>(pts, IL, nullptr, 0, part);
+        if (parts > 1) k_wmax<<<ni, 256, 0, stream_>>>(pts, IL, part, parts, out);
         check();
     }
-    void wmax(const pt4* pts, const InstLayout& IL, int ni, double* out) {
-        k_wmax<<<ni, 256, 0, stream_>>>(pts, IL, out);
+    // out: minima, maxima
+    void extent(const double* xyz, long long n, double* out) {
+        const unsigned g = (unsigned)std::min(256ll, 1 + n / 2048);
+        double* part = g > 1 ? (double*)temp(sizeof(double) * 6 * g) : out;
+        k_extent<<<g, 256, 0, stream_>>>(xyz, nullptr, n, part);
+        if (g > 1) k_extent<<<1, 256, 0, stream_>>>(xyz, part, g, out);
         check();
     }
     void knn(int K, const pf4* pf, const bnode* nodes, const InstLayout& IL, const int* queries,
@@ -1580,6 +1667,15 @@ struct HipBackend {
                    : launch_clip_exact_list(S, P, waves_, stream_);
         else
             gather ? launch_clip_gather(S, P, waves_, stream_) : launch_clip_list(S, P, waves_, stream_);
+        check();
+    }
+    // the FP64 first pass of the d_count cells listed in items (at most
+    // P.n_items; the count stays on the device)
+    void clip_listed(const ClipParams& P, const int* items, const unsigned* d_count) {
+        if (P.n_items <= 0) return;
+        ClipParams Q = P;
+        Q.items = items;
+        launch_clip_listed(Q, d_count, stream_);
         check();
     }
     void radius_r2(const int* items, int ni, const pt4* pts, const double* r2, const int* inst_of,
@@ -1657,18 +1753,14 @@ struct HipBackend {
         k_rebase<<<blocks_for(n, 256), 256, 0, stream_>>>(off, n, base, out);
         check();
     }
-    // k_census into out_cell / out_flag (n_items capacity); returns the count
-    unsigned census(const int* items, int n_items, const uint32_t* flags, uint32_t mask,
-                    const unsigned* skip, const int* inst_of, int* out_cell, uint32_t* out_flag,
-                    unsigned* d_count) {
-        VGC_HIP_CHECK(hipMemsetAsync(d_count, 0, sizeof(unsigned), stream_));
+    // k_census; d_count: cleared by the caller
+    void census(const int* items, int n_items, const uint32_t* flags, uint32_t any, uint32_t all,
+                const unsigned* skip, const int* inst_of, int* out_cell, unsigned* out_pair,
+                unsigned* d_count) {
         if (n_items > 0)
             k_census<<<blocks_for(n_items, 256), 256, 0, stream_>>>(
-                items, n_items, flags, mask, skip, inst_of, out_cell, out_flag, d_count);
+                items, n_items, flags, any, all, skip, inst_of, out_cell, out_pair, d_count);
         check();
-        unsigned cnt = 0;
-        d2h(&cnt, d_count, sizeof(unsigned));
-        return cnt;
     }
     void power_nearest(const pt4* pts, const bnode* nodes, const InstLayout& IL, const double* q,
                        int nq, float cs2, double* wout) {
@@ -2152,7 +2244,10 @@ private:
     hipStream_t stream_ = nullptr;
     hipStream_t caller_ = nullptr;
     hipEvent_t enter_ev_ = nullptr;
-    hipEvent_t ev_[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};
+    hipEvent_t ev_[3][2] = {};
+    static constexpr size_t kPinBytes = 256 << 10, kPinChunk = 32 << 10;
+    char* pin_ = nullptr;   // pinned buffer of the small copies
+    size_t pin_used_ = 0;
     void* temp_ = nullptr;
     size_t temp_bytes_ = 0;
     double* red_ = nullptr;

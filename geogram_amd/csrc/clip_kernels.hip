@@ -1,6 +1,6 @@
 // The clipping kernels, compiled once per VGC_CLIP_PART (0: gathered
 // neighbours, 1: lists, 2 and 3: the same with exact signs, 4: the FP32 first
-// pass), so that the parts build in parallel.
+// pass, 5: the cells that leaves), so that the parts build in parallel.
 #include <stdexcept>
 
 #include "clip_launch.h"
@@ -76,6 +76,24 @@ void launch_clip_exact_list(int S, const ClipParams& P, int waves, hipStream_t s
     clip_eg<true, false>(S, P, waves, stream);
 }
 #endif
+#elif VGC_CLIP_PART == 5
+// The cells that the FP32 first pass left (0.3 % of the 2M mixture), their
+// list and its length read on the device: up to 4096 wavefronts, the number
+// the chip holds, share them.
+template <bool W>
+__global__ __launch_bounds__(64, 4) void k_clip_listed(ClipParams P, const unsigned* count) {
+    __shared__ CellLds<1> lds;
+    const int n = (int)*count;
+    for (int item = blockIdx.x; item < n; item += gridDim.x)
+        process_cell<1, false, true, W, W>(P, item, lds);
+}
+void launch_clip_listed(const ClipParams& P, const unsigned* count, hipStream_t stream) {
+    const unsigned g = (unsigned)(P.n_items < 4096 ? P.n_items : 4096);
+    if (P.weighted)
+        k_clip_listed<true><<<g, 64, 0, stream>>>(P, count);
+    else
+        k_clip_listed<false><<<g, 64, 0, stream>>>(P, count);
+}
 #else
 // The first pass with FP32 corner state: two cells per wavefront
 // (pair_cell.h).

@@ -25,6 +25,9 @@ void launch_clip_gather(int S, const ClipParams& P, int waves, hipStream_t strea
 void launch_clip_list(int S, const ClipParams& P, int waves, hipStream_t stream);
 void launch_clip_exact_gather(int S, const ClipParams& P, int waves, hipStream_t stream);
 void launch_clip_exact_list(int S, const ClipParams& P, int waves, hipStream_t stream);
+// the first pass with FP64 corners of the *count cells in P.items (at most
+// P.n_items), by wavefronts that take one after the other
+void launch_clip_listed(const ClipParams& P, const unsigned* count, hipStream_t stream);
 // the FP32 first pass (pair_cell.h)
 void launch_pairs(const ClipParams& P, int waves, hipStream_t stream);
 

@@ -554,6 +554,7 @@ VGC_SD int radius_query(const pf4* pf, const bnode* nodes, const InstLayout& IL,
 }
 
 // ---------------------------------------------------------- tree build
+constexpr int kTreeLeaves = 256;  // leaves per work-group of the build
 VGC_SD void bvh_leaf(const pt4* pts, const InstLayout& IL, bnode* nodes, int inst, int leaf) {
     const int p0 = IL.p0[inst], n = IL.n[inst], nb = IL.nb[inst], L = IL.L[inst];
     bnode B;

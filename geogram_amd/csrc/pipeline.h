@@ -71,6 +71,15 @@ struct Problem {
     bool want_neighbors = true;
     bool want_e2 = false;           // integral of |x - p|^2 per cell (CVT energy)
     bool count_work = false;        // algorithmic work counters (global atomics)
+    // device memory for the outputs, if the caller's arrays can take them
+    // directly (not periodic, no subset of instances; the CSR entries only if
+    // they fit out_cap)
+    double* out_vol = nullptr;
+    double* out_mg = nullptr;
+    long long* out_ptr = nullptr;
+    int* out_nbr = nullptr;
+    double* out_area = nullptr;
+    long long out_cap = 0;
     bool abort_on_empty = false;    // an instance with an empty cell stops (and is bad)
                                     // (cells() then returns 1; outputs unset)
     // per instance, nonzero = compute its cells; the others keep the outputs
@@ -161,7 +170,6 @@ public:
         h_nb_.assign(ni_, 0);
         h_L_.assign(ni_, 1);
         h_t0_.assign(ni_, 0);
-        h_leaf_off_.assign(ni_ + 1, 0);
         long long pp = 0, bb = 0, tt = 0;
         max_h_ = 0;
         for (int i = 0; i < ni_; ++i) {
@@ -180,30 +188,41 @@ public:
             max_h_ = std::max(max_h_, h);
             h_t0_[i] = tt;
             tt += 2LL * L;
-            h_leaf_off_[i + 1] = h_leaf_off_[i] + L;
         }
         if (pp != n_) {
             error = "instance sizes do not add up to n";
             return -1;
         }
         n_nodes_ = tt;
-        int* d_p0 = (int*)slot(S_P0, sizeof(int) * ni_);
-        int* d_n = (int*)slot(S_N, sizeof(int) * ni_);
-        int* d_b0 = (int*)slot(S_B0, sizeof(int) * ni_);
-        int* d_nb = (int*)slot(S_NB, sizeof(int) * ni_);
-        int* d_L = (int*)slot(S_L, sizeof(int) * ni_);
-        long long* d_t0 = (long long*)slot(S_T0, sizeof(long long) * ni_);
-        long long* d_leaf_off = (long long*)slot(S_LEAFOFF, sizeof(long long) * (ni_ + 1));
-        double* d_box = (double*)slot(S_BOX, sizeof(double) * 6 * ni_);
-        be_.h2d(d_p0, h_p0_.data(), sizeof(int) * ni_);
-        be_.h2d(d_n, h_n_.data(), sizeof(int) * ni_);
-        be_.h2d(d_b0, h_b0_.data(), sizeof(int) * ni_);
-        be_.h2d(d_nb, h_nb_.data(), sizeof(int) * ni_);
-        be_.h2d(d_L, h_L_.data(), sizeof(int) * ni_);
+        // every small table in one copy
+        std::vector<long long> blk_off(ni_ + 1, 0);  // work-groups of the tree build
+        for (int i = 0; i < ni_; ++i)
+            blk_off[i + 1] = blk_off[i] + std::max(1, h_L_[i] / kTreeLeaves);
+        std::vector<char> tab;
+        auto put = [&](const void* src, size_t bytes) {
+            const size_t at = tab.size();
+            tab.resize(at + (bytes + 15) / 16 * 16);
+            std::memcpy(tab.data() + at, src, bytes);
+            return at;
+        };
+        const size_t o_box = put(pb.box.data(), sizeof(double) * 6 * ni_);
+        const size_t o_t0 = put(h_t0_.data(), sizeof(long long) * ni_);
+        const size_t o_blk = put(blk_off.data(), sizeof(long long) * (ni_ + 1));
+        const size_t o_p0 = put(h_p0_.data(), sizeof(int) * ni_);
+        const size_t o_n = put(h_n_.data(), sizeof(int) * ni_);
+        const size_t o_b0 = put(h_b0_.data(), sizeof(int) * ni_);
+        const size_t o_nb = put(h_nb_.data(), sizeof(int) * ni_);
+        const size_t o_L = put(h_L_.data(), sizeof(int) * ni_);
+        char* d_tab = (char*)slot(S_TAB, tab.size());
+        be_.h2d(d_tab, tab.data(), tab.size());
+        int* d_p0 = (int*)(d_tab + o_p0);
+        int* d_n = (int*)(d_tab + o_n);
+        int* d_b0 = (int*)(d_tab + o_b0);
+        int* d_nb = (int*)(d_tab + o_nb);
+        int* d_L = (int*)(d_tab + o_L);
+        long long* d_t0 = (long long*)(d_tab + o_t0);
+        const double* d_box = (const double*)(d_tab + o_box);
         be_.set_tree_leaves(*std::max_element(h_L_.begin(), h_L_.begin() + ni_));
-        be_.h2d(d_t0, h_t0_.data(), sizeof(long long) * ni_);
-        be_.h2d(d_leaf_off, h_leaf_off_.data(), sizeof(long long) * (ni_ + 1));
-        be_.h2d(d_box, pb.box.data(), sizeof(double) * 6 * ni_);
         d_box_ = d_box;
 
         // Morton sort
@@ -234,21 +253,12 @@ public:
         IL.t0 = d_t0;
         IL.L = d_L;
         d_nodes = (bnode*)slot(S_NODES, sizeof(bnode) * (size_t)n_nodes_);
-        be_.bvh_leaves(d_pts, IL, d_nodes, d_leaf_off, ni_, h_leaf_off_[ni_]);
-        std::vector<long long> off(ni_ + 1);
-        long long* d_lvl = (long long*)slot(S_LVLOFF, sizeof(long long) * (ni_ + 1));
-        for (int h = 1; h <= max_h_; ++h) {
-            off[0] = 0;
-            for (int i = 0; i < ni_; ++i) off[i + 1] = off[i] + (h_L_[i] >> h);
-            if (off[ni_] == 0) break;
-            be_.h2d(d_lvl, off.data(), sizeof(long long) * (ni_ + 1));
-            be_.bvh_level(IL, d_nodes, d_lvl, ni_, off[ni_], h);
-        }
+        be_.bvh_build(d_pts, IL, d_nodes, (const long long*)(d_tab + o_blk), ni_, blk_off[ni_], max_h_);
         // weights: max per instance (security radius of Laguerre cells)
         weighted_ = pb.d_w != nullptr;
         d_wmax_ = (double*)slot(S_WMAX, sizeof(double) * ni_);
-        if (weighted_) be_.wmax(d_pts, IL, ni_, d_wmax_);
-        be_.sync();
+        if (weighted_) be_.wmax(d_pts, IL, ni_, *std::max_element(h_n_.begin(), h_n_.begin() + ni_), d_wmax_);
+        // (launched, not awaited: the phase times are host times)
         st.t_build_ms += ms_since(t0);
         return 0;
     }
@@ -524,16 +534,18 @@ public:
             st.t_knn_gpu_ms += be_.event_ms(0);
         }
 
-        d_vol = (double*)slot(S_VOL, sizeof(double) * (size_t)n_);
-        d_mg = (double*)slot(S_MG, sizeof(double) * 3 * (size_t)n_);
+        d_vol = pb.out_vol ? pb.out_vol : (double*)slot(S_VOL, sizeof(double) * (size_t)n_);
+        d_mg = pb.out_mg ? pb.out_mg : (double*)slot(S_MG, sizeof(double) * 3 * (size_t)n_);
         int* d_cnt = (int*)slot(S_CNT, sizeof(int) * (size_t)n_);
         int* d_nbr_tmp = (int*)slot(S_NBRTMP, sizeof(int) * (size_t)n_ * kFaceStride);
         double* d_area_tmp = (double*)slot(S_AREATMP, sizeof(double) * (size_t)n_ * kFaceStride);
         uint32_t* d_flags = (uint32_t*)slot(S_FLAGS, sizeof(uint32_t) * (size_t)n_);
         double* d_r2 = (double*)slot(S_R2, sizeof(double) * (size_t)n_);
         unsigned long long* d_ctr = (unsigned long long*)slot(S_CTR, sizeof(unsigned long long) * 8);
-        be_.dzero(d_ctr, sizeof(unsigned long long) * 8);
-        be_.dzero(d_flags, sizeof(uint32_t) * (size_t)n_);
+        if (pb.count_work) be_.dzero(d_ctr, sizeof(unsigned long long) * 8);
+        // (every computed cell writes its flag, except those of an instance
+        // that stopped)
+        if (pb.abort_on_empty) be_.dzero(d_flags, sizeof(uint32_t) * (size_t)n_);
         // a subset of instances: the others keep their neighbour counts
         std::vector<int> aitems;
         if (pb.active) {
@@ -664,10 +676,8 @@ public:
         be_.event_begin(1);
         if (P.n_items > 0) be_.clip(1, false, gather, P);
         be_.event_end(1);
-        be_.sync();
-        st.t_clip_ms += ms_since(t2);
-        st.t_clip_a_gpu_ms += be_.event_ms(1);
-        {
+        st.a_cells += P.n_items;
+        if (pb.count_work) {
             unsigned long long c[8];
             be_.d2h(c, d_ctr, sizeof(c));
             st.a_tests += c[1];
@@ -675,42 +685,24 @@ public:
             st.a_new += c[3];
             st.a_tets += c[4];
             st.a_facets += c[5];
-            st.a_cells += P.n_items;
         }
-        if (P.fp32) {
+        // census buffers: {cells listed, cells redone}, then (cell, flag)
+        const size_t ncen = std::max(1, P.n_items);
+        unsigned* d_cen = (unsigned*)slot(S_CENS_N, sizeof(unsigned) * (2 + 2 * ncen));
+        be_.dzero(d_cen, sizeof(unsigned) * 2);
+        const bool redo = P.fp32 && P.n_items > 0;
+        if (redo) {
             // cells with a sign or corner the FP32 corners could not certify
             // (flagged uncertain and left without outputs): the FP64 first
-            // pass, which writes every output of them
+            // pass, which writes every output of them.  Their list and its
+            // length stay on the device.
             P.fp32 = 0;
-            const size_t cap = std::max(1, P.n_items);
-            int* d_cc = (int*)slot(S_CENS_C, sizeof(int) * cap);
-            uint32_t* d_cf = (uint32_t*)slot(S_CENS_F, sizeof(uint32_t) * cap);
-            unsigned* d_cn = (unsigned*)slot(S_CENS_N, sizeof(unsigned));
-            const unsigned m = be_.census(P.items, P.n_items, d_flags, CELL_UNCERTAIN, P.abort_flag,
-                                          P.inst_of, d_cc, d_cf, d_cn);
-            std::vector<int> cc(m), redo;
-            std::vector<uint32_t> cf(m);
-            if (m) {
-                be_.d2h(cc.data(), d_cc, sizeof(int) * m);
-                be_.d2h(cf.data(), d_cf, sizeof(uint32_t) * m);
-            }
-            for (unsigned i = 0; i < m; ++i)
-                if (cf[i] & CELL_UNCERTAIN) redo.push_back(cc[i]);
-            std::sort(redo.begin(), redo.end());
-            st.nb_fp64_redo += redo.size();
-            if (redo.size() * 2 > (size_t)P.n_items) fp32_skip_ = kFp32Skip;
-            if (!redo.empty()) {
-                int* d_items = (int*)slot(S_ITEMS, sizeof(int) * redo.size());
-                be_.h2d(d_items, redo.data(), sizeof(int) * redo.size());
-                ClipParams Q = P;
-                Q.items = d_items;
-                Q.n_items = (int)redo.size();
-                be_.event_begin(1);
-                be_.clip(1, false, gather, Q);
-                be_.event_end(1);
-                be_.sync();
-                st.t_redo_gpu_ms += be_.event_ms(1);
-            }
+            int* d_cc = (int*)slot(S_CENS_C, sizeof(int) * ncen);
+            be_.census(P.items, P.n_items, d_flags, CELL_UNCERTAIN, 0, P.abort_flag, P.inst_of, d_cc,
+                       nullptr, d_cen + 1);
+            be_.event_begin(2);
+            be_.clip_listed(P, d_cc, d_cen + 1);
+            be_.event_end(2);
         }
         auto t3 = now();
         // instances stopped by an empty cell: bad; no further pass for them
@@ -718,6 +710,7 @@ public:
         if (P.abort_flag) {
             stopped.resize(ni_);
             be_.d2h(stopped.data(), P.abort_flag, sizeof(unsigned) * (size_t)ni_);
+            // (a pass that stops here has no other wait)
             int nstop = 0, nlive = 0;
             for (int k = 0; k < ni_; ++k) {
                 nstop += stopped[k] != 0;
@@ -727,37 +720,47 @@ public:
             if (nstop == nlive) {
                 inst_bad.assign(ni_, 0);
                 for (int k = 0; k < ni_; ++k) inst_bad[k] = stopped[k] ? 1 : 0;
+                st.t_clip_ms += ms_since(t2);
+                st.t_clip_a_gpu_ms += be_.event_ms(1);
                 st.t_total_ms += ms_since(tstart);
                 return 1;
             }
         }
         // the cells that are not plainly done, with their flags, sorted by
         // Morton position: the later passes only touch these, and h_flags is
-        // kept current for them alone
-        h_flags.resize(n_);
+        // kept current for them alone.  The neighbour offsets are scanned
+        // along with them (again below if a later pass changes a count).
+        if ((int)h_flags.size() < n_) h_flags.resize(n_);
         census_.clear();
+        d_ptr = pb.out_ptr ? pb.out_ptr : (long long*)slot(S_PTR, sizeof(long long) * ((size_t)n_ + 1));
         {
-            const size_t cap = std::max(1, P.n_items);
-            int* d_cc = (int*)slot(S_CENS_C, sizeof(int) * cap);
-            uint32_t* d_cf = (uint32_t*)slot(S_CENS_F, sizeof(uint32_t) * cap);
-            unsigned* d_cn = (unsigned*)slot(S_CENS_N, sizeof(unsigned));
-            const unsigned m = be_.census(P.items, P.n_items, d_flags, kCensusMask, P.abort_flag,
-                                          P.inst_of, d_cc, d_cf, d_cn);
-            std::vector<int> cc(m);
-            std::vector<uint32_t> cf(m);
-            if (m) {
-                be_.d2h(cc.data(), d_cc, sizeof(int) * m);
-                be_.d2h(cf.data(), d_cf, sizeof(uint32_t) * m);
+            be_.census(P.items, P.n_items, d_flags, kCensusMask, CELL_DONE, P.abort_flag, P.inst_of,
+                       nullptr, d_cen + 2, d_cen);
+            be_.scan_i32(d_cnt, d_ptr, n_);
+            std::vector<unsigned> head(2 + 2 * std::min<size_t>(ncen, kCensusHead));
+            be_.d2h2(head.data(), d_cen, sizeof(unsigned) * head.size(), &total_neighbors, d_ptr + n_,
+                     sizeof(long long));
+            const size_t m = head[0];
+            if (head.size() < 2 + 2 * m) {
+                head.resize(2 + 2 * m);
+                be_.d2h(head.data(), d_cen, sizeof(unsigned) * head.size());
             }
-            std::vector<unsigned> ord(m);
-            for (unsigned i = 0; i < m; ++i) ord[i] = i;
-            std::sort(ord.begin(), ord.end(), [&](unsigned a, unsigned b) { return cc[a] < cc[b]; });
+            if (redo) {
+                st.nb_fp64_redo += head[1];
+                if ((size_t)head[1] * 2 > (size_t)P.n_items) fp32_skip_ = kFp32Skip;
+                st.t_redo_gpu_ms += be_.event_ms(2);
+            }
+            std::vector<std::pair<int, uint32_t>> ord(m);
+            for (size_t i = 0; i < m; ++i) ord[i] = {(int)head[2 + 2 * i], head[3 + 2 * i]};
+            std::sort(ord.begin(), ord.end());
             census_.resize(m);
-            for (unsigned i = 0; i < m; ++i) {
-                census_[i] = cc[ord[i]];
-                h_flags[cc[ord[i]]] = cf[ord[i]];
+            for (size_t i = 0; i < m; ++i) {
+                census_[i] = ord[i].first;
+                h_flags[ord[i].first] = ord[i].second;
             }
         }
+        st.t_clip_ms += ms_since(t2);
+        st.t_clip_a_gpu_ms += be_.event_ms(1);
         std::vector<int> need, over;
         long long nempty = 0;
         for (int c : census_) {
@@ -780,6 +783,7 @@ public:
             return 1;
         }
         P.abort_flag = nullptr;
+        bool later = !need.empty() || !over.empty();  // passes beyond the first two
         if (gather) {
             // cells that used up the first pass's ring limit: gather again
             // without the limit (a wave per cell) before any list tier
@@ -811,6 +815,7 @@ public:
         for (int c : census_)
             if (h_flags[c] & (CELL_UNCERTAIN | CELL_BAD_TOPO)) unsure.push_back(c);
         st.nb_pass_e += unsure.size();
+        later = later || !unsure.empty();
         if (!unsure.empty()) {
             int ni = (int)unsure.size();
             int* d_items = (int*)slot(S_ITEMS, sizeof(int) * ni);
@@ -833,10 +838,12 @@ public:
         st.t_pass_bc_ms += ms_since(t3);
 
         // statistics
-        unsigned long long ctr[8];
-        be_.d2h(ctr, d_ctr, sizeof(ctr));
-        st.nb_clips += ctr[0];
-        st.nb_tests += ctr[1];
+        if (pb.count_work) {
+            unsigned long long ctr[8];
+            be_.d2h(ctr, d_ctr, sizeof(ctr));
+            st.nb_clips += ctr[0];
+            st.nb_tests += ctr[1];
+        }
         st.nb_cells += P.n_items;
         // the other computed cells are done with no flag
         inst_bad.assign(ni_, 0);
@@ -858,20 +865,23 @@ public:
 
         // CSR
         auto t4 = now();
-        d_ptr = (long long*)slot(S_PTR, sizeof(long long) * ((size_t)n_ + 1));
-        be_.scan_i32(d_cnt, d_ptr, n_);
-        be_.d2h(&total_neighbors, d_ptr + n_, sizeof(long long));
+        if (later) {
+            be_.scan_i32(d_cnt, d_ptr, n_);
+            be_.d2h(&total_neighbors, d_ptr + n_, sizeof(long long));
+        }
         st.nb_neighbors += total_neighbors;
         if (pb.want_neighbors) {
-            d_nbr = (int*)slot(S_NBR, sizeof(int) * std::max<long long>(1, total_neighbors));
-            d_area = (double*)slot(S_AREA, sizeof(double) * std::max<long long>(1, total_neighbors));
+            const bool direct = pb.out_nbr && pb.out_area && total_neighbors <= pb.out_cap;
+            d_nbr = direct ? pb.out_nbr
+                           : (int*)slot(S_NBR, sizeof(int) * std::max<long long>(1, total_neighbors));
+            d_area = direct ? pb.out_area
+                            : (double*)slot(S_AREA, sizeof(double) * std::max<long long>(1, total_neighbors));
             be_.compact(n_, d_cnt, d_ptr, d_nbr_tmp, d_area_tmp, kFaceStride, d_nbr, d_area);
             if (!piece_cells_.empty())
                 be_.piece_copy((int)piece_cells_.size(), (const int*)slots_[S_XCELLS].p, d_orig,
                                (const long long*)slots_[S_XOFF].p, (const int*)slots_[S_XNBR].p,
                                (const double*)slots_[S_XAREA].p, d_cnt, d_ptr, d_nbr, d_area);
         }
-        be_.sync();
         st.t_compact_ms += ms_since(t4);
         st.t_total_ms += ms_since(tstart);
         return 0;
@@ -939,8 +949,8 @@ public:
 
 private:
     enum Slot {
-        S_P0, S_N, S_B0, S_NB, S_L, S_T0, S_LEAFOFF, S_BOX, S_INSTORIG, S_KEYS, S_KEYS2,
-        S_VALS, S_VALS2, S_PTS, S_PF, S_ORIG, S_INSTOF, S_NODES, S_LVLOFF, S_WMAX, S_LIST,
+        S_TAB, S_INSTORIG, S_KEYS, S_KEYS2,
+        S_VALS, S_VALS2, S_PTS, S_PF, S_ORIG, S_INSTOF, S_NODES, S_WMAX, S_LIST,
         S_VOL, S_MG, S_CNT, S_NBRTMP, S_AREATMP, S_FLAGS, S_R2, S_CTR, S_PTR, S_NBR, S_AREA,
         S_ITEMS, S_RHO2, S_RCNT, S_ROFF, S_RLIST, S_RD2, S_RLIST2, S_RD22, S_RLEN, S_BALL,
         S_FILT, S_COFF, S_AITEMS, S_TITEMS, S_CENS_C, S_CENS_F, S_CENS_N, S_ABORT, S_E2,
@@ -1274,19 +1284,20 @@ private:
     long long n_nodes_ = 0;
     bool weighted_ = false;
     int tuned_n_ = -1;
-    double* d_box_ = nullptr;
+    const double* d_box_ = nullptr;
     double* d_wmax_ = nullptr;
     double* d_r2_ = nullptr;  // squared radius per cell of the last pass (Morton order)
     std::vector<int> h_p0_, h_n_, h_b0_, h_nb_, h_L_;
     // first passes left to run with FP64 corners (after an FP32 pass that
     // redid more than half of its cells)
     static constexpr int kFp32Skip = 8;
+    static constexpr size_t kCensusHead = 500;  // census entries read with the count
     int fp32_skip_ = 0;
     std::vector<int> piece_cells_;  // cells of this pass computed in pieces
     long long x_total_ = 0;         // their merged neighbour entries
     static constexpr int kPieceLevels = 4;
     static constexpr long long kMaxPieces = 1 << 16;
-    std::vector<long long> h_t0_, h_leaf_off_;
+    std::vector<long long> h_t0_;
 };
 
 }  // namespace vgc
