@@ -742,6 +742,19 @@ VGC_HD LF lane_dist2(const pf4* pf, const LI& idx, const LB& m, float px, float 
 #endif
 }
 
+// Start of a tree walk: the nodes of the 64-node level (the root of a smaller
+// tree) into front; returns their number.  A wavefront tests 64 nodes in the
+// time of one, so the levels above only added dependent steps (three of eight
+// in a tree of 16k buckets).
+template <class LDS>
+VGC_HD int walk_start(LDS& L, int Lv) {
+    const LI lane = lane_id();
+    const int k = Lv >= kWave ? kWave : 1;
+    lds_st(&L.front[0][0], select(lane < k, lane, LI(0)), k + lane, lane < k);
+    wave_sync();
+    return k;
+}
+
 // Seeds q != c of the instance with rlo2 < d2 <= rhi2 (FP32 squared
 // distance) into L.cand as (d2 bits << 32 | q), unsorted.  Returns their
 // number (only the first kCandCap are stored), or -1 when the tree walk
@@ -754,9 +767,7 @@ VGC_HD int gather_ring(const ClipParams& P, LDS& L, int c, int inst, float px, f
     const LI lane = lane_id();
     const int p0 = P.IL.p0[inst], n = P.IL.n[inst], nb = P.IL.nb[inst], Lv = P.IL.L[inst];
     const bnode* T = P.nodes + P.IL.t0[inst];
-    lds_st(&L.front[0][0], LI(0), LI(1), lane == 0);
-    wave_sync();
-    int nf = 1, cur = 0, nbk = 0;
+    int nf = walk_start(L, Lv), cur = 0, nbk = 0;
     bool overflow = false;
     while (nf > 0) {
         int nn = 0;
@@ -966,9 +977,7 @@ VGC_HD int gather_dfs(const ClipParams& P, LDS& L, int c, int inst, float px, fl
     const int p0 = P.IL.p0[inst], n = P.IL.n[inst], nb = P.IL.nb[inst], Lv = P.IL.L[inst];
     const bnode* T = P.nodes + P.IL.t0[inst];
     int* stk = &L.front[0][0];
-    lds_st(stk, LI(0), LI(1), lane == 0);
-    wave_sync();
-    int top = 1, cnt = 0;
+    int top = walk_start(L, Lv), cnt = 0;
     float lim = rhi2;
     while (top > 0) {
         const int k = top < kWave ? top : kWave;

@@ -561,9 +561,7 @@ VGC_HD int near_buckets(const ClipParams& P, LDS& L, int inst, const SeedLanes& 
     const float hz = wave_maxf(select(has, p.z, LF(-INFINITY))), lz = -wave_maxf(select(has, -p.z, LF(-INFINITY)));
     const int nb = P.IL.nb[inst], Lv = P.IL.L[inst];
     const bnode* T = P.nodes + P.IL.t0[inst];
-    lds_st(&L.front[0][0], LI(0), LI(1), lane == 0);
-    wave_sync();
-    int nf = 1, cur = 0, nbk = 0;
+    int nf = walk_start(L, Lv), cur = 0, nbk = 0;
     while (nf > 0) {
         int nn = 0;
         for (int base = 0; base < nf; base += kWave) {
