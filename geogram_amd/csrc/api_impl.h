@@ -152,12 +152,12 @@ int api_cells(Ctx<B>* ctx, const double* xyz, const double* w, const uint32_t* i
             }
         }
         if (dev && !pb.periodic) {
-            // straight into the caller's arrays
-            pb.out_vol = vol;
-            pb.out_mg = mg;
-            pb.out_ptr = (long long*)nbr_ptr;
-            pb.out_nbr = nbr;
-            pb.out_area = farea;
+            // straight into the caller's arrays, where they are on this device
+            if (be.on_device(vol)) pb.out_vol = vol;
+            if (be.on_device(mg)) pb.out_mg = mg;
+            if (be.on_device(nbr_ptr)) pb.out_ptr = (long long*)nbr_ptr;
+            if (be.on_device(nbr)) pb.out_nbr = nbr;
+            if (be.on_device(farea)) pb.out_area = farea;
             pb.out_cap = (long long)std::min<uint64_t>(cap, 1ull << 62);
         }
         EngineStats es;
@@ -167,6 +167,7 @@ int api_cells(Ctx<B>* ctx, const double* xyz, const double* w, const uint32_t* i
         ctx->eng.begin_call();
         if (ctx->eng.cells(pb, es)) {
             ctx->err = "vgc_cells: " + ctx->eng.error;
+            be.sync();  // nothing writes to the caller's arrays after the return
             return VGC_ERR_INTERNAL;
         }
         Engine<B>& E = ctx->eng;
@@ -199,6 +200,10 @@ int api_cells(Ctx<B>* ctx, const double* xyz, const double* w, const uint32_t* i
         return VGC_OK;
     } catch (const std::exception& e) {
         ctx->err = e.what();
+        try {
+            ctx->be.sync();
+        } catch (const std::exception&) {
+        }
         return VGC_ERR_DEVICE;
     }
 }

@@ -28,6 +28,7 @@ struct EmuBackend {
         return p;
     }
     void dfree(void* p) { std::free(p); }
+    bool on_device(const void* p) { return p != nullptr; }
     void h2d(void* d, const void* s, size_t b) { std::memcpy(d, s, b); }
     void d2h(void* d, const void* s, size_t b) { std::memcpy(d, s, b); }
     void d2h2(void* d, const void* s, size_t b, void* d2, const void* s2, size_t b2) {

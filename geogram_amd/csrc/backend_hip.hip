@@ -123,8 +123,8 @@ __global__ __launch_bounds__(1024) void k_tree_top(InstLayout IL, bnode* nodes) 
 }
 
 // Largest weight of each instance, by gridDim.y work-groups each (part: their
-// maxima, reduced by a second launch; the single work-group of before read
-// 120k weights in 112 us).
+// maxima, reduced by a second launch): 10 us for 300k weights; a single
+// work-group read 120k in 112 us.
 __global__ void k_wmax(const pt4* __restrict__ pts, InstLayout IL, const double* __restrict__ part,
                        int nparts, double* out) {
     __shared__ double red[256];
@@ -534,14 +534,21 @@ __global__ void k_knn_select(const int* __restrict__ items, int ni,
 // reduces by halving strides, and one block reduces the partials the same way.
 constexpr int kRedBlocks = 512;
 
+// Sum of 256 values by a halving tree (+128, +64, ..., +1); every wavefront
+// adds them itself, so the work-group waits twice, not at each of the eight
+// levels.
+__device__ __forceinline__ double tree_sum(const double* sh) {
+    const int l = threadIdx.x & 63;
+    double s = (sh[l] + sh[l + 128]) + (sh[l + 64] + sh[l + 192]);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off);
+    return __shfl(s, 0);
+}
 __device__ __forceinline__ double block_sum(double v, double* sh) {
+    __syncthreads();  // an earlier sum's readers are done
     sh[threadIdx.x] = v;
     __syncthreads();
-    for (int off = 128; off > 0; off >>= 1) {
-        if ((int)threadIdx.x < off) sh[threadIdx.x] += sh[threadIdx.x + off];
-        __syncthreads();
-    }
-    return sh[0];
+    return tree_sum(sh);
 }
 
 __global__ __launch_bounds__(256) void k_dot_partial(int n, const double* __restrict__ a,
@@ -823,18 +830,12 @@ __global__ void k_ot_features(int n, const double* __restrict__ xyz, const doubl
 // kernel is a no-op afterwards, so extra launched iterations change nothing.
 __device__ __forceinline__ void block_sum2(double a, double b, double* sh, double* sh2, double& ta,
                                            double& tb) {
+    __syncthreads();  // an earlier sum's readers are done
     sh[threadIdx.x] = a;
     sh2[threadIdx.x] = b;
     __syncthreads();
-    for (int off = 128; off > 0; off >>= 1) {
-        if ((int)threadIdx.x < off) {
-            sh[threadIdx.x] += sh[threadIdx.x + off];
-            sh2[threadIdx.x] += sh2[threadIdx.x + off];
-        }
-        __syncthreads();
-    }
-    ta = sh[0];
-    tb = sh2[0];
+    ta = tree_sum(sh);
+    tb = tree_sum(sh2);
 }
 
 __global__ __launch_bounds__(256) void k_cg_start_partial(int n, const double* __restrict__ b,
@@ -1520,6 +1521,16 @@ struct HipBackend {
         VGC_HIP_CHECK(hipStreamWaitEvent(stream_, enter_ev_, 0));
     }
 
+    // memory of this context's device
+    bool on_device(const void* p) {
+        hipPointerAttribute_t a;
+        if (!p) return false;
+        if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+        return a.type == hipMemoryTypeDevice && a.device == dev_;
+    }
     void* dalloc(size_t b) {
         void* p = nullptr;
         VGC_HIP_CHECK(hipMalloc(&p, b ? b : 1));
