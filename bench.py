@@ -25,7 +25,7 @@ The JSON line also carries:
                 traffic (HBM bytes per launch) and valu_busy_frac (share of
                 the VALU issue slots in use, the kernel's actual bound) are
                 read from the committed rocprofv3 counter summary
-                profiles/k_clip_counters_2M_mixture.md (default workload only);
+                profiles/k_pair_counters_2M_mixture.md (default workload only);
   cpu_baseline  the oracle (a plain-C restatement of geogram's VBW cell +
                 security-radius loop with exact predicates) on the host cores,
                 on a bounded sample of the same workload;
@@ -56,7 +56,7 @@ sys.path.insert(0, ROOT)
 
 FP64_PEAK_TFLOPS = 78.6
 HBM_PEAK_GBS = 8000.0
-COUNTERS = os.path.join(ROOT, "profiles", "k_clip_counters_2M_mixture.md")
+COUNTERS = os.path.join(ROOT, "profiles", "k_pair_counters_2M_mixture.md")
 
 
 def profile_figure(key):
@@ -202,8 +202,8 @@ def main():
     clip_ms = float(np.mean([t["t_clip_a_gpu_ms"] for t in stats]))
     achieved = flops_a / (clip_ms * 1e-3) / 1e12
     roofline = {
-        "kernel": "k_clip<1,1,false,true,false,false,true> (first clipping pass, every cell, "
-                  "FP32 corner state)",
+        "kernel": "k_pair<1,false,false> (first clipping pass, every cell, two per "
+                  "wavefront, FP32 corner state)",
         "bound": "valu",
         "achieved": round(achieved, 4),
         "peak": FP64_PEAK_TFLOPS,
@@ -211,7 +211,7 @@ def main():
         "frac": round(achieved / FP64_PEAK_TFLOPS, 5),
         "traffic": profile_figure("traffic_bytes_per_launch") if args.n == 2_000_000 and args.k0 == 0 else None,
         "traffic_unit": "bytes per launch (rocprofv3 FETCH_SIZE + WRITE_SIZE, copy-calibrated; "
-                        "from profiles/k_clip_counters_2M_mixture.md when it was taken of "
+                        "from profiles/k_pair_counters_2M_mixture.md when it was taken of "
                         "these kernel sources, else null)",
         "valu_busy_frac": profile_figure("valu_busy_frac") if args.n == 2_000_000 and args.k0 == 0 else None,
         "alg_flops_per_launch": int(flops_a),

@@ -1,0 +1,108 @@
+"""The wavefront kernels at the edges of their sizes: the FP32 first pass
+(1, 2, 4 or 8 cells per wavefront, in halves) against the FP64 first pass,
+which writes the same bits; the exact kNN (up to 96 entries by a wavefront, 128
+candidates) against brute force; device outputs against host outputs."""
+import numpy as np
+import pytest
+
+
+def _same_cells(a, b):
+    assert np.array_equal(a.vol, b.vol)
+    assert np.array_equal(a.mg, b.mg)
+    assert np.array_equal(a.nbr_ptr, b.nbr_ptr)
+    m = int(a.nbr_ptr[-1])
+    assert np.array_equal(a.nbr[:m], b.nbr[:m])
+    assert np.array_equal(a.farea[:m], b.farea[:m])
+
+
+def _seeds(n, kind, seed=3):
+    rng = np.random.default_rng(seed)
+    x = rng.random((n, 3))
+    if kind == "clusters":  # cells of many rings beside dense clusters
+        k = n // 2
+        x[:k] = 0.5 + 0.004 * rng.standard_normal((k, 3))
+    elif kind == "shell":  # the seed inside has more than 64 corners
+        x = rng.standard_normal((n, 3))
+        x = 0.5 + 0.4 * x / np.linalg.norm(x, axis=1)[:, None]
+        x[n // 2] = 0.5
+    return x
+
+
+def _check_first_pass(ctx, n, kind):
+    x = _seeds(n, "uniform" if kind == "weighted" else kind)
+    w = 3.0 * n ** (-2 / 3) * np.cos(5.0 * x[:, 0]) if kind == "weighted" else None
+    a = ctx.cells(x, weights=w)
+    b = ctx.cells(x, weights=w, fp64_first=True)
+    _same_cells(a, b)
+    assert a.stats["nb_failed"] == b.stats["nb_failed"] == 0
+
+
+# one cell per wavefront up to 4096 cells, then two; trees of one leaf, of
+# fewer and of more than 64 and 256 leaves
+@pytest.mark.parametrize("n,kind", [
+    (1, "uniform"), (2, "uniform"), (3, "weighted"), (17, "uniform"), (129, "shell"),
+    (1025, "clusters"), (4096, "uniform"), (4097, "weighted"), (4099, "clusters")])
+def test_first_pass_sizes(emu_ctx, n, kind):
+    _check_first_pass(emu_ctx, n, kind)
+
+
+# the lines to 2, 4 and 8 cells per wavefront, odd remainders
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,kind", [
+    (1, "weighted"), (129, "shell"), (4095, "clusters"), (4097, "uniform"), (149_999, "uniform"),
+    (150_003, "clusters"), (150_001, "weighted"), (400_007, "uniform")])
+def test_first_pass_sizes_gpu(gpu_ctx, n, kind):
+    _check_first_pass(gpu_ctx, n, kind)
+
+
+def _check_knn(ctx, n, k, kind):
+    x = _seeds(n, "clusters" if kind == "clusters" else "uniform")
+    if kind == "lattice":  # ties, by index
+        x = np.floor(x * 6) / 6 + 1 / 12
+        x = np.unique(x, axis=0)
+        n = len(x)
+    d = ((x[:, None, :] - x[None, :, :]) ** 2)
+    d = d[:, :, 0] + d[:, :, 1] + d[:, :, 2]  # the kernel's order of operations
+    idx, d2 = ctx.knn(x, k)
+    for i in range(n):
+        o = np.lexsort((np.arange(n), d[i]))
+        o = o[o != i][:k]
+        assert np.array_equal(idx[i, :len(o)], o)
+        assert np.array_equal(d2[i, :len(o)], d[i, o])
+        assert np.all(idx[i, len(o):] == -1)
+
+
+# 1 to 96 entries by wavefronts, more by lists; every other point
+KNN = [(2, 1, "uniform"), (40, 39, "uniform"), (65, 64, "uniform"), (97, 95, "uniform"),
+       (500, 1, "uniform"), (500, 63, "clusters"), (500, 64, "uniform"), (500, 95, "uniform"),
+       (500, 96, "clusters"), (500, 16, "lattice")]
+
+
+@pytest.mark.parametrize("n,k,kind", KNN)
+def test_knn_sizes(emu_ctx, n, k, kind):
+    _check_knn(emu_ctx, n, k, kind)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,k,kind", KNN)
+def test_knn_sizes_gpu(gpu_ctx, n, k, kind):
+    _check_knn(gpu_ctx, n, k, kind)
+
+
+# outputs written straight into the caller's device arrays: not for a torus,
+# and the neighbours only where they fit
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,kw", [(1, {}), (5001, {}), (5001, {"periodic": True}),
+                                  (5001, {"neighbors": False})])
+def test_device_outputs(gpu_ctx, n, kw):
+    import torch
+    x = _seeds(n, "uniform")
+    a = gpu_ctx.cells(x, **kw)
+    b = gpu_ctx.cells(torch.from_numpy(x).cuda(), **kw)
+    assert np.array_equal(a.vol, b.vol.cpu().numpy())
+    assert np.array_equal(a.mg, b.mg.cpu().numpy())
+    if kw.get("neighbors", True):
+        m = int(a.nbr_ptr[-1])
+        assert np.array_equal(a.nbr_ptr.astype(np.int64), b.nbr_ptr.cpu().numpy())
+        assert np.array_equal(a.nbr[:m], b.nbr[:m].cpu().numpy())
+        assert np.array_equal(a.farea[:m], b.farea[:m].cpu().numpy())
