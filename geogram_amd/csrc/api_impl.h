@@ -286,7 +286,8 @@ template <class B>
 void point_extent(Ctx<B>* ctx, const double* xyz, uint32_t n, bool dev, double lo[3], double hi[3],
                   double& S) {
     if (dev) {
-        double* d = (double*)ctx->staging(7, sizeof(double) * 6);
+        // (a place of its own: callers hold others across this call)
+        double* d = (double*)ctx->staging(36, sizeof(double) * 6);
         ctx->be.extent(xyz, (long long)n, d);
         double h[6];
         ctx->be.d2h(h, d, sizeof(h));

@@ -5,6 +5,8 @@
 // library libvgc.so is the HIP build and has no CPU path.
 #define VGC_EMU 1
 
+#include <malloc.h>
+
 #include <algorithm>
 #include <cstdlib>
 #include <cstring>
@@ -21,13 +23,37 @@ namespace vgc {
 
 struct EmuBackend {
     explicit EmuBackend(int) {}
+    ~EmuBackend() {
+        for (void* p : freed_) std::free(p);
+    }
 
     void* dalloc(size_t b) {
         void* p = std::malloc(b ? b : 1);
         if (!p) throw std::bad_alloc();
         return p;
     }
-    void dfree(void* p) { std::free(p); }
+    void dfree(void* p) {
+        if (!p || !watch_) {
+            std::free(p);
+            return;
+        }
+        std::memset(p, kFreed, malloc_usable_size(p));
+        freed_.push_back(p);
+    }
+    // test hook: blocks freed from now on are filled and kept;
+    // freed_writes counts those that were written to afterwards
+    void watch_frees() { watch_ = true; }
+    int freed_writes() const {
+        int k = 0;
+        for (void* p : freed_) {
+            const unsigned char* c = (const unsigned char*)p;
+            k += !std::all_of(c, c + malloc_usable_size(p), [](unsigned char x) { return x == kFreed; });
+        }
+        return k;
+    }
+    static constexpr unsigned char kFreed = 0xA5;
+    bool watch_ = false;
+    std::vector<void*> freed_;
     bool on_device(const void* p) { return p != nullptr; }
     void h2d(void* d, const void* s, size_t b) { std::memcpy(d, s, b); }
     void d2h(void* d, const void* s, size_t b) { std::memcpy(d, s, b); }
@@ -1003,6 +1029,10 @@ int vgc_emu_mlp_adam(void* ctx, float* params, const float* grad, float* m, floa
 }
 // test hook: entries per chunk of the list tiers
 void vgc_emu_set_list_chunk(void* ctx, long long n) { ((EmuCtx*)ctx)->eng.list_chunk = n; }
+// test hooks: keep and watch the device blocks freed from now on; how many of
+// them were written to afterwards
+void vgc_emu_watch_frees(void* ctx) { ((EmuCtx*)ctx)->be.watch_frees(); }
+int vgc_emu_freed_writes(void* ctx) { return ((EmuCtx*)ctx)->be.freed_writes(); }
 int vgc_emu_det4_sign(const double* rows) {
     return vgc::det4_sign_exact(rows, rows + 4, rows + 8, rows + 12);
 }
