@@ -188,8 +188,10 @@ int api_cells(Ctx<B>* ctx, const double* xyz, const double* w, const uint32_t* i
                 ctx->err = "vgc_cells: neighbour capacity too small";
                 return VGC_ERR_CAPACITY;
             }
-            out(nbr, E.d_nbr, sizeof(int) * (size_t)E.total_neighbors);
-            out(farea, E.d_area, sizeof(double) * (size_t)E.total_neighbors);
+            if (pb.want_neighbors) {
+                out(nbr, E.d_nbr, sizeof(int) * (size_t)E.total_neighbors);
+                out(farea, E.d_area, sizeof(double) * (size_t)E.total_neighbors);
+            }
         }
         be.sync();
         if (es.nb_failed || es.nb_uncertain) {

@@ -521,6 +521,8 @@ public:
         if (build(pb, st)) return -1;
         piece_cells_.clear();
         x_total_ = 0;
+        d_nbr = nullptr;  // unless this pass wants them
+        d_area = nullptr;
         const int K0 = pb.k0;
         const bool gather = K0 == 0;
         auto t1 = now();

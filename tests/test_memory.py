@@ -1,8 +1,49 @@
 """The library's own memory and its caller's, on the CPU emulation, whose
 "device" memory is the host's."""
+import ctypes
+
 import numpy as np
 
 import geogram_amd as ga
+from geogram_amd._lib import Stats, VGC_DEVICE_PTRS, VGC_NO_NEIGHBORS, VGC_OK
+from geogram_amd import _ptr
+
+
+class _Arrays:
+    """Output arrays of n cells for the C entry, filled with -7."""
+
+    def __init__(self, n):
+        self.vol, self.mg, self.farea = np.full(n, -7.0), np.full((n, 3), -7.0), np.full(24 * n, -7.0)
+        self.ptr = np.full(n + 1, 7, dtype=np.uint64)
+        self.nbr = np.full(24 * n, -7, dtype=np.int32)
+
+    def untouched(self):
+        return (np.all(self.vol == -7) and np.all(self.mg == -7) and np.all(self.ptr == 7)
+                and self.no_neighbors())
+
+    def no_neighbors(self):
+        return bool(np.all(self.nbr == -7) and np.all(self.farea == -7))
+
+
+def _cells(ctx, x, out, flags=0, mg=None):
+    """vgc_cells on "device" arrays."""
+    box, st = np.array([0.0, 0, 0, 1, 1, 1]), Stats()
+    return ctx.lib.fn("cells")(ctx.ctx, _ptr(x), None, len(x), _ptr(box), 0, VGC_DEVICE_PTRS | flags,
+                               _ptr(out.vol), _ptr(out.mg if mg is None else mg), _ptr(out.ptr),
+                               _ptr(out.nbr), _ptr(out.farea), len(out.nbr), ctypes.byref(st))
+
+
+def test_no_neighbors_leaves_the_arrays_alone():
+    """A pass without neighbours writes none, also where an earlier pass on the
+    same context had some."""
+    x = np.random.default_rng(1).random((200, 3))
+    ctx = ga.Context.emulated()
+    a, b = _Arrays(200), _Arrays(200)
+    assert _cells(ctx, x, a) == VGC_OK
+    assert _cells(ctx, x, b, VGC_NO_NEIGHBORS) == VGC_OK
+    assert np.array_equal(a.vol, b.vol)
+    assert b.no_neighbors()
+    ctx.close()
 
 
 def test_convex_levels_of_five_seeds():
