@@ -153,11 +153,15 @@ int api_cells(Ctx<B>* ctx, const double* xyz, const double* w, const uint32_t* i
         }
         if (dev && !pb.periodic) {
             // straight into the caller's arrays, where they are on this device
-            if (be.on_device(vol)) pb.out_vol = vol;
-            if (be.on_device(mg)) pb.out_mg = mg;
-            if (be.on_device(nbr_ptr)) pb.out_ptr = (long long*)nbr_ptr;
-            if (be.on_device(nbr)) pb.out_nbr = nbr;
-            if (be.on_device(farea)) pb.out_area = farea;
+            // (and aligned: the copies below take any address)
+            auto to = [&](auto* p) {
+                return (uintptr_t)p % sizeof(*p) == 0 && be.on_device(p) ? p : nullptr;
+            };
+            pb.out_vol = to(vol);
+            pb.out_mg = to(mg);
+            pb.out_ptr = (long long*)to(nbr_ptr);
+            pb.out_nbr = to(nbr);
+            pb.out_area = to(farea);
             pb.out_cap = (long long)std::min<uint64_t>(cap, 1ull << 62);
         }
         EngineStats es;
@@ -167,20 +171,21 @@ int api_cells(Ctx<B>* ctx, const double* xyz, const double* w, const uint32_t* i
         ctx->eng.begin_call();
         if (ctx->eng.cells(pb, es)) {
             ctx->err = "vgc_cells: " + ctx->eng.error;
-            be.sync();  // nothing writes to the caller's arrays after the return
+            be.sync();  // nothing reads the caller's arrays after the return
             return VGC_ERR_INTERNAL;
         }
         Engine<B>& E = ctx->eng;
         auto out = [&](void* dst, const void* src, size_t bytes) {
-            if (!dst || dst == src) return;
+            if (!dst || !src) return;
             if (dev)
                 be.d2d(dst, src, bytes);
             else
                 be.d2h(dst, src, bytes);
         };
-        out(vol, E.d_vol, sizeof(double) * (size_t)n);
-        out(mg, E.d_mg, sizeof(double) * 3 * (size_t)n);
-        out(nbr_ptr, E.d_ptr, sizeof(long long) * ((size_t)n + 1));
+        // what the pass has not written there itself
+        if (!pb.out_vol) out(vol, E.d_vol, sizeof(double) * (size_t)n);
+        if (!pb.out_mg) out(mg, E.d_mg, sizeof(double) * 3 * (size_t)n);
+        if (!pb.out_ptr) out(nbr_ptr, E.d_ptr, sizeof(long long) * ((size_t)n + 1));
         fill_stats(es, stats);
         if (nbr || farea) {
             if ((uint64_t)E.total_neighbors > cap) {
@@ -188,10 +193,9 @@ int api_cells(Ctx<B>* ctx, const double* xyz, const double* w, const uint32_t* i
                 ctx->err = "vgc_cells: neighbour capacity too small";
                 return VGC_ERR_CAPACITY;
             }
-            if (pb.want_neighbors) {
-                out(nbr, E.d_nbr, sizeof(int) * (size_t)E.total_neighbors);
-                out(farea, E.d_area, sizeof(double) * (size_t)E.total_neighbors);
-            }
+            // (null where the pass has written them there itself or has none)
+            out(nbr, E.d_nbr, sizeof(int) * (size_t)E.total_neighbors);
+            out(farea, E.d_area, sizeof(double) * (size_t)E.total_neighbors);
         }
         be.sync();
         if (es.nb_failed || es.nb_uncertain) {

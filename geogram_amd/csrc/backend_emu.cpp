@@ -28,6 +28,7 @@ struct EmuBackend {
     }
 
     void* dalloc(size_t b) {
+        if (fail_alloc_ && --fail_alloc_ == 0) throw std::bad_alloc();
         void* p = std::malloc(b ? b : 1);
         if (!p) throw std::bad_alloc();
         return p;
@@ -53,6 +54,7 @@ struct EmuBackend {
     }
     static constexpr unsigned char kFreed = 0xA5;
     bool watch_ = false;
+    int fail_alloc_ = 0;  // test hook: this allocation from now on fails (0: none)
     std::vector<void*> freed_;
     bool on_device(const void* p) { return p != nullptr; }
     void h2d(void* d, const void* s, size_t b) { std::memcpy(d, s, b); }
@@ -376,12 +378,15 @@ struct EmuBackend {
     }
 
     void compact(int n, const int* cnt, const long long* ptr, const int* nbr_tmp,
-                 const double* area_tmp, int stride, int* nbr, double* area) {
-        for (int i = 0; i < n; ++i)
+                 const double* area_tmp, int stride, int* nbr, double* area, const CellOut& O) {
+        for (int i = 0; nbr && i < n; ++i)
             for (int k = 0; k < std::min(cnt[i], stride); ++k) {
                 nbr[ptr[i] + k] = nbr_tmp[(size_t)i * stride + k];
                 area[ptr[i] + k] = area_tmp[(size_t)i * stride + k];
             }
+        if (O.to_vol) std::copy(O.vol, O.vol + n, O.to_vol);
+        if (O.to_mg) std::copy(O.mg, O.mg + 3 * (size_t)n, O.to_mg);
+        if (O.to_ptr) std::copy(ptr, ptr + n + 1, O.to_ptr);
     }
 
     void lloyd_update(double* xyz, const double* vol, const double* mg, int n,
@@ -1029,9 +1034,10 @@ int vgc_emu_mlp_adam(void* ctx, float* params, const float* grad, float* m, floa
 }
 // test hook: entries per chunk of the list tiers
 void vgc_emu_set_list_chunk(void* ctx, long long n) { ((EmuCtx*)ctx)->eng.list_chunk = n; }
-// test hooks: keep and watch the device blocks freed from now on; how many of
-// them were written to afterwards
+// test hooks: the k-th device allocation from now on fails; keep and watch the
+// blocks freed from now on; how many of them were written to afterwards
 void vgc_emu_watch_frees(void* ctx) { ((EmuCtx*)ctx)->be.watch_frees(); }
+void vgc_emu_fail_alloc(void* ctx, int k) { ((EmuCtx*)ctx)->be.fail_alloc_ = k; }
 int vgc_emu_freed_writes(void* ctx) { return ((EmuCtx*)ctx)->be.freed_writes(); }
 int vgc_emu_det4_sign(const double* rows) {
     return vgc::det4_sign_exact(rows, rows + 4, rows + 8, rows + 12);

@@ -330,14 +330,20 @@ __global__ void k_rebase(const long long* __restrict__ off, int n, long long bas
 constexpr int kCompactLanes = 16;
 __global__ void k_compact(int n, const int* __restrict__ cnt, const long long* __restrict__ ptr,
                           const int* __restrict__ nbr_tmp, const double* __restrict__ area_tmp,
-                          int stride, int* nbr, double* area) {
+                          int stride, int* nbr, double* area, CellOut O) {
     const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     const long long i = t / kCompactLanes;
     if (i >= n) return;
+    const int l = int(t % kCompactLanes);
+    if (l < 3 && O.to_mg) O.to_mg[3 * i + l] = O.mg[3 * i + l];
+    if (l == 3 && O.to_vol) O.to_vol[i] = O.vol[i];
+    if (l == 4 && O.to_ptr) O.to_ptr[i] = ptr[i];
+    if (l == 5 && O.to_ptr && i == n - 1) O.to_ptr[n] = ptr[n];
+    if (!nbr) return;
     const long long o = ptr[i];
     const int m = min(cnt[i], stride);  // longer lists (pieces) are copied on their own
     const size_t row = (size_t)i * stride;
-    for (int k = int(t % kCompactLanes); k < m; k += kCompactLanes) {
+    for (int k = l; k < m; k += kCompactLanes) {
         nbr[o + k] = nbr_tmp[row + k];
         area[o + k] = area_tmp[row + k];
     }
@@ -1810,9 +1816,9 @@ struct HipBackend {
                                                           off + 1, 0, 32, stream_));
     }
     void compact(int n, const int* cnt, const long long* ptr, const int* nbr_tmp,
-                 const double* area_tmp, int stride, int* nbr, double* area) {
+                 const double* area_tmp, int stride, int* nbr, double* area, const CellOut& O) {
         k_compact<<<blocks_for((long long)n * kCompactLanes, 256), 256, 0, stream_>>>(
-            n, cnt, ptr, nbr_tmp, area_tmp, stride, nbr, area);
+            n, cnt, ptr, nbr_tmp, area_tmp, stride, nbr, area, O);
         check();
     }
     void lloyd_update(double* xyz, const double* vol, const double* mg, int n,

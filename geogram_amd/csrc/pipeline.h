@@ -71,9 +71,10 @@ struct Problem {
     bool want_neighbors = true;
     bool want_e2 = false;           // integral of |x - p|^2 per cell (CVT energy)
     bool count_work = false;        // algorithmic work counters (global atomics)
-    // device memory for the outputs, if the caller's arrays can take them
-    // directly (not periodic, no subset of instances; the CSR entries only if
-    // they fit out_cap)
+    // the caller's device arrays that take the outputs directly (not periodic;
+    // the CSR entries only if both are given and they fit out_cap).  They are
+    // written by the last launch of a pass that succeeded, and the members
+    // d_vol .. d_area below never point to them.
     double* out_vol = nullptr;
     double* out_mg = nullptr;
     long long* out_ptr = nullptr;
@@ -536,8 +537,8 @@ public:
             st.t_knn_gpu_ms += be_.event_ms(0);
         }
 
-        d_vol = pb.out_vol ? pb.out_vol : (double*)slot(S_VOL, sizeof(double) * (size_t)n_);
-        d_mg = pb.out_mg ? pb.out_mg : (double*)slot(S_MG, sizeof(double) * 3 * (size_t)n_);
+        d_vol = (double*)slot(S_VOL, sizeof(double) * (size_t)n_);
+        d_mg = (double*)slot(S_MG, sizeof(double) * 3 * (size_t)n_);
         int* d_cnt = (int*)slot(S_CNT, sizeof(int) * (size_t)n_);
         int* d_nbr_tmp = (int*)slot(S_NBRTMP, sizeof(int) * (size_t)n_ * kFaceStride);
         double* d_area_tmp = (double*)slot(S_AREATMP, sizeof(double) * (size_t)n_ * kFaceStride);
@@ -734,7 +735,7 @@ public:
         // along with them (again below if a later pass changes a count).
         if ((int)h_flags.size() < n_) h_flags.resize(n_);
         census_.clear();
-        d_ptr = pb.out_ptr ? pb.out_ptr : (long long*)slot(S_PTR, sizeof(long long) * ((size_t)n_ + 1));
+        d_ptr = (long long*)slot(S_PTR, sizeof(long long) * ((size_t)n_ + 1));
         {
             be_.census(P.items, P.n_items, d_flags, kCensusMask, CELL_DONE, P.abort_flag, P.inst_of,
                        nullptr, d_cen + 2, d_cen);
@@ -872,18 +873,25 @@ public:
             be_.d2h(&total_neighbors, d_ptr + n_, sizeof(long long));
         }
         st.nb_neighbors += total_neighbors;
+        int* nbr = nullptr;
+        double* area = nullptr;
         if (pb.want_neighbors) {
-            const bool direct = pb.out_nbr && pb.out_area && total_neighbors <= pb.out_cap;
-            d_nbr = direct ? pb.out_nbr
-                           : (int*)slot(S_NBR, sizeof(int) * std::max<long long>(1, total_neighbors));
-            d_area = direct ? pb.out_area
-                            : (double*)slot(S_AREA, sizeof(double) * std::max<long long>(1, total_neighbors));
-            be_.compact(n_, d_cnt, d_ptr, d_nbr_tmp, d_area_tmp, kFaceStride, d_nbr, d_area);
-            if (!piece_cells_.empty())
-                be_.piece_copy((int)piece_cells_.size(), (const int*)slots_[S_XCELLS].p, d_orig,
-                               (const long long*)slots_[S_XOFF].p, (const int*)slots_[S_XNBR].p,
-                               (const double*)slots_[S_XAREA].p, d_cnt, d_ptr, d_nbr, d_area);
+            if (pb.out_nbr && pb.out_area && total_neighbors <= pb.out_cap) {
+                nbr = pb.out_nbr;
+                area = pb.out_area;
+            } else {
+                const size_t m = (size_t)std::max<long long>(1, total_neighbors);
+                nbr = d_nbr = (int*)slot(S_NBR, sizeof(int) * m);
+                area = d_area = (double*)slot(S_AREA, sizeof(double) * m);
+            }
         }
+        const CellOut O{d_vol, d_mg, pb.out_vol, pb.out_mg, pb.out_ptr};
+        if (nbr || O.any())
+            be_.compact(n_, d_cnt, d_ptr, d_nbr_tmp, d_area_tmp, kFaceStride, nbr, area, O);
+        if (nbr && !piece_cells_.empty())
+            be_.piece_copy((int)piece_cells_.size(), (const int*)slots_[S_XCELLS].p, d_orig,
+                           (const long long*)slots_[S_XOFF].p, (const int*)slots_[S_XNBR].p,
+                           (const double*)slots_[S_XAREA].p, d_cnt, d_ptr, nbr, area);
         st.t_compact_ms += ms_since(t4);
         st.t_total_ms += ms_since(tstart);
         return 0;

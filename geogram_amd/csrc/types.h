@@ -57,6 +57,15 @@ VGC_SD float dist2f(const pf4& a, float px, float py, float pz) {
     return dx * dx + dy * dy + dz * dz;
 }
 
+// Per-cell outputs and the caller's device arrays that take them at the end of
+// a pass (null: not wanted).
+struct CellOut {
+    const double *vol, *mg;
+    double *to_vol, *to_mg;
+    long long* to_ptr;
+    bool any() const { return to_vol || to_mg || to_ptr; }
+};
+
 // Per-instance layout of the Morton-ordered seeds, buckets and trees.
 struct InstLayout {
     const int* inst_of;       // Morton position -> instance (nullptr: one)

@@ -177,7 +177,9 @@ int vgc_knn_search(vgc_ctx* ctx, const double* xyz, uint32_t n, const double* q,
    v_global_index of contributing planes, convex_cell.h:728-741,830) and their
    facet areas (ConvexCell::facet_area, convex_cell.cpp:1160-1191).
    nbr / farea may be NULL; if cap is too small the call returns
-   VGC_ERR_CAPACITY with the required size in stats->nb_neighbors.
+   VGC_ERR_CAPACITY with the required size in stats->nb_neighbors, vol, mg and
+   nbr_ptr written.  Any other error leaves the arrays as they were: they are
+   written when every pass has succeeded.
    k0: 0 (default) lets each cell's wavefront gather its own neighbours,
    nearest first, ring after ring of distance, until the security radius is
    reached; 16, 24, 32, 48 or 64 first computes kNN lists of that size. */

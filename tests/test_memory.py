@@ -5,7 +5,7 @@ import ctypes
 import numpy as np
 
 import geogram_amd as ga
-from geogram_amd._lib import Stats, VGC_DEVICE_PTRS, VGC_NO_NEIGHBORS, VGC_OK
+from geogram_amd._lib import Stats, VGC_DEVICE_PTRS, VGC_NO_NEIGHBORS, VGC_OK, VGC_ERR_DEVICE
 from geogram_amd import _ptr
 
 
@@ -60,4 +60,35 @@ def test_convex_levels_of_five_seeds():
     assert all(s["converged"] for s in sts)
     vol = ctx.cells(x, weights=w).vol
     assert np.abs(vol - nu).max() <= 1e-6 * 0.2
+    ctx.close()
+
+
+def test_a_failed_call_leaves_the_arrays_alone():
+    """The caller's arrays are written when every pass has succeeded: whichever
+    allocation of a call fails, they hold what they held."""
+    x = np.random.default_rng(2).random((300, 3))
+    x[:2] = x[2]  # coincident seeds: the exact pass runs too
+    failures = 0
+    while True:
+        ctx, a = ga.Context.emulated(), _Arrays(300)
+        ctx.lib.cdll.vgc_emu_fail_alloc(ctx.ctx, failures + 1)
+        rc = _cells(ctx, x, a)
+        ctx.close()
+        if rc == VGC_OK:
+            break
+        assert rc == VGC_ERR_DEVICE
+        assert a.untouched(), f"allocation {failures + 1}"
+        failures += 1
+    assert failures > 10 and not a.untouched()
+
+
+def test_outputs_over_inputs():
+    """Centroids written over the seeds, as in a Lloyd step in place."""
+    x = np.random.default_rng(4).random((500, 3))
+    ctx, a, b = ga.Context.emulated(), _Arrays(500), _Arrays(500)
+    assert _cells(ctx, x, a) == VGC_OK
+    y = x.copy()
+    assert _cells(ctx, y, b, mg=y) == VGC_OK
+    assert np.array_equal(a.mg, y) and np.array_equal(a.vol, b.vol)
+    assert np.array_equal(a.nbr, b.nbr) and np.array_equal(a.farea, b.farea)
     ctx.close()
