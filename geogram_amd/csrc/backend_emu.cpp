@@ -180,9 +180,11 @@ struct EmuBackend {
         }
     }
 
+    int groups_ = 0;  // test hook: cells per wavefront of the launches so far
     // the first pass with FP32 corner state, two cells per wavefront
     void clip_pairs(const ClipParams& P) {
-        const int group = pair_group(P.n_items);
+        const int group = P.group;
+        groups_ |= group;
 #pragma omp parallel
         {
             std::unique_ptr<PairLds> L(new PairLds());
@@ -1039,6 +1041,10 @@ void vgc_emu_set_list_chunk(void* ctx, long long n) { ((EmuCtx*)ctx)->eng.list_c
 void vgc_emu_watch_frees(void* ctx) { ((EmuCtx*)ctx)->be.watch_frees(); }
 void vgc_emu_fail_alloc(void* ctx, int k) { ((EmuCtx*)ctx)->be.fail_alloc_ = k; }
 int vgc_emu_freed_writes(void* ctx) { return ((EmuCtx*)ctx)->be.freed_writes(); }
+// test hooks: cells per run of the work-group tuner's sample; the cells per
+// wavefront that first passes have run with (1, 2, 4, 8: one bit each)
+void vgc_emu_set_tune_run(void* ctx, int n) { ((EmuCtx*)ctx)->eng.tune_run = n; }
+int vgc_emu_pair_groups(void* ctx) { return ((EmuCtx*)ctx)->be.groups_; }
 int vgc_emu_det4_sign(const double* rows) {
     return vgc::det4_sign_exact(rows, rows + 4, rows + 8, rows + 12);
 }

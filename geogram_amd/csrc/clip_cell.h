@@ -189,7 +189,8 @@ struct ClipParams {
     const double* item_box;
     int piece;
     // host dispatch: the first pass with FP32 corner state (pair_cell.h), and
-    // its cells per wavefront (even, at most 16)
+    // its cells per wavefront (pair_group: 1, 2, 4 or 8; with 1, and at an odd
+    // end, a pair has no second cell)
     int fp32;
     int group;
     int pair_rings;  // its filtered rings before the cell goes to the second gather

@@ -108,12 +108,10 @@ __global__ __launch_bounds__(64 * WAVES, 4) void k_pair(ClipParams P) {
 
 template <bool W, bool COUNT>
 static void clip_pairs(const ClipParams& P, int waves, hipStream_t stream) {
-    ClipParams Q = P;
-    Q.group = pair_group(P.n_items);
     if (waves == 1)
-        k_pair<1, W, COUNT><<<blocks_for(Q.n_items, Q.group), 64, 0, stream>>>(Q);
+        k_pair<1, W, COUNT><<<blocks_for(P.n_items, P.group), 64, 0, stream>>>(P);
     else
-        k_pair<4, W, COUNT><<<blocks_for(Q.n_items, 4 * Q.group), 256, 0, stream>>>(Q);
+        k_pair<4, W, COUNT><<<blocks_for(P.n_items, 4 * P.group), 256, 0, stream>>>(P);
 }
 
 void launch_pairs(const ClipParams& P, int waves, hipStream_t stream) {

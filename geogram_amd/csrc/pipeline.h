@@ -137,6 +137,7 @@ public:
     long long total_neighbors = 0;
     long long list_chunk = 1ll << 27;  // entries per chunk of the list tiers
     bool autotune = false;             // pick the first pass's work-group size by timing
+    int tune_run = 2048;               // cells per run of the tuner's sample
     bool waves4 = false;               // first pass with 4-wavefront work-groups (no tuner)
     bool fp64_first = false;           // first pass with FP64 corner state (default FP32)
     // start of a library call: the FP32 / FP64 choice of the first pass
@@ -613,6 +614,7 @@ public:
         P.list_stride = K0;
         P.list_complete = 0;
         P.ring_limit = weighted_ ? kMaxFilteredRings : kMaxVoronoiRings;
+        P.group = pair_group(P.n_items);  // (the tuner's sample runs with it too)
         P.pair_rings = weighted_ ? kMaxPairRingsW : kMaxPairRings;
         P.corner = 0;
         // FP32 corner state for the first pass, except for cell meshes (those
@@ -644,13 +646,13 @@ public:
             ClipParams T = P;
             T.counters = nullptr;
             T.abort_flag = nullptr;
-            const int kRun = 2048, kRuns = 128;
-            if (P.n_items > 2 * kRun * kRuns) {
+            const int kRuns = 128;
+            if (P.n_items > 2 * tune_run * kRuns) {
                 std::vector<int> titems;
-                titems.reserve((size_t)kRun * kRuns);
+                titems.reserve((size_t)tune_run * kRuns);
                 for (int j = 0; j < kRuns; ++j) {
                     const long long b = (long long)P.n_items * j / kRuns;
-                    for (int i = 0; i < kRun; ++i)
+                    for (int i = 0; i < tune_run; ++i)
                         titems.push_back(pb.active ? aitems[b + i] : (int)(b + i));
                 }
                 int* d_t = (int*)slot(S_TITEMS, sizeof(int) * titems.size());

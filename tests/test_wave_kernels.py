@@ -5,6 +5,8 @@ candidates) against brute force; device outputs against host outputs."""
 import numpy as np
 import pytest
 
+import geogram_amd as ga
+
 
 def _same_cells(a, b):
     assert np.array_equal(a.vol, b.vol)
@@ -106,3 +108,16 @@ def test_device_outputs(gpu_ctx, n, kw):
         assert np.array_equal(a.nbr_ptr.astype(np.int64), b.nbr_ptr.cpu().numpy())
         assert np.array_equal(a.nbr[:m], b.nbr[:m].cpu().numpy())
         assert np.array_equal(a.farea[:m], b.farea[:m].cpu().numpy())
+
+
+def test_tuner_times_the_launch_that_runs():
+    """The work-group tuner's sample runs with the cells per wavefront of the
+    whole pass (here 2; the sample alone would take 1)."""
+    ctx = ga.Context.emulated()
+    ctx.lib.cdll.vgc_emu_set_tune_run(ctx.ctx, 8)
+    x = _seeds(4100, "uniform")
+    a = ctx.cells(x, autotune=True)
+    assert a.stats["tuned_waves"] in (1, 4)
+    assert ctx.lib.cdll.vgc_emu_pair_groups(ctx.ctx) == 2
+    _same_cells(a, ctx.cells(x))
+    ctx.close()
