@@ -31,7 +31,7 @@ import sys
 
 _CSRC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc")
 KERNEL_SOURCES = ("clip_cell.h", "pair_cell.h", "knn_wave.h", "wave.h", "types.h", "common.h",
-                  "exact_det.h", "clip_kernels.hip", "backend_hip.hip", "ot_kernels.h",
+                  "exact_det.h", "clip_kernels.hip", "clip_launch.h", "backend_hip.hip", "ot_kernels.h",
                   "surface.h", "mlp.h")
 
 # MI355X: 256 CUs x 4 SIMDs; SQ_BUSY_CYCLES is summed over 32 shader engines

@@ -2,6 +2,9 @@
 (1, 2, 4 or 8 cells per wavefront, in halves) against the FP64 first pass,
 which writes the same bits; the exact kNN (up to 96 entries by a wavefront, 128
 candidates) against brute force; device outputs against host outputs."""
+import pathlib
+import re
+
 import numpy as np
 import pytest
 
@@ -121,3 +124,15 @@ def test_tuner_times_the_launch_that_runs():
     assert ctx.lib.cdll.vgc_emu_pair_groups(ctx.ctx) == 2
     _same_cells(a, ctx.cells(x))
     ctx.close()
+
+
+def test_profiled_sources_are_all_kernel_sources():
+    """The hash that dates a committed profile covers every file with device
+    code."""
+    from geogram_amd import profiling
+    csrc = pathlib.Path(profiling._CSRC)
+    device = {f.name for f in csrc.iterdir()
+              if re.search(r"__global__|__device__|VGC_HD|VGC_SD", f.read_text())}
+    device.discard("backend_emu.cpp")
+    assert device <= set(profiling.KERNEL_SOURCES)
+    assert set(profiling.KERNEL_SOURCES) <= {f.name for f in csrc.iterdir()}
