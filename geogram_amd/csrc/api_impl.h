@@ -175,6 +175,15 @@ int api_cells(Ctx<B>* ctx, const double* xyz, const double* w, const uint32_t* i
             return VGC_ERR_INTERNAL;
         }
         Engine<B>& E = ctx->eng;
+        if (stats) {
+            // the compaction is launched, not awaited, by the pass
+            const auto t = std::chrono::steady_clock::now();
+            be.sync();
+            const double ms = std::chrono::duration<double, std::milli>(
+                                  std::chrono::steady_clock::now() - t).count();
+            es.t_compact_ms += ms;
+            es.t_total_ms += ms;
+        }
         auto out = [&](void* dst, const void* src, size_t bytes) {
             if (!dst || !src) return;
             if (dev)

@@ -1586,7 +1586,7 @@ struct HipBackend {
         pin_used_ = 0;
     }
     // HIP events on the launch stream around a phase (slot 0: kNN, 1: pass A,
-    // 2: its FP64 redo)
+    // 2: its FP64 redo, 3: build)
     void event_begin(int k) {
         if (!ev_[k][0]) {
             VGC_HIP_CHECK(hipEventCreate(&ev_[k][0]));
@@ -2261,7 +2261,7 @@ private:
     hipStream_t stream_ = nullptr;
     hipStream_t caller_ = nullptr;
     hipEvent_t enter_ev_ = nullptr;
-    hipEvent_t ev_[3][2] = {};
+    hipEvent_t ev_[4][2] = {};
     static constexpr size_t kPinBytes = 256 << 10, kPinChunk = 32 << 10;
     char* pin_ = nullptr;   // pinned buffer of the small copies
     size_t pin_used_ = 0;

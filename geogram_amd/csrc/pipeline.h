@@ -260,7 +260,7 @@ public:
         weighted_ = pb.d_w != nullptr;
         d_wmax_ = (double*)slot(S_WMAX, sizeof(double) * ni_);
         if (weighted_) be_.wmax(d_pts, IL, ni_, *std::max_element(h_n_.begin(), h_n_.begin() + ni_), d_wmax_);
-        // (launched, not awaited: the phase times are host times)
+        // (launched, not awaited)
         st.t_build_ms += ms_since(t0);
         return 0;
     }
@@ -520,23 +520,34 @@ public:
 
     int cells_core(const Problem& pb, EngineStats& st) {
         auto tstart = now();
+        const double tb0 = st.t_build_ms;
+        be_.event_begin(3);
         if (build(pb, st)) return -1;
+        be_.event_end(3);
+        // after the first wait: the build's time (its launches return early)
+        // counted as such, the rest of the time so far is the next phase's
+        auto after_build = [&] {
+            const double launch = st.t_build_ms - tb0, all = ms_since(tstart);
+            const double ms = std::min(all, std::max(launch, be_.event_ms(3)));
+            st.t_build_ms = tb0 + ms;
+            return all - ms;
+        };
         piece_cells_.clear();
         x_total_ = 0;
         d_nbr = nullptr;  // unless this pass wants them
         d_area = nullptr;
         const int K0 = pb.k0;
         const bool gather = K0 == 0;
-        auto t1 = now();
         int* d_list = nullptr;
         if (!gather) {
             be_.event_begin(0);
             knn_lists(K0, d_list);
             be_.event_end(0);
             be_.sync();
-            st.t_knn_ms += ms_since(t1);
+            st.t_knn_ms += after_build();
             st.t_knn_gpu_ms += be_.event_ms(0);
         }
+        auto t2 = now();
 
         d_vol = (double*)slot(S_VOL, sizeof(double) * (size_t)n_);
         d_mg = (double*)slot(S_MG, sizeof(double) * 3 * (size_t)n_);
@@ -599,7 +610,6 @@ public:
         d_r2_ = d_r2;
 
         // pass A over every cell, then the tiers for the flagged ones
-        auto t2 = now();
         P.items = nullptr;
         P.n_items = n_;
         if (pb.active) {
@@ -709,7 +719,15 @@ public:
             be_.clip_listed(P, d_cc, d_cen + 1);
             be_.event_end(2);
         }
-        auto t3 = now();
+        // after the wait: pass A's time and that of its redo
+        auto after_pass = [&] {
+            const double ms = gather ? after_build() : ms_since(t2);
+            const double r = redo ? std::min(ms, be_.event_ms(2)) : 0.0;
+            st.t_clip_ms += ms - r;
+            st.t_pass_bc_ms += r;
+            st.t_redo_gpu_ms += r;
+            st.t_clip_a_gpu_ms += be_.event_ms(1);
+        };
         // instances stopped by an empty cell: bad; no further pass for them
         std::vector<unsigned> stopped;
         if (P.abort_flag) {
@@ -725,8 +743,7 @@ public:
             if (nstop == nlive) {
                 inst_bad.assign(ni_, 0);
                 for (int k = 0; k < ni_; ++k) inst_bad[k] = stopped[k] ? 1 : 0;
-                st.t_clip_ms += ms_since(t2);
-                st.t_clip_a_gpu_ms += be_.event_ms(1);
+                after_pass();
                 st.t_total_ms += ms_since(tstart);
                 return 1;
             }
@@ -753,7 +770,6 @@ public:
             if (redo) {
                 st.nb_fp64_redo += head[1];
                 if ((size_t)head[1] * 2 > (size_t)P.n_items) fp32_skip_ = kFp32Skip;
-                st.t_redo_gpu_ms += be_.event_ms(2);
             }
             std::vector<std::pair<int, uint32_t>> ord(m);
             for (size_t i = 0; i < m; ++i) ord[i] = {(int)head[2 + 2 * i], head[3 + 2 * i]};
@@ -764,8 +780,8 @@ public:
                 h_flags[ord[i].first] = ord[i].second;
             }
         }
-        st.t_clip_ms += ms_since(t2);
-        st.t_clip_a_gpu_ms += be_.event_ms(1);
+        after_pass();
+        auto t3 = now();
         std::vector<int> need, over;
         long long nempty = 0;
         for (int c : census_) {

@@ -104,6 +104,10 @@ typedef struct vgc_stats {
     uint64_t nb_clips;        /* planes that cut a cell (VGC_COUNT_WORK)          */
     uint64_t nb_tests;        /* planes tested against a cell (VGC_COUNT_WORK)    */
     uint64_t radius_entries;  /* seeds gathered by the radius pass                */
+    /* phases of a call, each moment counted once: building (sort and tree),
+       kNN lists (k0 > 0), the first clipping pass, the passes after it (the
+       FP64 redo of the first one included), the neighbour CSR (vgc_cells and
+       vgc_cells_batch; elsewhere its launch only) */
     double t_build_ms, t_knn_ms, t_clip_ms, t_pass_bc_ms, t_compact_ms, t_total_ms;
     /* first clipping pass (one launch over every cell): GPU time from events
        on the launch stream, and (with VGC_COUNT_WORK) its algorithmic work:
