@@ -19,7 +19,14 @@ template <int S, int WAVES, bool EXACT, bool GATHER, bool W, bool CORNER = W>
 __global__ __launch_bounds__(64 * WAVES, (S == 1 && !EXACT) ? 4 : 1) void k_clip(ClipParams P) {
     __shared__ CellLds<S> lds[WAVES];
     const int wave = WAVES == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int item = xcd_block() * WAVES + wave;
+    int item = xcd_block() * WAVES + wave;
+    // The item in a vector register: with a scalar one the compiler keeps all
+    // that follows from it in scalar registers, runs out of them and spills
+    // (S = 4 from lists: 124 spilled and 308 vector registers, against 36 and
+    // 231).  50 large cells of a clustered transport of 1M seeds: S = 2, 4, 8
+    // 34, 65, 140 ms scalar; cells of its first 13 Newton steps 3.07 s scalar,
+    // 2.39 s so.
+    asm volatile("" : "+v"(item));
     if (item >= P.n_items) return;  // whole wavefront
     process_cell<S, EXACT, GATHER, W, CORNER>(P, item, lds[wave]);
 }
