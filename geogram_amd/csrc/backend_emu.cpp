@@ -878,7 +878,9 @@ struct EmuBackend {
             for (int t = 0; t < K.nq; t += kKnnGroup)
                 process_knn(K, t, std::min(kKnnGroup, K.nq - t), *L);
         }
+        knn_left_ += *K.nfail;
     }
+    unsigned knn_left_ = 0;  // test hook: queries left to the lists so far
     void knn_count(const pf4* pf, const bnode* nodes, const InstLayout& IL, const pf4* qf,
                    const int* items, int ni, const float* rr, int* cnt) {
 #pragma omp parallel for schedule(dynamic, 64)
@@ -1041,6 +1043,7 @@ void vgc_emu_set_list_chunk(void* ctx, long long n) { ((EmuCtx*)ctx)->eng.list_c
 void vgc_emu_watch_frees(void* ctx) { ((EmuCtx*)ctx)->be.watch_frees(); }
 void vgc_emu_fail_alloc(void* ctx, int k) { ((EmuCtx*)ctx)->be.fail_alloc_ = k; }
 int vgc_emu_freed_writes(void* ctx) { return ((EmuCtx*)ctx)->be.freed_writes(); }
+unsigned vgc_emu_knn_left(void* ctx) { return ((EmuCtx*)ctx)->be.knn_left_; }
 // test hooks: cells per run of the work-group tuner's sample; the cells per
 // wavefront that first passes have run with (1, 2, 4, 8: one bit each)
 void vgc_emu_set_tune_run(void* ctx, int n) { ((EmuCtx*)ctx)->eng.tune_run = n; }

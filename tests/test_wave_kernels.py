@@ -60,6 +60,38 @@ def test_first_pass_sizes_gpu(gpu_ctx, n, kind):
     _check_first_pass(gpu_ctx, n, kind)
 
 
+# instances that meet within a wavefront, of spacings far apart: it starts the
+# cells of all of them from the first one's
+def _check_batch(ctx, count, weighted):
+    rng = np.random.default_rng(11)
+    sizes = rng.integers(1, 12, count)
+    scale = 10.0 ** rng.uniform(-4, 4, count)
+    x = np.concatenate([s * rng.random((n, 3)) for n, s in zip(sizes, scale)])
+    boxes = np.zeros((count, 6))
+    boxes[:, 3:] = scale[:, None]
+    w = np.repeat(0.05 * scale ** 2, sizes) * rng.random(len(x)) if weighted else None
+    a = ctx.cells(x, weights=w, inst_n=sizes, boxes=boxes)
+    b = ctx.cells(x, weights=w, inst_n=sizes, boxes=boxes, fp64_first=True)
+    _same_cells(a, b)
+    assert a.stats["nb_failed"] == 0
+    # every instance fills its box
+    vol = np.add.reduceat(a.vol, np.concatenate([[0], np.cumsum(sizes)[:-1]]))
+    assert np.abs(vol / scale ** 3 - 1.0).max() < 1e-10
+
+
+@pytest.mark.parametrize("count,weighted", [(100, False), (900, False), (900, True)])
+def test_first_pass_batches(emu_ctx, count, weighted):
+    _check_batch(emu_ctx, count, weighted)
+
+
+# 1, 2, 4 and 8 cells per wavefront
+@pytest.mark.gpu
+@pytest.mark.parametrize("count,weighted", [(100, False), (900, True), (30_000, False),
+                                            (30_000, True), (70_000, False)])
+def test_first_pass_batches_gpu(gpu_ctx, count, weighted):
+    _check_batch(gpu_ctx, count, weighted)
+
+
 def _check_knn(ctx, n, k, kind):
     x = _seeds(n, "clusters" if kind == "clusters" else "uniform")
     if kind == "lattice":  # ties, by index
@@ -92,6 +124,37 @@ def test_knn_sizes(emu_ctx, n, k, kind):
 @pytest.mark.parametrize("n,k,kind", KNN)
 def test_knn_sizes_gpu(gpu_ctx, n, k, kind):
     _check_knn(gpu_ctx, n, k, kind)
+
+
+# queries whose first radius holds far too few points: beside the points, and
+# lone points around a dense cluster.  A wavefront finds the radius of each (the
+# lists take a thousand times as long for such a query).
+def _check_knn_far(ctx, left):
+    rng = np.random.default_rng(8)
+    u = rng.random((4000, 3))
+    x = 0.5 + 0.02 * rng.standard_normal((20000, 3))
+    x[:100] = rng.random((100, 3))
+    for pts, q, k in [(u, 5.0 + rng.random((500, 3)), 8), (u, 3.0 * rng.random((500, 3)) - 1.0, 16),
+                      (x, x[:100], 17), (x, rng.random((200, 3)), 1), (x, rng.random((200, 3)), 96)]:
+        idx, d2 = ctx.knn_search(pts, q, k)
+        for i in range(len(q)):
+            d = (pts - q[i]) ** 2
+            d = d[:, 0] + d[:, 1] + d[:, 2]
+            o = np.argsort(d, kind="stable")[:k]
+            assert np.array_equal(idx[i], o) and np.array_equal(d2[i], d[o])
+    if left is not None:
+        assert left() <= 5
+
+
+def test_knn_far(emu_ctx):
+    f, c = emu_ctx.lib.cdll.vgc_emu_knn_left, emu_ctx.ctx
+    before = f(c)
+    _check_knn_far(emu_ctx, lambda: f(c) - before)
+
+
+@pytest.mark.gpu
+def test_knn_far_gpu(gpu_ctx):
+    _check_knn_far(gpu_ctx, None)
 
 
 # outputs written straight into the caller's device arrays: not for a torus,
