@@ -175,15 +175,6 @@ int api_cells(Ctx<B>* ctx, const double* xyz, const double* w, const uint32_t* i
             return VGC_ERR_INTERNAL;
         }
         Engine<B>& E = ctx->eng;
-        if (stats) {
-            // the compaction is launched, not awaited, by the pass
-            const auto t = std::chrono::steady_clock::now();
-            be.sync();
-            const double ms = std::chrono::duration<double, std::milli>(
-                                  std::chrono::steady_clock::now() - t).count();
-            es.t_compact_ms += ms;
-            es.t_total_ms += ms;
-        }
         auto out = [&](void* dst, const void* src, size_t bytes) {
             if (!dst || !src) return;
             if (dev)
@@ -192,7 +183,17 @@ int api_cells(Ctx<B>* ctx, const double* xyz, const double* w, const uint32_t* i
                 be.d2h(dst, src, bytes);
         };
         // what the pass has not written there itself
-        if (!pb.out_vol) out(vol, E.d_vol, sizeof(double) * (size_t)n);
+        {
+            // the compaction is launched, not awaited, by the pass: the first
+            // wait is its
+            const auto t = std::chrono::steady_clock::now();
+            if (dev) be.sync();
+            if (!pb.out_vol) out(vol, E.d_vol, sizeof(double) * (size_t)n);
+            const double ms = std::chrono::duration<double, std::milli>(
+                                  std::chrono::steady_clock::now() - t).count();
+            es.t_compact_ms += ms;
+            es.t_total_ms += ms;
+        }
         if (!pb.out_mg) out(mg, E.d_mg, sizeof(double) * 3 * (size_t)n);
         if (!pb.out_ptr) out(nbr_ptr, E.d_ptr, sizeof(long long) * ((size_t)n + 1));
         fill_stats(es, stats);

@@ -69,6 +69,7 @@ struct EmuBackend {
     void event_begin(int) {}
     void event_end(int) {}
     double event_ms(int) { return 0.0; }
+    double event_gap(int, int) { return 0.0; }
 
     void fill_inst(int* inst_orig, int n, const int* p0, int ni) {
         for (int i = 0; i < n; ++i) {

@@ -1586,7 +1586,7 @@ struct HipBackend {
         pin_used_ = 0;
     }
     // HIP events on the launch stream around a phase (slot 0: kNN, 1: pass A,
-    // 2: its FP64 redo, 3: build)
+    // 2: its FP64 redo; 3: before the build)
     void event_begin(int k) {
         if (!ev_[k][0]) {
             VGC_HIP_CHECK(hipEventCreate(&ev_[k][0]));
@@ -1599,6 +1599,13 @@ struct HipBackend {
         float ms = 0.f;
         VGC_HIP_CHECK(hipEventSynchronize(ev_[k][1]));
         VGC_HIP_CHECK(hipEventElapsedTime(&ms, ev_[k][0], ev_[k][1]));
+        return ms;
+    }
+    // from the begin of phase a to that of phase b
+    double event_gap(int a, int b) {
+        float ms = 0.f;
+        VGC_HIP_CHECK(hipEventSynchronize(ev_[b][0]));
+        VGC_HIP_CHECK(hipEventElapsedTime(&ms, ev_[a][0], ev_[b][0]));
         return ms;
     }
     void check() { VGC_HIP_CHECK(hipGetLastError()); }

@@ -523,12 +523,14 @@ public:
         const double tb0 = st.t_build_ms;
         be_.event_begin(3);
         if (build(pb, st)) return -1;
-        be_.event_end(3);
-        // after the first wait: the build's time (its launches return early)
-        // counted as such, the rest of the time so far is the next phase's
-        auto after_build = [&] {
+        // after the first wait, that for phase k: the build's time (its
+        // launches return early) counted as such, the rest of the time so far
+        // is phase k's (the tuner's launches too)
+        bool tuned = false;
+        auto after_build = [&](int k) {
             const double launch = st.t_build_ms - tb0, all = ms_since(tstart);
-            const double ms = std::min(all, std::max(launch, be_.event_ms(3)));
+            const double ms =
+                std::min(all, std::max(launch, tuned ? 0.0 : be_.event_gap(3, k)));
             st.t_build_ms = tb0 + ms;
             return all - ms;
         };
@@ -544,7 +546,7 @@ public:
             knn_lists(K0, d_list);
             be_.event_end(0);
             be_.sync();
-            st.t_knn_ms += after_build();
+            st.t_knn_ms += after_build(0);
             st.t_knn_gpu_ms += be_.event_ms(0);
         }
         auto t2 = now();
@@ -686,6 +688,7 @@ public:
                                                       : (t1w < 0.97 * t4w ? 1 : 4);
             be_.set_clip_waves(best_w);
             tuned_n_ = n_;
+            tuned = true;
             st.tuned_waves = best_w;
         }
         be_.event_begin(1);
@@ -721,7 +724,7 @@ public:
         }
         // after the wait: pass A's time and that of its redo
         auto after_pass = [&] {
-            const double ms = gather ? after_build() : ms_since(t2);
+            const double ms = gather ? after_build(1) : ms_since(t2);
             const double r = redo ? std::min(ms, be_.event_ms(2)) : 0.0;
             st.t_clip_ms += ms - r;
             st.t_pass_bc_ms += r;
