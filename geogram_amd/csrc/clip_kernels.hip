@@ -20,13 +20,13 @@ __global__ __launch_bounds__(64 * WAVES, (S == 1 && !EXACT) ? 4 : 1) void k_clip
     __shared__ CellLds<S> lds[WAVES];
     const int wave = WAVES == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     int item = xcd_block() * WAVES + wave;
-    // The item in a vector register: with a scalar one the compiler keeps all
-    // that follows from it in scalar registers, runs out of them and spills
-    // (S = 4 from lists: 124 spilled and 308 vector registers, against 36 and
-    // 231).  50 large cells of a clustered transport of 1M seeds: S = 2, 4, 8
-    // 34, 65, 140 ms scalar; cells of its first 13 Newton steps 3.07 s scalar,
-    // 2.39 s so.
-    asm volatile("" : "+v"(item));
+    // From lists, the item in a vector register: with a scalar one the compiler
+    // keeps all that follows from it in scalar registers, runs out of them and
+    // spills (S = 4: 124 spilled and 308 vector registers, against 36 and 231).
+    // Cells of the first 13 Newton steps of a clustered transport of 1M seeds:
+    // 3.07 s scalar, 2.39 s so.  Gathering kernels spill either way, and run
+    // 10 to 25 % faster scalar.
+    if constexpr (!GATHER) asm volatile("" : "+v"(item));
     if (item >= P.n_items) return;  // whole wavefront
     process_cell<S, EXACT, GATHER, W, CORNER>(P, item, lds[wave]);
 }
