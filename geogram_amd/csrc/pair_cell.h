@@ -27,7 +27,7 @@
 // bounds are those of the unscaled rows.
 //
 // A cell that needs anything rare (a sign or corner that FP32 cannot certify,
-// more than 64 corners or planes, a coincident or duplicate seed, a walk that
+// more than 64 corners or planes, a coincident earlier seed, a walk that
 // outgrows its buffers) is flagged CELL_UNCERTAIN without outputs; the FP64
 // first pass redoes it from the start.  One that uses up its rings goes to the
 // second gather.
@@ -437,11 +437,13 @@ VGC_HD uint64_t pair_cut(PairState& st, PairLds& L, LI& np, const RowLanes& r, c
 // number staged.  A candidate with the position and weight of the one before
 // it gives the same plane and is not staged: its id takes the other's place
 // (under the exact tie rule the copy takes over the face of the first one).
-// -1 when a candidate needs the general kernel: one at the seed's own
-// position, or a row out of the range of the FP32 bounds.
+// A candidate at the position of the seed c itself is not staged either if it
+// comes later in the caller's order (consider's rule).  -1 when a candidate
+// needs the general kernel: an earlier one at the seed's position, or a row out
+// of the range of the FP32 bounds.
 template <bool W>
-VGC_HD int pair_stage(const ClipParams& P, PairLds& L, int h, float scale, const pt4& pc, double cw,
-                      int cnt) {
+VGC_HD int pair_stage(const ClipParams& P, PairLds& L, int h, int c, float scale, const pt4& pc,
+                      double cw, int cnt) {
     const LI lane = lane_id();
     const LB ok = lane < cnt;
     const LU64 key = lds_ld(L.h[h].key, select(ok, lane, LI(0)));
@@ -468,18 +470,24 @@ VGC_HD int pair_stage(const ClipParams& P, PairLds& L, int h, float scale, const
     lds_st(aux, lane * 2, fr, ok);
     lds_st(aux, lane * 2 + 1, e1, ok);
     wave_sync();
-    const LB out = ok & (!(d2 > 0.0) | !(e1 >= kPairE1Min) | !(e1 <= kPairE1Max) | !(vabs(fh) <= kPairHMax));
+    const uint64_t zm = ballot(ok & (d2 == 0.0));
+    if (zm) {
+        const LI oj = gld(P.orig, select(mask_bit(zm), j, LI(0)), mask_bit(zm));
+        if (ballot(mask_bit(zm) & (oj < P.orig[c]))) return -1;
+    }
+    const LB out = ok & !mask_bit(zm) &
+                   (!(d2 > 0.0) | !(e1 >= kPairE1Min) | !(e1 <= kPairE1Max) | !(vabs(fh) <= kPairHMax));
     if (ballot(out)) return -1;
     // copies follow one another in the sorted order, at one FP32 distance
     const LU64 kp = lds_ld(L.h[h].key, select(ok & (lane > 0), lane - 1, LI(0)));
-    const LB same = ok & (lane > 0) & ((kp >> LU64(32)) == (key >> LU64(32)));
-    if (ballot(same) == 0) return cnt;
+    const LB same = ok & !mask_bit(zm) & (lane > 0) & ((kp >> LU64(32)) == (key >> LU64(32)));
+    if (ballot(same) == 0 && zm == 0) return cnt;
     const LI jp = cvt<int>(cvt<uint32_t>(kp));
     const Lane<pt4> qp = gld(P.pts, jp, same);
     const uint64_t dm = ballot(same & (pt_x(qp) == pt_x(q)) & (pt_y(qp) == pt_y(q)) &
                                (pt_z(qp) == pt_z(q)) & (pt_w(qp) == pt_w(q)));
-    if (dm == 0) return cnt;
-    const uint64_t okm = ballot(ok), keep = okm & ~dm, last = okm & ~(dm >> 1);
+    if ((dm | zm) == 0) return cnt;
+    const uint64_t okm = ballot(ok) & ~zm, keep = okm & ~dm, last = okm & ~(dm >> 1);
     const LI at = mbcnt(keep) - select(mask_bit(keep), LI(0), LI(1));
     wave_sync();
     lds_st_row(row, at, fx, fy, fz, fh, mask_bit(keep));
@@ -961,7 +969,7 @@ VGC_HD void process_pair(const ClipParams& P, int item0, int end, PairLds& L, co
             if (!(live & hm)) continue;
             const int ch = uni(L.ctl[h].c);
             const pt4 pc = P.pts[ch];
-            const int k = pair_stage<W>(P, L, h, uni(L.ctl[h].scale), pc,
+            const int k = pair_stage<W>(P, L, h, ch, uni(L.ctl[h].scale), pc,
                                         W ? pc.w - P.wmax[uni(L.ctl[h].inst)] : 0.0,
                                         readlane(cnt, 32 * h));
             if (k < 0) live &= ~hm;

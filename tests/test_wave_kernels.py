@@ -26,11 +26,39 @@ def _seeds(n, kind, seed=3):
     if kind == "clusters":  # cells of many rings beside dense clusters
         k = n // 2
         x[:k] = 0.5 + 0.004 * rng.standard_normal((k, 3))
+    elif kind == "copies":  # pairs and triples of coincident seeds, any order
+        x = np.concatenate([x[: n // 3], x[: n // 3], x])[:n]
+        x = x[rng.permutation(n)]
     elif kind == "shell":  # the seed inside has more than 64 corners
         x = rng.standard_normal((n, 3))
         x = 0.5 + 0.4 * x / np.linalg.norm(x, axis=1)[:, None]
         x[n // 2] = 0.5
     return x
+
+
+# Of coincident seeds only the one of smallest index has a cell; the first pass
+# computes that one itself and leaves the others (the box, by the coincident-seed
+# rule).
+def _check_copies(ctx, n, weighted):
+    x = _seeds(n, "copies")
+    w = 0.3 * n ** (-2 / 3) * np.random.default_rng(5).random(n) if weighted else None
+    a = ctx.cells(x, weights=w)
+    _same_cells(a, ctx.cells(x, weights=w, fp64_first=True))
+    copies = n - len(np.unique(x, axis=0))
+    assert copies <= a.stats["nb_fp64_redo"] <= copies + n // 20
+    assert a.stats["nb_disconnected"] == copies
+
+
+@pytest.mark.parametrize("n,weighted", [(3, False), (900, False), (900, True), (4500, False)])
+def test_first_pass_copies(emu_ctx, n, weighted):
+    _check_copies(emu_ctx, n, weighted)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,weighted", [(900, True), (4500, False), (160_000, False),
+                                        (160_000, True)])
+def test_first_pass_copies_gpu(gpu_ctx, n, weighted):
+    _check_copies(gpu_ctx, n, weighted)
 
 
 def _check_first_pass(ctx, n, kind):
