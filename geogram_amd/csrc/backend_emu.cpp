@@ -85,12 +85,12 @@ struct EmuBackend {
         }
     }
 
-    void morton(const double* xyz, const int* inst_orig, const double* box, int n,
+    void morton(const double* xyz, const int* inst_orig, const double* box, int n, int drop,
                 uint64_t* keys, int* vals) {
         for (int i = 0; i < n; ++i) {
             int inst = inst_orig ? inst_orig[i] : 0;
             keys[i] = morton_key(xyz[3 * (size_t)i], xyz[3 * (size_t)i + 1], xyz[3 * (size_t)i + 2],
-                                 box + 6 * inst, (uint64_t)inst);
+                                 box + 6 * inst, (uint64_t)inst, drop);
             vals[i] = i;
         }
     }

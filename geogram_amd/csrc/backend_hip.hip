@@ -64,12 +64,13 @@ __global__ void k_fill_inst(int* inst_orig, int n, const int* p0, int ni) {
 }
 
 __global__ void k_morton(const double* __restrict__ xyz, const int* __restrict__ inst_orig,
-                         const double* __restrict__ box, int n, uint64_t* keys, int* vals) {
+                         const double* __restrict__ box, int n, int drop, uint64_t* keys,
+                         int* vals) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     int inst = inst_orig ? inst_orig[i] : 0;
     keys[i] = morton_key(xyz[3 * (size_t)i], xyz[3 * (size_t)i + 1], xyz[3 * (size_t)i + 2],
-                         box + 6 * inst, (uint64_t)inst);
+                         box + 6 * inst, (uint64_t)inst, drop);
     vals[i] = i;
 }
 
@@ -1623,9 +1624,9 @@ struct HipBackend {
         k_fill_inst<<<blocks_for(n, 256), 256, 0, stream_>>>(inst_orig, n, p0, ni);
         check();
     }
-    void morton(const double* xyz, const int* inst_orig, const double* box, int n, uint64_t* keys,
-                int* vals) {
-        k_morton<<<blocks_for(n, 256), 256, 0, stream_>>>(xyz, inst_orig, box, n, keys, vals);
+    void morton(const double* xyz, const int* inst_orig, const double* box, int n, int drop,
+                uint64_t* keys, int* vals) {
+        k_morton<<<blocks_for(n, 256), 256, 0, stream_>>>(xyz, inst_orig, box, n, drop, keys, vals);
         check();
     }
     void sort_pairs(uint64_t* keys, int* vals, uint64_t* keys2, int* vals2, int n, int end_bit) {

@@ -32,11 +32,15 @@ VGC_SD uint64_t quant16(double x, double lo, double hi) {
     return uint64_t(t * 65536.0);
 }
 
-VGC_SD uint64_t morton_key(double x, double y, double z, const double* box, uint64_t inst) {
+// The instance above the Morton code, of which the lowest `drop` bits give way
+// to an instance number of more than 16 bits.
+VGC_SD uint64_t morton_key(double x, double y, double z, const double* box, uint64_t inst,
+                           int drop) {
     uint64_t qx = quant16(x, box[0], box[3]);
     uint64_t qy = quant16(y, box[1], box[4]);
     uint64_t qz = quant16(z, box[2], box[5]);
-    return (inst << 48) | spread16(qx) | (spread16(qy) << 1) | (spread16(qz) << 2);
+    return (inst << (48 - drop)) |
+           ((spread16(qx) | (spread16(qy) << 1) | (spread16(qz) << 2)) >> drop);
 }
 
 // --------------------------------------------------------------- kNN

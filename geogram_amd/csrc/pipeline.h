@@ -237,10 +237,11 @@ public:
         uint64_t* keys2 = (uint64_t*)slot(S_KEYS2, sizeof(uint64_t) * (size_t)n_);
         int* vals = (int*)slot(S_VALS, sizeof(int) * (size_t)n_);
         int* vals2 = (int*)slot(S_VALS2, sizeof(int) * (size_t)n_);
-        be_.morton(pb.d_xyz, d_inst_orig, d_box, n_, keys, vals);
-        int end_bit = 48;
-        while ((1LL << (end_bit - 48)) < ni_) ++end_bit;
-        be_.sort_pairs(keys, vals, keys2, vals2, n_, end_bit);  // result in keys2 / vals2
+        int ibits = 0;
+        while ((1LL << ibits) < ni_) ++ibits;
+        const int drop = std::max(0, ibits - 16);
+        be_.morton(pb.d_xyz, d_inst_orig, d_box, n_, drop, keys, vals);
+        be_.sort_pairs(keys, vals, keys2, vals2, n_, 48 - drop + ibits);  // into keys2 / vals2
         d_pts = (pt4*)slot(S_PTS, sizeof(pt4) * (size_t)n_);
         d_pf = (pf4*)slot(S_PF, sizeof(pf4) * (size_t)n_);
         d_orig = (int*)slot(S_ORIG, sizeof(int) * (size_t)n_);
@@ -326,7 +327,7 @@ public:
             uint64_t* k2 = (uint64_t*)slot(S_QKEYS2, sizeof(uint64_t) * (size_t)nq);
             int* v1 = (int*)slot(S_QVALS, sizeof(int) * (size_t)nq);
             int* v2 = (int*)slot(S_QVALS2, sizeof(int) * (size_t)nq);
-            be_.morton(d_q, nullptr, d_box_, nq, k1, v1);
+            be_.morton(d_q, nullptr, d_box_, nq, 0, k1, v1);
             be_.sort_pairs(k1, v1, k2, v2, nq, 48);
             pt4* qp_ = (pt4*)slot(S_QPTS, sizeof(pt4) * (size_t)nq);
             pf4* qf_ = (pf4*)slot(S_QPF, sizeof(pf4) * (size_t)nq);

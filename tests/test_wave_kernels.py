@@ -90,9 +90,9 @@ def test_first_pass_sizes_gpu(gpu_ctx, n, kind):
 
 # instances that meet within a wavefront, of spacings far apart: it starts the
 # cells of all of them from the first one's
-def _check_batch(ctx, count, weighted):
+def _check_batch(ctx, count, weighted, nmax=11):
     rng = np.random.default_rng(11)
-    sizes = rng.integers(1, 12, count)
+    sizes = rng.integers(1, nmax + 1, count)
     scale = 10.0 ** rng.uniform(-4, 4, count)
     x = np.concatenate([s * rng.random((n, 3)) for n, s in zip(sizes, scale)])
     boxes = np.zeros((count, 6))
@@ -110,6 +110,10 @@ def _check_batch(ctx, count, weighted):
 @pytest.mark.parametrize("count,weighted", [(100, False), (900, False), (900, True)])
 def test_first_pass_batches(emu_ctx, count, weighted):
     _check_batch(emu_ctx, count, weighted)
+
+
+def test_more_instances_than_16_bits(emu_ctx):
+    _check_batch(emu_ctx, 66_000, False, nmax=2)
 
 
 # 1, 2, 4 and 8 cells per wavefront
