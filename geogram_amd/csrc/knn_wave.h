@@ -55,22 +55,25 @@ VGC_HD void knn_fail(const KnnParams& K, int t) {
 #endif
 }
 
-// Query t; N: the wave's bucket list, r: the first radius to try (beyond the
-// box of the points), last2: the squared radius that served the wave's last
-// query far from its points (0: none yet).
-VGC_HD void knn_wave_query(const KnnParams& K, KnnLds& L, const NearList& N, int t, float r,
+// The distance of a query to the box of the points.
+VGC_HD float knn_box_distance(const KnnParams& K, const pf4& q) {
+    const bnode b = K.C.nodes[K.C.IL.t0[0] + 1];
+    const float x = fmaxf(fmaxf(b.lo[0] - q.x, q.x - b.hi[0]), 0.0f);
+    const float y = fmaxf(fmaxf(b.lo[1] - q.y, q.y - b.hi[1]), 0.0f);
+    const float z = fmaxf(fmaxf(b.lo[2] - q.z, q.z - b.hi[2]), 0.0f);
+    return sqrtf(x * x + y * y + z * z);
+}
+
+// Query t; N: the wave's bucket list, r2: the first squared radius to try,
+// last2: the one that served the wave's last query far from its points (0:
+// none yet).
+VGC_HD void knn_wave_query(const KnnParams& K, KnnLds& L, const NearList& N, int t, float r2,
                            float& last2) {
     const LI lane = lane_id_here();
     const pf4 q = K.qf[t];
     const pt4 p = K.qp[t];
-    const bnode b = K.C.nodes[K.C.IL.t0[0] + 1];
-    const float bx = fmaxf(fmaxf(b.lo[0] - q.x, q.x - b.hi[0]), 0.0f);
-    const float by = fmaxf(fmaxf(b.lo[1] - q.y, q.y - b.hi[1]), 0.0f);
-    const float bz = fmaxf(fmaxf(b.lo[2] - q.z, q.z - b.hi[2]), 0.0f);
-    const float d0 = sqrtf(bx * bx + by * by + bz * bz);
-    // lo2 holds too few points, hi2 too many
-    float lo2 = uni(0.99999f * d0 * d0), hi2 = INFINITY, r2 = uni((d0 + r) * (d0 + r));
-    bool grown = false;
+    float lo2 = 0.0f, hi2 = INFINITY;  // too few and too many points
+    bool far = false;
     int n = 0;
     for (int it = 0; it < kKnnTries; ++it) {
         if (uni(N.inst >= 0 && r2 <= N.r2)) {
@@ -89,15 +92,21 @@ VGC_HD void knn_wave_query(const KnnParams& K, KnnLds& L, const NearList& N, int
         }
         if (n < K.kk && n < K.n) {
             const float f = cbrtf((1.2f * K.kk + 4.0f) / float(n > 0 ? n : 1));
-            const bool far = 4 * n < K.kk;
-            grown = grown || far;
             lo2 = r2;
             r2 = uni(r2 * f * f);
-            if (far && r2 < last2) r2 = last2;
+            if (4 * n < K.kk) {
+                if (!far) {
+                    const float d = knn_box_distance(K, q);
+                    lo2 = uni(fmaxf(lo2, 0.99999f * d * d));
+                    r2 = uni(fmaxf(r2, (d + sqrtf(r2)) * (d + sqrtf(r2))));
+                }
+                far = true;
+                r2 = uni(fmaxf(r2, last2));
+            }
             if (!(r2 < hi2)) r2 = uni(sqrtf(lo2) * sqrtf(hi2));
             continue;
         }
-        if (grown) last2 = r2;
+        if (far) last2 = r2;
         // FP64 distances and caller's indices of the listed points
         LD d[2];
         LI id[2], rank[2] = {LI(0), LI(0)};
@@ -177,23 +186,24 @@ VGC_HD void process_knn(const KnnParams& K, int first, int count, KnnLds& L) {
     // kNearRing spacings hold about 60 points; a quarter more than wanted, and
     // within the candidate buffer
     const float want = fminf(1.25f * K.kk + 8.0f, 108.0f);
-    float r = kNearRing * d4 * cbrtf(want * (1.0f / 60.0f));
+    const float r = kNearRing * d4 * cbrtf(want * (1.0f / 60.0f));
     NearList N;
     N.inst = 0;
     N.r2 = (1.25f * r) * (1.25f * r);
     N.n = d4 > 0.0f ? near_buckets(K.C, L, 0, lane_seed(K.qf, t, has), has, N.r2) : -1;
     if (N.n < 0) N.inst = -1;
+    float r2 = r * r;
     if (!(d4 > 0.0f)) {
         // a bucket of copies, or of fewer than five points: the whole tree's
         // box over the point count
         const bnode b = K.C.nodes[K.C.IL.t0[0] + 1];
         const float x = b.hi[0] - b.lo[0], y = b.hi[1] - b.lo[1], z = b.hi[2] - b.lo[2];
         const float f = cbrtf((1.25f * K.kk + 8.0f) / float(K.n));
-        r = sqrtf((x * x + y * y + z * z) * f * f + 1e-30f);
+        r2 = (x * x + y * y + z * z) * f * f + 1e-30f;
     }
-    r = uni(r);
+    r2 = uni(r2);
     float last2 = 0.0f;
-    for (int k = 0; k < count; ++k) knn_wave_query(K, L, N, first + k, r, last2);
+    for (int k = 0; k < count; ++k) knn_wave_query(K, L, N, first + k, r2, last2);
 }
 
 }  // namespace vgc

@@ -470,24 +470,25 @@ VGC_HD int pair_stage(const ClipParams& P, PairLds& L, int h, int c, float scale
     lds_st(aux, lane * 2, fr, ok);
     lds_st(aux, lane * 2 + 1, e1, ok);
     wave_sync();
-    const uint64_t zm = ballot(ok & (d2 == 0.0));
-    if (zm) {
+    const LB out = ok & (!(d2 > 0.0) | !(e1 >= kPairE1Min) | !(e1 <= kPairE1Max) | !(vabs(fh) <= kPairHMax));
+    const uint64_t om = ballot(out);
+    uint64_t zm = 0;  // at the seed
+    if (om) {
+        zm = ballot(ok & (d2 == 0.0));
+        if (om & ~zm) return -1;
         const LI oj = gld(P.orig, select(mask_bit(zm), j, LI(0)), mask_bit(zm));
         if (ballot(mask_bit(zm) & (oj < P.orig[c]))) return -1;
     }
-    const LB out = ok & !mask_bit(zm) &
-                   (!(d2 > 0.0) | !(e1 >= kPairE1Min) | !(e1 <= kPairE1Max) | !(vabs(fh) <= kPairHMax));
-    if (ballot(out)) return -1;
     // copies follow one another in the sorted order, at one FP32 distance
     const LU64 kp = lds_ld(L.h[h].key, select(ok & (lane > 0), lane - 1, LI(0)));
-    const LB same = ok & !mask_bit(zm) & (lane > 0) & ((kp >> LU64(32)) == (key >> LU64(32)));
+    const LB same = ok & (lane > 0) & ((kp >> LU64(32)) == (key >> LU64(32)));
     if (ballot(same) == 0 && zm == 0) return cnt;
     const LI jp = cvt<int>(cvt<uint32_t>(kp));
     const Lane<pt4> qp = gld(P.pts, jp, same);
     const uint64_t dm = ballot(same & (pt_x(qp) == pt_x(q)) & (pt_y(qp) == pt_y(q)) &
                                (pt_z(qp) == pt_z(q)) & (pt_w(qp) == pt_w(q)));
     if ((dm | zm) == 0) return cnt;
-    const uint64_t okm = ballot(ok) & ~zm, keep = okm & ~dm, last = okm & ~(dm >> 1);
+    const uint64_t okm = ballot(ok) & ~zm, keep = okm & ~dm, last = okm & ~((dm & ~zm) >> 1);
     const LI at = mbcnt(keep) - select(mask_bit(keep), LI(0), LI(1));
     wave_sync();
     lds_st_row(row, at, fx, fy, fz, fh, mask_bit(keep));
