@@ -633,8 +633,11 @@ public:
         // FP32 corner state for the first pass, except for cell meshes (those
         // are emitted by the FP64 pass) and for a few passes after one that
         // had to redo more than half of its cells in FP64 (ties everywhere,
-        // as on lattices; the FP32 pass costs less than half of the FP64
-        // one, and the outputs are the same either way)
+        // as on lattices; the outputs are the same either way).  Calls with
+        // FP32 and FP64 first passes, in ms: jittered lattices of 512k seeds,
+        // 15 % redone 6.1 and 9.8, 41 % 8.8 and 9.8, 79 % 12.5 and 9.8; weighted
+        // cells, 1M at the weights of a 16-Gaussian transport, 7 % redone 151
+        // and 154, part lattices, 20 to 50 % redone, within 2 %
         P.fp32 = (gather && !fp64_first && !pb.mesh_mode && fp32_skip_ == 0) ? 1 : 0;
         if (fp32_skip_ > 0) --fp32_skip_;
         if (pb.abort_on_empty) {

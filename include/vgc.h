@@ -117,11 +117,11 @@ typedef struct vgc_stats {
     uint64_t a_cells, a_tests, a_live, a_new, a_tets, a_facets;
     uint64_t nb_fail_capacity; /* failed cells that exceed 256 corners / planes or
                                   the facet staging stride                          */
-    /* first pass cells handed to the list tiers, by cause: ring limit of the
-       weighted search, a tree walk beyond the wave's buffers, a ring that
-       could not be narrowed */
+    /* first pass cells handed on, by cause: ring limit (to the second gather), a
+       tree walk beyond the wave's buffers, a ring that could not be narrowed
+       (to the list tiers) */
     uint64_t why_rings, why_walk, why_narrow;
-    uint64_t nb_regather; /* weighted cells gathered again without the ring limit */
+    uint64_t nb_regather; /* cells gathered again without the ring limit */
     uint64_t tuned_waves; /* VGC_AUTOTUNE: wavefronts per work-group chosen (0: none) */
     uint64_t nb_periodic_retries; /* VGC_PERIODIC: passes redone with a wider image
                                      margin */
