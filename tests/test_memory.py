@@ -1,11 +1,13 @@
-"""The library's own memory and its caller's, on the CPU emulation, whose
+"""The library's own memory and its caller's, most of it on the CPU emulation, whose
 "device" memory is the host's."""
 import ctypes
 
 import numpy as np
+import pytest
 
 import geogram_amd as ga
-from geogram_amd._lib import Stats, VGC_DEVICE_PTRS, VGC_NO_NEIGHBORS, VGC_OK, VGC_ERR_DEVICE
+from geogram_amd._lib import (Stats, VGC_DEVICE_PTRS, VGC_ERR_CAPACITY, VGC_ERR_DEVICE,
+                              VGC_NO_NEIGHBORS, VGC_OK)
 from geogram_amd import _ptr
 
 
@@ -92,3 +94,56 @@ def test_outputs_over_inputs():
     assert np.array_equal(a.mg, y) and np.array_equal(a.vol, b.vol)
     assert np.array_equal(a.nbr, b.nbr) and np.array_equal(a.farea, b.farea)
     ctx.close()
+
+
+# what a call may be given: arrays that hold the neighbours or are too small for
+# them, only one of the two neighbour arrays, none of the others, arrays at
+# addresses that are no multiple of their type
+def _check_outputs(ctx, n, case, on_gpu):
+    box, st = np.array([0.0, 0, 0, 1, 1, 1]), Stats()
+    x = np.random.default_rng(9).random((n, 3))
+    r = ctx.cells(x)
+    nnz = int(r.nbr_ptr[-1])
+    cap = nnz - 1 if case == "too small" else nnz
+    off = 4 if case == "unaligned" else 0
+    host = {k: np.full(m * s + off + 8, 0xA5, dtype=np.uint8)
+            for k, m, s in (("vol", n, 8), ("mg", 3 * n, 8), ("ptr", n + 1, 8), ("nbr", nnz, 4),
+                            ("farea", nnz, 8))}
+    give = {"no areas": ("vol", "mg", "ptr", "nbr"), "no ids": ("vol", "mg", "ptr", "farea"),
+            "areas only": ("farea",)}.get(case, tuple(host))
+    xs = x
+    if on_gpu:
+        import torch
+        host = {k: torch.from_numpy(v).cuda() for k, v in host.items()}
+        xs = torch.from_numpy(x).cuda()
+        torch.cuda.synchronize()
+    addr = {k: ctypes.c_void_p(_ptr(v).value + off) if k in give else None for k, v in host.items()}
+    rc = ctx.lib.fn("cells")(ctx.ctx, _ptr(xs), None, n, _ptr(box), 0, VGC_DEVICE_PTRS, addr["vol"],
+                             addr["mg"], addr["ptr"], addr["nbr"], addr["farea"], cap,
+                             ctypes.byref(st))
+    assert rc == (VGC_ERR_CAPACITY if case == "too small" else VGC_OK)
+    assert st.nb_neighbors == nnz
+    want = {"vol": r.vol, "mg": r.mg, "ptr": r.nbr_ptr, "nbr": r.nbr, "farea": r.farea}
+    for k, v in host.items():
+        v = (v.cpu().numpy() if on_gpu else v)[off:]
+        if k in give and not (case == "too small" and k in ("nbr", "farea")):
+            w = np.ascontiguousarray(want[k]).tobytes()
+            assert v[:len(w)].tobytes() == w and np.all(v[len(w):] == 0xA5), k
+        else:
+            assert np.all(v == 0xA5), k
+
+
+OUTPUTS = [(n, c) for n in (1, 300) for c in
+           ("all", "too small", "no areas", "no ids", "areas only", "unaligned")
+           if not (n == 1 and c == "too small")]
+
+
+@pytest.mark.parametrize("n,case", OUTPUTS)
+def test_outputs(emu_ctx, n, case):
+    _check_outputs(emu_ctx, n, case, False)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,case", [(n if n == 1 else 5001, c) for n, c in OUTPUTS if c != "unaligned"])
+def test_outputs_gpu(gpu_ctx, n, case):
+    _check_outputs(gpu_ctx, n, case, True)
