@@ -70,6 +70,7 @@ struct EmuBackend {
     void event_end(int) {}
     double event_ms(int) { return 0.0; }
     double event_gap(int, int) { return 0.0; }
+    double event_after(int, int) { return 0.0; }
 
     void fill_inst(int* inst_orig, int n, const int* p0, int ni) {
         for (int i = 0; i < n; ++i) {
@@ -381,7 +382,9 @@ struct EmuBackend {
     }
 
     void compact(int n, const int* cnt, const long long* ptr, const int* nbr_tmp,
-                 const double* area_tmp, int stride, int* nbr, double* area, const CellOut& O) {
+                 const double* area_tmp, int stride, int* nbr, double* area, const CellOut& O,
+                 const unsigned* left) {
+        if (left && *left) return;
         for (int i = 0; nbr && i < n; ++i)
             for (int k = 0; k < std::min(cnt[i], stride); ++k) {
                 nbr[ptr[i] + k] = nbr_tmp[(size_t)i * stride + k];

@@ -331,7 +331,9 @@ __global__ void k_rebase(const long long* __restrict__ off, int n, long long bas
 constexpr int kCompactLanes = 16;
 __global__ void k_compact(int n, const int* __restrict__ cnt, const long long* __restrict__ ptr,
                           const int* __restrict__ nbr_tmp, const double* __restrict__ area_tmp,
-                          int stride, int* nbr, double* area, CellOut O) {
+                          int stride, int* nbr, double* area, CellOut O,
+                          const unsigned* __restrict__ left) {
+    if (left && *left) return;  // (the whole grid)
     const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     const long long i = t / kCompactLanes;
     if (i >= n) return;
@@ -1586,29 +1588,25 @@ struct HipBackend {
         VGC_HIP_CHECK(hipStreamSynchronize(stream_));
         pin_used_ = 0;
     }
-    // HIP events on the launch stream around a phase (slot 0: kNN, 1: pass A,
-    // 2: its FP64 redo; 3: before the build)
-    void event_begin(int k) {
-        if (!ev_[k][0]) {
-            VGC_HIP_CHECK(hipEventCreate(&ev_[k][0]));
-            VGC_HIP_CHECK(hipEventCreate(&ev_[k][1]));
-        }
-        VGC_HIP_CHECK(hipEventRecord(ev_[k][0], stream_));
+    // HIP events on the launch stream around a phase (slot 0: kNN, 1: pass A;
+    // 2: after its FP64 redo; 3: before the build)
+    hipEvent_t& event(int k, int end) {
+        hipEvent_t& e = ev_[k][end];
+        if (!e) VGC_HIP_CHECK(hipEventCreate(&e));
+        return e;
     }
-    void event_end(int k) { VGC_HIP_CHECK(hipEventRecord(ev_[k][1], stream_)); }
-    double event_ms(int k) {
+    void event_begin(int k) { VGC_HIP_CHECK(hipEventRecord(event(k, 0), stream_)); }
+    void event_end(int k) { VGC_HIP_CHECK(hipEventRecord(event(k, 1), stream_)); }
+    double elapsed(hipEvent_t a, hipEvent_t b) {
         float ms = 0.f;
-        VGC_HIP_CHECK(hipEventSynchronize(ev_[k][1]));
-        VGC_HIP_CHECK(hipEventElapsedTime(&ms, ev_[k][0], ev_[k][1]));
+        VGC_HIP_CHECK(hipEventSynchronize(b));
+        VGC_HIP_CHECK(hipEventElapsedTime(&ms, a, b));
         return ms;
     }
-    // from the begin of phase a to that of phase b
-    double event_gap(int a, int b) {
-        float ms = 0.f;
-        VGC_HIP_CHECK(hipEventSynchronize(ev_[b][0]));
-        VGC_HIP_CHECK(hipEventElapsedTime(&ms, ev_[a][0], ev_[b][0]));
-        return ms;
-    }
+    double event_ms(int k) { return elapsed(event(k, 0), event(k, 1)); }
+    // from the begin of phase a to that of phase b, from end to end
+    double event_gap(int a, int b) { return elapsed(event(a, 0), event(b, 0)); }
+    double event_after(int a, int b) { return elapsed(event(a, 1), event(b, 1)); }
     void check() { VGC_HIP_CHECK(hipGetLastError()); }
 
     void* temp(size_t b) {
@@ -1824,9 +1822,10 @@ struct HipBackend {
                                                           off + 1, 0, 32, stream_));
     }
     void compact(int n, const int* cnt, const long long* ptr, const int* nbr_tmp,
-                 const double* area_tmp, int stride, int* nbr, double* area, const CellOut& O) {
+                 const double* area_tmp, int stride, int* nbr, double* area, const CellOut& O,
+                 const unsigned* left) {
         k_compact<<<blocks_for((long long)n * kCompactLanes, 256), 256, 0, stream_>>>(
-            n, cnt, ptr, nbr_tmp, area_tmp, stride, nbr, area, O);
+            n, cnt, ptr, nbr_tmp, area_tmp, stride, nbr, area, O, left);
         check();
     }
     void lloyd_update(double* xyz, const double* vol, const double* mg, int n,

@@ -722,14 +722,13 @@ public:
             int* d_cc = (int*)slot(S_CENS_C, sizeof(int) * ncen);
             be_.census(P.items, P.n_items, d_flags, CELL_UNCERTAIN, 0, P.abort_flag, P.inst_of, d_cc,
                        nullptr, d_cen + 1);
-            be_.event_begin(2);
             be_.clip_listed(P, d_cc, d_cen + 1);
             be_.event_end(2);
         }
         // after the wait: pass A's time and that of its redo
         auto after_pass = [&] {
             const double ms = gather ? after_build(1) : ms_since(t2);
-            const double r = redo ? std::min(ms, be_.event_ms(2)) : 0.0;
+            const double r = redo ? std::min(ms, be_.event_after(1, 2)) : 0.0;
             st.t_clip_ms += ms - r;
             st.t_pass_bc_ms += r;
             st.t_redo_gpu_ms += r;
@@ -762,14 +761,23 @@ public:
         if ((int)h_flags.size() < n_) h_flags.resize(n_);
         census_.clear();
         d_ptr = (long long*)slot(S_PTR, sizeof(long long) * ((size_t)n_ + 1));
+        const CellOut O{d_vol, d_mg, pb.out_vol, pb.out_mg, pb.out_ptr};
+        bool delivered = false;
         {
             be_.census(P.items, P.n_items, d_flags, kCensusMask, CELL_DONE, P.abort_flag, P.inst_of,
                        nullptr, d_cen + 2, d_cen);
             be_.scan_i32(d_cnt, d_ptr, n_);
+            // without neighbours to size, the outputs are delivered here if no
+            // cell is left over (the host would have to launch it after the
+            // wait: 16 us of a small call's 190)
+            if (!pb.want_neighbors && O.any())
+                be_.compact(n_, d_cnt, d_ptr, d_nbr_tmp, d_area_tmp, kFaceStride, nullptr, nullptr,
+                            O, d_cen);
             std::vector<unsigned> head(2 + 2 * std::min<size_t>(ncen, kCensusHead));
             be_.d2h2(head.data(), d_cen, sizeof(unsigned) * head.size(), &total_neighbors, d_ptr + n_,
                      sizeof(long long));
             const size_t m = head[0];
+            delivered = !pb.want_neighbors && m == 0;
             if (head.size() < 2 + 2 * m) {
                 head.resize(2 + 2 * m);
                 be_.d2h(head.data(), d_cen, sizeof(unsigned) * head.size());
@@ -910,9 +918,8 @@ public:
                 area = d_area = (double*)slot(S_AREA, sizeof(double) * m);
             }
         }
-        const CellOut O{d_vol, d_mg, pb.out_vol, pb.out_mg, pb.out_ptr};
-        if (nbr || O.any())
-            be_.compact(n_, d_cnt, d_ptr, d_nbr_tmp, d_area_tmp, kFaceStride, nbr, area, O);
+        if (nbr || (O.any() && !delivered))
+            be_.compact(n_, d_cnt, d_ptr, d_nbr_tmp, d_area_tmp, kFaceStride, nbr, area, O, nullptr);
         if (nbr && !piece_cells_.empty())
             be_.piece_copy((int)piece_cells_.size(), (const int*)slots_[S_XCELLS].p, d_orig,
                            (const long long*)slots_[S_XOFF].p, (const int*)slots_[S_XNBR].p,

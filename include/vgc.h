@@ -130,7 +130,7 @@ typedef struct vgc_stats {
                              voronoi/convex_cell.cpp:1086-1101) */
     uint64_t nb_fp64_redo; /* cells of the FP32 first pass redone by the FP64
                               first pass (a sign or corner not certified) */
-    double t_redo_gpu_ms;  /* GPU time of that FP64 launch */
+    double t_redo_gpu_ms;  /* GPU time of that FP64 launch and of listing its cells */
 } vgc_stats;
 
 /* Context on one GPU (device index as seen by HIP).  Replaces nothing in

@@ -65,16 +65,19 @@ def test_convex_levels_of_five_seeds():
     ctx.close()
 
 
-def test_a_failed_call_leaves_the_arrays_alone():
+@pytest.mark.parametrize("flags", [0, VGC_NO_NEIGHBORS])
+@pytest.mark.parametrize("copies", [True, False])
+def test_a_failed_call_leaves_the_arrays_alone(flags, copies):
     """The caller's arrays are written when every pass has succeeded: whichever
     allocation of a call fails, they hold what they held."""
     x = np.random.default_rng(2).random((300, 3))
-    x[:2] = x[2]  # coincident seeds: the exact pass runs too
+    if copies:
+        x[:2] = x[2]  # cells for the passes after the first
     failures = 0
     while True:
         ctx, a = ga.Context.emulated(), _Arrays(300)
         ctx.lib.cdll.vgc_emu_fail_alloc(ctx.ctx, failures + 1)
-        rc = _cells(ctx, x, a)
+        rc = _cells(ctx, x, a, flags)
         ctx.close()
         if rc == VGC_OK:
             break
