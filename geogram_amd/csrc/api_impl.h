@@ -40,7 +40,9 @@ struct Ctx {
         if ((int)stage.size() <= id) stage.resize(id + 1);
         Buf& b = stage[id];
         if (b.bytes < bytes) {
-            if (b.p) be.dfree(b.p);
+            Buf old = b;
+            b = Buf();  // (an allocation that fails leaves none)
+            if (old.p) be.dfree(old.p);
             b.p = be.dalloc(bytes);
             b.bytes = bytes;
         }

@@ -1609,12 +1609,20 @@ struct HipBackend {
     double event_after(int a, int b) { return elapsed(event(a, 1), event(b, 1)); }
     void check() { VGC_HIP_CHECK(hipGetLastError()); }
 
+    // p replaced by n elements of `size` bytes (none if that fails)
+    template <class T, class N>
+    void regrow(T*& p, N& cap, N n, size_t size) {
+        T* old = p;
+        p = nullptr;
+        cap = 0;
+        if (old) VGC_HIP_CHECK(hipFree(old));
+        void* q = nullptr;
+        VGC_HIP_CHECK(hipMalloc(&q, size * (size_t)n));
+        p = (T*)q;
+        cap = n;
+    }
     void* temp(size_t b) {
-        if (b > temp_bytes_) {
-            if (temp_) VGC_HIP_CHECK(hipFree(temp_));
-            temp_bytes_ = b + b / 4;
-            VGC_HIP_CHECK(hipMalloc(&temp_, temp_bytes_));
-        }
+        if (b > temp_bytes_) regrow(temp_, temp_bytes_, b + b / 4, 1);
         return temp_;
     }
 
@@ -1755,21 +1763,13 @@ struct HipBackend {
         const long long fstride = std::max(1, tree_leaves_);
         const long long g = std::min(wide_waves(), (long long)ni);
         const long long need = g * 2 * fstride;
-        if (wide_front_cap_ < need) {
-            if (wide_front_) VGC_HIP_CHECK(hipFree(wide_front_));
-            VGC_HIP_CHECK(hipMalloc(&wide_front_, sizeof(int) * (size_t)need));
-            wide_front_cap_ = need;
-        }
+        if (wide_front_cap_ < need) regrow(wide_front_, wide_front_cap_, need, sizeof(int));
         k_radius_wide<<<(unsigned)g, 64, 0, stream_>>>(pf, nodes, IL, items, ni, rho2, filt, wide,
                                                        wide_front_, fstride, cnt, off, base, list,
                                                        d2);
     }
     unsigned char* wide_flags(int ni) {
-        if (wide_cap_ < ni) {
-            if (wide_) VGC_HIP_CHECK(hipFree(wide_));
-            VGC_HIP_CHECK(hipMalloc(&wide_, (size_t)ni));
-            wide_cap_ = ni;
-        }
+        if (wide_cap_ < ni) regrow(wide_, wide_cap_, ni, 1);
         return wide_;
     }
     void rebase(const long long* off, int n, long long base, long long* out) {
@@ -1982,11 +1982,7 @@ struct HipBackend {
     // block partials (p.q, and r.z, r.r of the two update parities)
     double* cg_part(int) {
         const long long need = 5ll * kRedBlocks;
-        if (cg_part_cap_ < need) {
-            if (cg_part_) VGC_HIP_CHECK(hipFree(cg_part_));
-            VGC_HIP_CHECK(hipMalloc(&cg_part_, sizeof(double) * (size_t)need));
-            cg_part_cap_ = need;
-        }
+        if (cg_part_cap_ < need) regrow(cg_part_, cg_part_cap_, need, sizeof(double));
         return cg_part_;
     }
     // Morton order of a Newton system (orig: Morton position -> caller index)
@@ -2021,11 +2017,7 @@ struct HipBackend {
     // --------------------------------------------------------- batched OT
     // block partials of the batched reductions: count doubles
     double* seg_part(long long count) {
-        if (seg_part_cap_ < count) {
-            if (seg_part_) VGC_HIP_CHECK(hipFree(seg_part_));
-            VGC_HIP_CHECK(hipMalloc(&seg_part_, sizeof(double) * (size_t)count));
-            seg_part_cap_ = count;
-        }
+        if (seg_part_cap_ < count) regrow(seg_part_, seg_part_cap_, count, sizeof(double));
         return seg_part_;
     }
     void seg_mass_stats(const SegTable& T, const double* m, const double* nu, double* out) {

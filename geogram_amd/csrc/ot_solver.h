@@ -544,9 +544,12 @@ private:
         if ((int)slots_.size() <= id) slots_.resize(id + 1);
         Buf& b = slots_[id];
         if (b.bytes < bytes) {
-            if (b.p) be_.dfree(b.p);
-            b.bytes = std::max(bytes, b.bytes + b.bytes / 4);
-            b.p = be_.dalloc(b.bytes);
+            const size_t nb = std::max(bytes, b.bytes + b.bytes / 4);
+            Buf old = b;
+            b = Buf();  // (an allocation that fails leaves none)
+            if (old.p) be_.dfree(old.p);
+            b.p = be_.dalloc(nb);
+            b.bytes = nb;
         }
         return b.p;
     }

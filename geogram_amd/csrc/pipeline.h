@@ -1024,8 +1024,10 @@ private:
         if (slots_.size() < S_COUNT) slots_.resize(S_COUNT);
         Buf& b = slots_[id];
         if (b.bytes < bytes) {
-            if (b.p) be_.dfree(b.p);
-            size_t nb = std::max(bytes, b.bytes + b.bytes / 4);
+            const size_t nb = std::max(bytes, b.bytes + b.bytes / 4);
+            Buf old = b;
+            b = Buf();  // (an allocation that fails leaves none)
+            if (old.p) be_.dfree(old.p);
             b.p = be_.dalloc(nb);
             b.bytes = nb;
         }

@@ -150,3 +150,32 @@ def test_outputs(emu_ctx, n, case):
 @pytest.mark.parametrize("n,case", [(n if n == 1 else 5001, c) for n, c in OUTPUTS if c != "unaligned"])
 def test_outputs_gpu(gpu_ctx, n, case):
     _check_outputs(gpu_ctx, n, case, True)
+
+
+def test_a_context_after_a_failed_allocation():
+    """Buffers that could not grow are gone, not kept as freed ones: smaller
+    calls on the same context go on as before, whichever growth failed."""
+    rng = np.random.default_rng(6)
+    small, large = rng.random((60, 3)), rng.random((900, 3))
+    small[0] = small[1]
+    ref = ga.Context.emulated()
+    want = ref.cells(small)
+    ref.close()
+    k, failed = 0, True
+    while failed:
+        k += 1
+        ctx = ga.Context.emulated()
+        ctx.cells(small)
+        ctx.lib.cdll.vgc_emu_watch_frees(ctx.ctx)
+        ctx.lib.cdll.vgc_emu_fail_alloc(ctx.ctx, k)
+        try:
+            ctx.ot_solve(large, np.full(900, 1 / 900), tol=1e-2, max_newton=1)
+            failed = False
+        except ga.VgcError as e:
+            assert e.code == VGC_ERR_DEVICE
+        ctx.lib.cdll.vgc_emu_fail_alloc(ctx.ctx, 0)
+        got = ctx.cells(small)
+        assert np.array_equal(got.vol, want.vol) and np.array_equal(got.nbr, want.nbr)
+        assert ctx.lib.cdll.vgc_emu_freed_writes(ctx.ctx) == 0, k
+        ctx.close()
+    assert k > 20
