@@ -327,7 +327,10 @@ __global__ void k_rebase(const long long* __restrict__ off, int n, long long bas
 }
 
 // 16 lanes per cell: each cell's row of the per-cell staging (stride
-// entries) is read and its CSR range written in contiguous 64-byte runs
+// entries) is read and its CSR range written in contiguous 64-byte runs (no CSR
+// if nbr is null).  A caller's arrays for the other outputs (O) are written
+// along; nothing is while *left, if given, counts cells that a later pass has
+// to finish.
 constexpr int kCompactLanes = 16;
 __global__ void k_compact(int n, const int* __restrict__ cnt, const long long* __restrict__ ptr,
                           const int* __restrict__ nbr_tmp, const double* __restrict__ area_tmp,

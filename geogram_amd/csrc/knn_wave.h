@@ -17,7 +17,7 @@ constexpr int kKnnGroup = 8;
 // lone point's ball touches a dense cluster (200k points, k = 16, 1000 of them
 // around the cluster of the others: with 8 tries and no bracket the queries
 // left to the lists took 192 ms, now 0.84 ms in all; 20k queries far from 100k
-// points 1.58 -> 0.28 ms)
+// points 1.56 -> 0.43 ms)
 constexpr int kKnnTries = 16;
 
 struct alignas(16) KnnLds {
